@@ -1,0 +1,1016 @@
+"""The registration path's performance cases.
+
+Every case drives the public Python entry points the way a host program does:
+a LiDAR sequence (generated here, see Drive) is registered scan by scan, by
+itself, in batches of many sequences, or through the continuous-batching
+server.  A pass takes the next scan of a closed ring: a room sequence returns
+to where it started, a street sequence runs through scenery that repeats along
+x, so any number of passes follows one another without a jump.
+
+  listed()              the listed cases
+  draw(rng)             one more case of the same ranges
+  prepare(case, seed)   sequences in HBM (or host memory for the node form),
+                        sessions, their first map
+  run(state)            one pass
+  work(case)            bytes and operations a pass cannot do without
+  exact(case, seed)     the first pass's outputs in 64 bits (plain numpy)
+"""
+import math
+
+import numpy as np
+import torch
+
+from voxelmapplus_fastlio2_amd import (
+    Context,
+    LIOBuilder,
+    LIOConfig,
+    Registrar,
+    initial_covariance,
+    register_batch,
+    register_batch_submit,
+    register_batch_wait,
+    set_raw_device_batch,
+    state_vector,
+)
+from voxelmapplus_fastlio2_amd.registration import LIO_MAPPING
+from voxelmapplus_fastlio2_amd.serving import Request, Server, make_requests
+from voxelmapplus_fastlio2_amd.synth import QDIAG
+
+DEV = "cuda:0"
+SCAN_DT = 0.1     # 10 Hz scans
+IMU_DT = 0.005    # 200 Hz IMU
+STREET_LEN = 8.0  # the street's scenery repeats after this many metres
+G = 9.81
+EXACT_POINTS = 24000  # larger scans take the 64-bit restatement too long
+
+
+# --------------------------------------------------------------------------
+# cases
+# --------------------------------------------------------------------------
+def _case(name, kind, **kw):
+    c = dict(name=name, kind=kind, scene="room", n=20000, n_min=0, ring=16, capacity=100000, sessions=1, groups=1,
+             scans=1, resolution=0.0, estimate_ext=False, noalloc=False)
+    c.update(kw)
+    return c
+
+
+def listed():
+    return [
+        # A host IESKF with vmp_observe as its measurement function, on the
+        # smallest scans in use: launch and round-trip latency.
+        _case("observe_room_2k", "observe", n=2000),
+        # The same with every return of a dense sensor and the extrinsics
+        # estimated (12 Jacobian columns).
+        _case("observe_street_120k_ext", "observe", scene="street", n=120000, estimate_ext=True),
+        # A small robot with an odometry prior: 2,003 returns per scan.
+        _case("odom_room_2k", "odom", n=2003, ring=64),
+        # The call for callers that may not allocate, ragged mid-size scans.
+        _case("noalloc_street_31k", "odom", scene="street", n=31111, n_min=30000, ring=32, noalloc=True),
+        # 20,000 raw returns and 200 Hz IMU in a room that has been seen
+        # before: most voxels are frozen planes.
+        _case("imu_room_20k", "imu", ring=64),
+        # 120,000 returns per raw scan along a street, 2M-voxel LRU.
+        _case("imu_street_120k", "imu", scene="street", n=120000, ring=32, capacity=2000000),
+        # The same street with an LRU that is full: every scan evicts, and
+        # the number of returns varies from scan to scan as a sensor's does.
+        _case("evict_street_60k", "imu", scene="street", n=61000, n_min=58001, ring=32, capacity=200000),
+        # The ROS node's loop: host clouds, the yaml's 0.1 m scan filter,
+        # odometry and the body cloud published after every scan.
+        _case("node_room_20k", "node", n=20000, n_min=19000, ring=64, resolution=0.1),
+        # A short log from nothing: a session is created, the map built,
+        # six scans registered, the map exported, the session closed.
+        _case("log_room_20k", "log", ring=16, scans=6, capacity=30000),
+        # Sixteen small robots advanced together.
+        _case("batch_16_small", "batch", scene="mixed", n=20000, n_min=2000, sessions=16),
+        # 128 sequences of 2k-120k returns in four groups (one stream each).
+        _case("batch_128", "batch", scene="mixed", n=120000, n_min=2000, sessions=128, groups=4,
+              capacity=100000),
+        # The server with a burst of requests: 64 sessions, two scans each,
+        # sizes log-uniform in 2k-120k.
+        _case("serve_64", "serve", scene="mixed", n=120000, n_min=2000, sessions=64, scans=2, groups=4,
+              capacity=100000),
+    ]
+
+
+def draw(rng):
+    def size(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    kind = rng.choice(["observe", "odom", "imu", "imu", "node", "log", "batch", "serve"])
+    scene = rng.choice(["room", "street"])
+    n = size(2000, 120000)
+    c = _case("", kind, scene=scene, n=n, ring=rng.choice([16, 32]))
+    del c["name"]
+    if rng.random() < 0.5:
+        c["n_min"] = max(2000, int(n * rng.uniform(0.9, 0.99)))
+    if kind == "observe":
+        c.update(n_min=0, estimate_ext=rng.random() < 0.5)
+    elif kind in ("odom", "imu"):
+        c["capacity"] = rng.choice([60000, 200000, 1000000])
+        c["estimate_ext"] = rng.random() < 0.2
+        c["noalloc"] = kind == "odom" and rng.random() < 0.3
+    elif kind == "node":
+        c["resolution"] = rng.choice([0.0, 0.1, 0.2])
+    elif kind == "log":
+        c.update(scans=rng.randint(3, 8), capacity=60000, n=min(n, 60000), n_min=0)
+    else:
+        c.update(scene=rng.choice(["room", "street", "mixed"]), sessions=size(4, 48), ring=16, n_min=2000,
+                 groups=rng.choice([1, 2, 4]))
+        if kind == "serve":
+            c["scans"] = rng.choice([1, 2, 4])
+    return c
+
+
+def work(case):
+    """Per registered scan: the points read (12 B, 16 B with their times),
+    the residual slots written (16 B), the voxels a scan touches (about one
+    per four points) read and their records (hash entry 16, plane 32, state
+    80, plane sums 64 B) written once; the filter state.  Operations: the
+    transform, gate, Jacobian and 27 sums of a point in the two passes a
+    scan takes at least, and its insertion."""
+    n = 0.5 * (case["n"] + case["n_min"]) if case["n_min"] else case["n"]
+    if case["kind"] == "serve":
+        n = (case["n"] - case["n_min"]) / math.log(case["n"] / case["n_min"])
+    scans = case["sessions"] * (case["scans"] if case["kind"] in ("log", "serve") else 1)
+    if case["kind"] == "observe":
+        b, f = n * (12 + 16) + n / 4 * 48, n * 200
+    else:
+        b, f = n * (16 + 16) + n / 4 * 2 * 192 + 2 * 4600, n * 700
+    return {"bytes": scans * b, "flops": scans * f}
+
+
+# --------------------------------------------------------------------------
+# sequences
+# --------------------------------------------------------------------------
+def _trajectory(m, scene, period, t):
+    """Pose at time t as (x, y, z, roll, pitch, yaw); periodic up to the
+    street's STREET_LEN along x.  m: numpy or torch."""
+    w = 2.0 * math.pi / period
+    s, c = m.sin(w * t), m.cos(w * t)
+    if scene == "street":
+        v, a = STREET_LEN / period, min(0.3, 0.5 / (w * w))
+        x, y, yaw = v * t, a * s, m.atan2(a * w * c, v + 0.0 * t)
+        z = 2.0 + min(0.02, 0.3 / (w * w)) * s
+    else:
+        a = min(4.0, 0.8 / w)
+        x, y, yaw = a * s, 0.25 * a * m.sin(2.0 * w * t), min(1.0, 0.5 / w) * s
+        z = 1.2 + min(0.05, 0.3 / (w * w)) * s
+    return x, y, z, min(0.03, 0.2 / w) * m.sin(w * t + 0.3), min(0.03, 0.2 / w) * m.sin(w * t + 1.1), yaw
+
+
+def _pose(scene, period, t):
+    """(R, p) at time t."""
+    x, y, z, r, p, h = (float(v) for v in _trajectory(np, scene, period, np.float64(t)))
+    cr, sr, cp, sp, ch, sh = (f(a) for a in (r, p, h) for f in (math.cos, math.sin))
+    R = np.array([[ch, -sh, 0], [sh, ch, 0], [0, 0, 1.0]]) @ np.array([[cp, 0, sp], [0, 1, 0], [-sp, 0, cp]])
+    return R @ np.array([[1.0, 0, 0], [0, cr, -sr], [0, sr, cr]]), np.array([x, y, z])
+
+
+def _scene(scene, rng):
+    """Boxes (centre, half size, yaw) and poles (x, y, z0, z1)."""
+    boxes, poles = [], []
+    if scene == "room":
+        while len(boxes) < 40:
+            h = 0.5 * rng.uniform(0.5, 3.0, 3)
+            c = rng.uniform(-13.0, 13.0, 2)
+            if abs(c[0]) < 6.5 and abs(c[1]) < 3.5:
+                continue  # the sensor's way
+            boxes.append((c[0], c[1], h[2], *h, rng.uniform(0.0, math.pi)))
+    else:
+        for side in (-1.0, 1.0):
+            length, back, height = rng.uniform(5.0, 7.0), rng.uniform(8.0, 12.0), rng.uniform(6.0, 25.0)
+            px = rng.uniform(0.0, STREET_LEN)
+            for rep in range(-6, 7):
+                x = rep * STREET_LEN
+                boxes.append((x + 0.5 * length, side * (back + 6.0), 0.5 * (height - 5.0),
+                              0.5 * length, 6.0, 0.5 * (height + 5.0), 0.0))
+                poles.append((x + px, side * 6.5, -5.0, 6.0))
+    return boxes, poles
+
+
+def _slab(o, d, lo, hi):
+    """Distance to an axis-aligned box along rays (its exit from inside), inf
+    for a miss."""
+    inv = 1.0 / d
+    a, b = (lo - o) * inv, (hi - o) * inv
+    near, far = torch.minimum(a, b).amax(-1), torch.maximum(a, b).amin(-1)
+    t = torch.where(near > 1e-6, near, far)
+    return torch.where((near <= far) & (far > 1e-6), t, torch.full_like(t, float("inf")))
+
+
+def _cast(scene, boxes, poles, o, d):
+    f = dict(dtype=torch.float32, device=o.device)
+    if scene == "room":
+        best = _slab(o, d, torch.tensor([-15.0, -15.0, 0.0], **f), torch.tensor([15.0, 15.0, 6.0], **f))
+    else:
+        n = torch.tensor([0.0, -0.005, 1.0], **f)
+        t = -(o @ n) / (d @ n)
+        y = o[..., 1] + t * d[..., 1]
+        best = torch.where((t > 1e-6) & (y.abs() <= 40.0), t, torch.full_like(t, float("inf")))
+    for cx, cy, cz, hx, hy, hz, yaw in boxes:
+        q, e = o - torch.tensor([cx, cy, cz], **f), d
+        if yaw:
+            c, s = math.cos(yaw), math.sin(yaw)
+            M = torch.tensor([[c, -s, 0.0], [s, c, 0.0], [0.0, 0.0, 1.0]], **f)
+            q, e = q @ M, e @ M
+        h = torch.tensor([hx, hy, hz], **f)
+        best = torch.minimum(best, _slab(q, e, -h, h))
+    for px, py, z0, z1 in poles:
+        ox, oy = o[..., 0] - px, o[..., 1] - py
+        a = d[..., 0] ** 2 + d[..., 1] ** 2
+        b = ox * d[..., 0] + oy * d[..., 1]
+        t = (-b - (b * b - a * (ox * ox + oy * oy - 0.09)).sqrt()) / a  # NaN for a miss
+        z = o[..., 2] + t * d[..., 2]
+        best = torch.where((t > 1e-6) & (z > z0) & (z < z1) & (t < best), t, best)
+    return best
+
+
+class Drive:
+    """One closed sequence of `ring` scans in HBM: a rosette pattern over
+    360 deg azimuth and -7..52 deg elevation ray-cast into a room (30 x 30 x
+    6 m, 40 boxes) or a street (facades, poles, 15 % foliage), range noise
+    N(0, 0.02 m), 0.1-40 m; with raw, each return at its own pose along the
+    0.1 s sweep, and a 200 Hz IMU with white noise and biases."""
+
+    def __init__(self, scene, sizes, seed, raw):
+        self.scene, self.ring, self.raw = scene, len(sizes), raw
+        self.period = SCAN_DT * self.ring
+        rng = np.random.default_rng([seed, 1])
+        self.boxes, self.poles = _scene(scene, rng)
+        self.gen = torch.Generator(device=DEV).manual_seed(int(rng.integers(1 << 62)))
+        sizes = torch.tensor(sizes, device=DEV)
+        share = min(self._cast(4096)[1].sum(1).min().item() / 4096.0, 1.0)
+        rays = int(float(sizes.max()) / share * 1.03) + 64
+        while True:
+            pts, ok = self._cast(rays)
+            if bool((ok.sum(1) >= sizes).all()):
+                break
+            rays += rays // 10
+        keep = ok & (ok.cumsum(1) <= sizes[:, None])
+        flat = pts[:, keep].contiguous()
+        off = np.concatenate([[0], np.cumsum(sizes.cpu().numpy())])
+        self.scans = [flat[:, off[k] : off[k + 1]].contiguous() for k in range(self.ring)]  # each [4, n]: x y z t_ms
+        self.counts = [int(s.shape[1]) for s in self.scans]
+        self._imu(rng)
+        self.steps = []  # the motion prior into scan k of the ring
+        for k in range(self.ring):
+            (R0, p0), (R1, p1) = self.pose(SCAN_DT * k), self.pose(SCAN_DT * (k + 1))
+            e = np.radians(0.2) * rng.standard_normal(3)
+            self.steps.append((R0.T @ R1 @ _exp(e), R0.T @ (p1 - p0) + 0.02 * rng.standard_normal(3)))
+
+    def pose(self, t):
+        return _pose(self.scene, self.period, t)
+
+    def _cast(self, rays):
+        f = dict(dtype=torch.float64, device=DEV)
+        j = torch.arange(rays, **f)
+        k = torch.arange(self.ring, **f)[:, None]
+        when = (k + j / rays) if self.raw else (k + 1.0 + 0.0 * j)
+        x, y, z, ro, pi, ya = _trajectory(torch, self.scene, self.period, SCAN_DT * when)
+        fa = 0.7548776662466927 * j + 0.1370 * k
+        fe = 0.5698402909980532 * j + 0.4210 * k
+        az = 2.0 * math.pi * (fa - fa.floor())
+        el = math.radians(-7.0) + math.radians(59.0) * (fe - fe.floor())
+        dl = torch.stack([el.cos() * az.cos(), el.cos() * az.sin(), el.sin()], -1)
+        a, b, c = dl.unbind(-1)
+        b, c = ro.cos() * b - ro.sin() * c, ro.sin() * b + ro.cos() * c
+        a, c = pi.cos() * a + pi.sin() * c, -pi.sin() * a + pi.cos() * c
+        a, b = ya.cos() * a - ya.sin() * b, ya.sin() * a + ya.cos() * b
+        o, d = torch.stack([x, y, z], -1).float(), torch.stack([a, b, c], -1).float()
+        r = _cast(self.scene, self.boxes, self.poles, o, d).double()
+        if self.scene == "street":
+            u = torch.rand((2, *r.shape), generator=self.gen, **f)
+            r = torch.where(u[0] < 0.15, r.clamp(max=40.0) * (0.05 + 0.95 * u[1]), r)
+        m = r + 0.02 * torch.randn(r.shape, generator=self.gen, **f)
+        ok = (r <= 40.0) & (m >= 0.1) & (m <= 40.0)
+        t_ms = (100.0 * j / rays).expand_as(m)
+        m = torch.where(ok, m, torch.zeros_like(m))
+        return torch.cat([(m[..., None] * dl).movedim(-1, 0), t_ms[None]]).float(), ok
+
+    def _imu(self, rng):
+        m = 20 * self.ring
+        t = IMU_DT * np.arange(m)
+        self.acc, self.gyro = np.empty((m, 3)), np.empty((m, 3))
+        bg, ba = 2e-3 * rng.standard_normal(3), 1e-2 * rng.standard_normal(3)
+        h = 1e-3
+        for q in range(m):
+            (Rm, pm), (R, p), (Rp, pp) = (self.pose(t[q] + s) for s in (-h, 0.0, h))
+            W = Rm.T @ Rp
+            self.gyro[q] = np.array([W[2, 1] - W[1, 2], W[0, 2] - W[2, 0], W[1, 0] - W[0, 1]]) / (4.0 * h)
+            self.acc[q] = R.T @ ((pp - 2.0 * p + pm) / (h * h) + [0.0, 0.0, G])
+        self.gyro += bg + 1e-3 * rng.standard_normal((m, 3))
+        self.acc += ba + 1e-2 * rng.standard_normal((m, 3))
+        R, _ = self.pose(0.0)
+        self.rest = (1.0 + IMU_DT * np.arange(-20, 0), R.T @ [0.0, 0.0, G] + ba + 1e-2 * rng.standard_normal((20, 3)),
+                     bg + 1e-3 * rng.standard_normal((20, 3)))
+        self.ends = [float(s[3, -1]) / 1000.0 for s in self.scans]
+        first = [int(math.ceil((SCAN_DT * k + e) / IMU_DT)) for k, e in enumerate(self.ends)]
+        spans = list(zip([first[-1] - m] + first[:-1], first)) + [(0, first[0])]  # the last: the first lap's scan 0
+        self.samples = [(np.arange(a, b), self.acc[np.arange(a, b) % m], self.gyro[np.arange(a, b) % m])
+                        for a, b in spans]
+
+    def package(self, k):
+        """(ring index, IMU samples, cloud start, cloud end) of the k-th
+        package; the clock starts at 1 s."""
+        lap, i = divmod(k, self.ring)
+        j, acc, gyro = self.samples[i if k else -1]
+        start = 1.0 + SCAN_DT * k
+        return i, (1.0 + IMU_DT * (j + 20 * self.ring * lap), acc, gyro), start, start + self.ends[i]
+
+    def start_state(self, s, t):
+        """The state at clock time t of the first lap (a known start)."""
+        s = s.copy()
+        R, p = self.pose(t)
+        s[0:3], s[3:12] = p, R.T.reshape(-1)
+        s[24:27] = (self.pose(t + 1e-3)[1] - self.pose(t - 1e-3)[1]) / 2e-3
+        return s
+
+
+def _exp(w):
+    """Rotation matrix of a rotation vector (Rodrigues)."""
+    th = math.sqrt(float(w @ w))
+    K = np.array([[0, -w[2], w[1]], [w[2], 0, -w[0]], [-w[1], w[0], 0]])
+    if th < 1e-10:
+        return np.eye(3) + K
+    return np.eye(3) + math.sin(th) / th * K + 2.0 * (math.sin(0.5 * th) / th) ** 2 * (K @ K)
+
+
+def _sizes(case, rng, ring, log=False):
+    if not case["n_min"]:
+        return [case["n"]] * ring
+    if log:
+        return [int(v) for v in np.exp(rng.uniform(math.log(case["n_min"]), math.log(case["n"] + 1), ring))]
+    return [int(v) for v in rng.integers(case["n_min"], case["n"] + 1, ring)]
+
+
+def _drives(case, seed):
+    rng = np.random.default_rng([case["n"], case["n_min"], 2])  # sizes belong to the case
+    raw = case["kind"] in ("imu", "node", "log", "batch")
+    out = []
+    for i in range(case["sessions"]):
+        scene = case["scene"] if case["scene"] != "mixed" else ("room", "street")[i % 2]
+        sizes = _sizes(case, rng, case["ring"], case["kind"] == "serve")
+        if case["kind"] in ("observe", "odom"):
+            sizes[0] = _map_points(case)
+        out.append(Drive(scene, sizes, seed * 1000 + i, raw))
+    return out
+
+
+def _map_points(case):
+    """Points of the sweep the map is built from where the scans that follow
+    are too sparse to fit planes by themselves."""
+    return max(case["n"], 20000)
+
+
+def _config(case):
+    most = _map_points(case) if case["kind"] in ("observe", "odom") else case["n"]
+    return LIOConfig(map_capacity=case["capacity"], max_scan_points=most, scan_resolution=case["resolution"],
+                     estimate_ext=int(case["estimate_ext"]))
+
+
+# --------------------------------------------------------------------------
+# the program's side
+# --------------------------------------------------------------------------
+class _Program:
+    """What a host program holds: contexts, sessions, its sequences."""
+
+    def __init__(self, case, seed):
+        self.case, self.k = case, 0
+        self.drives = _drives(case, seed)
+        self.drive = self.drives[0]
+        self.cfg = _config(case)
+        self.ctxs, self.regs, self.server = [], [], None
+
+    def context(self):
+        self.ctxs.append(Context(0))
+        return self.ctxs[-1]
+
+    def bind_raw(self, reg, drive, k):
+        i, imu, start, end = drive.package(k)
+        s = drive.scans[i]
+        p, row = s.data_ptr(), s.stride(0) * 4
+        reg.set_raw_device(p, p + row, p + 2 * row, p + 3 * row, drive.counts[i], imu, start, end)
+
+    def bind_points(self, reg, drive, i, most):
+        s = drive.scans[i]
+        p, row = s.data_ptr(), s.stride(0) * 4
+        reg.set_points_device(p, p + row, p + 2 * row, min(drive.counts[i], most))
+
+    def first_map(self, reg, drive):
+        """IMU_INIT at rest, the start's pose and speed, MAP_INIT."""
+        assert reg.imu_init(drive.rest, 1.0)
+        s, P = reg.get_state()
+        reg.set_state(drive.start_state(s, 0.0), P)
+        self.bind_raw(reg, drive, 0)
+        reg.build()
+
+    def close(self):
+        for r in self.regs:
+            r.close()
+        if self.server:
+            self.server.close()
+        for c in self.ctxs:
+            c.close()
+        self.regs, self.ctxs, self.server = [], [], None
+
+    def __del__(self):
+        self.close()
+
+
+def _ints(*structs):
+    """The counters of statistics structures as one integer array."""
+    return np.concatenate([np.frombuffer(s, np.int32) for s in structs])
+
+
+MAP_INTS = 11  # counters up to the maintenance flags; the rest describe the replay's schedule
+
+
+class _Observe(_Program):
+    def __init__(self, case, seed):
+        super().__init__(case, seed)
+        d = self.drive
+        reg = Registrar(self.context(), self.cfg)
+        self.regs = [reg]
+        s0, self.x = _observe_states(d)
+        reg.set_state(s0, _observe_cov())
+        self.bind_points(reg, d, 0, d.counts[0])
+        reg.build()
+        self.bind_points(reg, d, 1, d.counts[1])
+
+    def run(self):
+        H, b, o = self.regs[0].observe(self.x)
+        return {"H": H, "b": b, "counts": _ints(o)}
+
+
+class _Odom(_Program):
+    def __init__(self, case, seed):
+        super().__init__(case, seed)
+        reg = Registrar(self.context(), self.cfg)
+        self.regs = [reg]
+        R, p = self.drive.pose(SCAN_DT)
+        reg.set_state(state_vector(R, p), initial_covariance())
+        self.bind_points(reg, self.drive, 0, self.drive.counts[0])
+        reg.build()
+
+    def run(self):
+        self.k += 1
+        i = self.k % self.case["ring"]
+        reg = self.regs[0]
+        reg.apply_motion(*self.drive.steps[i], QDIAG)
+        self.bind_points(reg, self.drive, i, self.case["n"])
+        o, m = reg.register_noalloc() if self.case["noalloc"] else reg.register()
+        x, P = reg.get_state()
+        return {"x": x, "P": P, "counts": _ints(o, m)[: 6 + MAP_INTS]}
+
+
+class _Imu(_Program):
+    def __init__(self, case, seed):
+        super().__init__(case, seed)
+        self.regs = [Registrar(self.context(), self.cfg)]
+        self.first_map(self.regs[0], self.drive)
+
+    def run(self):
+        self.k += 1
+        reg = self.regs[0]
+        self.bind_raw(reg, self.drive, self.k)
+        o, m = reg.register()
+        x, P = reg.get_state()
+        return {"x": x, "P": P, "counts": _ints(o, m)[: 6 + MAP_INTS]}
+
+
+class _Node(_Program):
+    def __init__(self, case, seed):
+        super().__init__(case, seed)
+        self.lio = LIOBuilder(self.context(), self.cfg)
+        self.regs = [self.lio.reg]
+        self.host = [s.cpu().numpy() for s in self.drive.scans]
+        self.lio.process(*self.host[0], self.drive.rest, 0.9, 1.0)
+        reg = self.lio.reg
+        s, P = reg.get_state()
+        reg.set_state(self.drive.start_state(s, 0.0), P)
+        self.process()
+        assert self.lio.status == LIO_MAPPING
+
+    def process(self):
+        i, imu, start, end = self.drive.package(self.k)
+        self.lio.process(*self.host[i], imu, start, end)
+        self.k += 1
+
+    def run(self):
+        self.process()
+        reg = self.lio.reg
+        pos, quat, cov = reg.odom()
+        return {"pos": pos, "quat": quat, "cov": cov, "cloud": reg.export_cloud_body(),
+                "counts": _ints(self.lio.last_obs, self.lio.last_map)[: 6 + MAP_INTS]}
+
+
+class _Log(_Program):
+    def __init__(self, case, seed):
+        super().__init__(case, seed)
+        self.context()
+
+    def run(self):
+        with Registrar(self.ctxs[0], self.cfg) as reg:
+            self.first_map(reg, self.drive)
+            for k in range(1, self.case["scans"]):
+                self.bind_raw(reg, self.drive, k)
+                reg.register()
+            x, P = reg.get_state()
+            return {"x": x, "P": P, **self.whole(reg.export_map())}
+
+    def whole(self, m):
+        """The map in arrays of the capacity's size."""
+        return {f: np.pad(a, [(0, self.case["capacity"] - len(a))] + [(0, 0)] * (a.ndim - 1)) for f, a in m.items()}
+
+
+class _Batch(_Program):
+    def __init__(self, case, seed):
+        super().__init__(case, seed)
+        n, g = case["sessions"], case["groups"]
+        ctxs = [self.context() for _ in range(g)]
+        self.members = [[i for i in range(n) if (i // 2) % g == j] for j in range(g)]
+        self.members = [m for m in self.members if m]
+        self.regs = [Registrar(ctxs[(i // 2) % g], self.cfg) for i in range(n)]
+        for reg, d in zip(self.regs, self.drives):
+            self.first_map(reg, d)
+
+    def bind(self, members):
+        a = []
+        for i in members:
+            d = self.drives[i]
+            j, imu, start, end = d.package(self.k)
+            s = d.scans[j]
+            p, row = s.data_ptr(), s.stride(0) * 4
+            a.append((p, p + row, p + 2 * row, p + 3 * row, d.counts[j], imu, start, end))
+        set_raw_device_batch([self.regs[i] for i in members], *zip(*a))
+
+    def run(self):
+        self.k += 1
+        counts = [None] * len(self.regs)
+        for m in self.members:
+            self.bind(m)
+            regs = [self.regs[i] for i in m]
+            if len(self.members) == 1:
+                o, mm = register_batch(regs)
+            else:
+                register_batch_submit(regs)
+        for m in self.members:
+            if len(self.members) > 1:
+                o, mm = register_batch_wait(self.regs[m[0]].ctx, len(m))
+            for q, i in enumerate(m):
+                counts[i] = _ints(o[q], mm[q])[: 6 + MAP_INTS]
+        x, P = zip(*(r.get_state() for r in self.regs))
+        return {"x": np.stack(x), "P": np.stack(P), "counts": np.stack(counts)}
+
+
+class _Serve(_Program):
+    REQ = np.dtype({"names": ["status", "kind", "iterations", "rot", "pos"],
+                    "formats": ["i4", "i4", "i4", ("f8", 9), ("f8", 3)],
+                    "offsets": [getattr(Request, f).offset for f in ("status", "kind", "iterations", "rot", "pos")],
+                    "itemsize": Request.pos.offset + 24})
+
+    def __init__(self, case, seed):
+        super().__init__(case, seed)
+        n, r = case["sessions"], case["scans"]
+        self.server = Server(self.cfg, n, executors=case["groups"], max_batch_sessions=-(-n // case["groups"]))
+        for i, d in enumerate(self.drives):
+            R, p = d.pose(SCAN_DT)
+            self.server.session_init(i, state_vector(R, p), initial_covariance())
+
+        def burst(scans):
+            return make_requests([self.request(i, d, k) for k in scans for i, d in enumerate(self.drives)])
+
+        self.server.run(burst([0]), QDIAG)  # MAP_INIT
+        ring = case["ring"]
+        self.bursts = [burst([(r * q + k + 1) % ring for k in range(r)]) for q in range(ring // r)]
+
+    def request(self, session, d, k):
+        s = d.scans[k]
+        p, row = s.data_ptr(), s.stride(0) * 4
+        R, t = d.steps[k]
+        return dict(session=session, n=d.counts[k], x=p, y=p + row, z=p + 2 * row, dR=R, dp=t, arrival=0.0)
+
+    def run(self):
+        reqs = self.bursts[self.k % len(self.bursts)]
+        self.k += 1
+        self.server.run(reqs, QDIAG)
+        a = np.frombuffer(reqs, self.REQ)
+        return {"rot": a["rot"].copy(), "pos": a["pos"].copy(),
+                "counts": np.stack([a["status"], a["kind"], a["iterations"]])}
+
+
+_KINDS = {"observe": _Observe, "odom": _Odom, "imu": _Imu, "node": _Node, "log": _Log, "batch": _Batch,
+          "serve": _Serve}
+
+
+def prepare(case, seed):
+    return _KINDS[case["kind"]](case, seed)
+
+
+def run(state):
+    return state.run()
+
+
+def _observe_states(d):
+    """The pose the map was built at, and a guess at the next scan's pose."""
+    (R0, p0), (dR, dp) = d.pose(SCAN_DT), d.steps[1]
+    return state_vector(R0, p0), state_vector(R0 @ dR, p0 + R0 @ dp)
+
+
+def _observe_cov():
+    return initial_covariance() * 1e-3
+
+
+# --------------------------------------------------------------------------
+# the first pass in 64 bits
+# --------------------------------------------------------------------------
+def exact(case, seed):
+    """Plain numpy in 64 bits, except where the path is defined in 32: the
+    inserted points (PCL's fp32 transform) and the filtered cloud."""
+    kind = case["kind"]
+    if kind in ("batch", "serve"):
+        return None
+    if kind != "observe" and case["n"] * (case["scans"] if kind == "log" else 1) > 6 * EXACT_POINTS:
+        return None
+    if kind in ("odom", "imu", "node") and case["n"] > EXACT_POINTS:
+        return None
+    d = _drives(case, seed)[0]
+    host = [s.cpu().numpy() for s in d.scans[: max(2, case["scans"])]]
+    ref = _Ref(case)
+    if kind == "observe":
+        s0, x = _observe_states(d)
+        ref.set(s0, _observe_cov())
+        ref.build(host[0][:3])
+        ref.scan(host[1][:3])
+        ref.x = _State(x)
+        H, b = ref.observe(ref.x)
+        return {"H": H, "b": b, "counts": None}
+    if kind == "odom":
+        R, p = d.pose(SCAN_DT)
+        ref.set(state_vector(R, p), initial_covariance())
+        ref.build(host[0][:3])
+        dR, dp = d.steps[1]
+        ref.x.pos = ref.x.pos + ref.x.rot @ dp
+        ref.x.rot = ref.x.rot @ dR
+        ref.P = ref.P + np.diag(QDIAG)
+        ref.register(host[1][:3])
+        return {"x": ref.x.flat(), "P": ref.P, "counts": None}
+    ref.imu_init(d.rest)
+    ref.x = _State(d.start_state(ref.x.flat(), 0.0))
+    ref.build(ref.undistort(host[0], *d.package(0)[1:]))
+    for k in range(1, max(2, case["scans"])):
+        cloud = ref.undistort(host[k], *d.package(k)[1:])
+        ref.register(ref.filtered(cloud))
+    if kind == "node":
+        q = _quat(ref.x.rot)
+        return {"pos": ref.x.pos, "quat": q, "cov": ref.P[:6, :6], "cloud": cloud, "counts": None}
+    out = {"x": ref.x.flat(), "P": ref.P}
+    return {**out, "counts": None} if kind == "imu" else {**out, **ref.export()}
+
+
+def _hat(v):
+    """Cross-product matrices of vectors (..., 3)."""
+    v = np.asarray(v)
+    z = np.zeros(v.shape[:-1])
+    return np.stack([np.stack([z, -v[..., 2], v[..., 1]], -1), np.stack([v[..., 2], z, -v[..., 0]], -1),
+                     np.stack([-v[..., 1], v[..., 0], z], -1)], -2)
+
+
+def _quat(R):
+    """(w, x, y, z) of a rotation by less than half a turn."""
+    w = 0.5 * math.sqrt(1.0 + np.trace(R))
+    return np.array([w, *(np.array([R[2, 1] - R[1, 2], R[0, 2] - R[2, 0], R[1, 0] - R[0, 1]]) / (4.0 * w))])
+
+
+def _log(R):
+    q = _quat(R)
+    n = math.sqrt(float(q[1:] @ q[1:]))
+    return 2.0 * q[1:] / q[0] if n < 1e-10 else 2.0 * math.atan(n / q[0]) / n * q[1:]
+
+
+def _jr(w):
+    """Right Jacobian of SO(3)."""
+    th2 = float(w @ w)
+    K = _hat(w)
+    if th2 < 1e-10:
+        return np.eye(3) - 0.5 * K
+    th = math.sqrt(th2)
+    return np.eye(3) - (1.0 - math.cos(th)) / th2 * K + (th - math.sin(th)) / (th2 * th) * (K @ K)
+
+
+class _State:
+    def __init__(self, s):
+        s = np.asarray(s, np.float64)
+        self.pos, self.rot, self.rot_ext, self.pos_ext = s[0:3], s[3:12].reshape(3, 3).T, s[12:21].reshape(3, 3).T, s[21:24]
+        self.vel, self.bg, self.ba, self.g = s[24:27], s[27:30], s[30:33], s[33:36]
+
+    def flat(self):
+        return np.concatenate([self.pos, self.rot.T.reshape(-1), self.rot_ext.T.reshape(-1), self.pos_ext, self.vel,
+                               self.bg, self.ba, self.g])
+
+    def bx(self):
+        a, b, c = self.g
+        return np.array([[-b, -c], [G - b * b / (G + a), -c * b / (G + a)], [-c * b / (G + a), G - c * c / (G + a)]]) / G
+
+    def mx(self, r=None):
+        if r is None:
+            return -_hat(self.g) @ self.bx()
+        u = self.bx() @ r
+        return -_exp(u) @ _hat(self.g) @ _jr(u) @ self.bx()
+
+    def nx(self):
+        return self.bx().T @ _hat(self.g) / (G * G)
+
+    def plus(self, d):
+        s = _State(self.flat())
+        s.pos, s.rot, s.rot_ext, s.pos_ext = s.pos + d[0:3], s.rot @ _exp(d[3:6]), s.rot_ext @ _exp(d[6:9]), s.pos_ext + d[9:12]
+        s.vel, s.bg, s.ba = s.vel + d[12:15], s.bg + d[15:18], s.ba + d[18:21]
+        s.g = _exp(self.bx() @ d[21:23]) @ self.g
+        return s
+
+    def minus(self, o):
+        h = _hat(self.g) @ o.g
+        vs, vc = math.sqrt(float(h @ h)), float(self.g @ o.g)
+        r = np.zeros(2) if vs < 1e-11 else math.atan2(vs, vc) / vs * (o.bx().T @ _hat(o.g) @ self.g)
+        return np.concatenate([self.pos - o.pos, _log(o.rot.T @ self.rot), _log(o.rot_ext.T @ self.rot_ext),
+                               self.pos_ext - o.pos_ext, self.vel - o.vel, self.bg - o.bg, self.ba - o.ba, r])
+
+
+class _Voxel:
+    __slots__ = ("key", "n", "mean", "pts", "covs", "held", "init", "plane", "enabled", "fresh", "norm", "tn", "tm", "group")
+
+    def __init__(self, key, group):
+        self.key, self.group = key, group
+        self.n, self.mean, self.norm, self.tn, self.tm = 0, np.zeros(3), np.zeros(3), 0.0, 0.0
+        self.pts, self.covs, self.held, self.fresh = [], [], 0, 0
+        self.init = self.plane = False
+        self.enabled = True
+
+
+class _Ref:
+    """The registration path restated in numpy: voxel map, IESKF, IMU side."""
+
+    def __init__(self, case):
+        self.cfg = _config(case)
+        self.map, self.groups = {}, 0  # key -> _Voxel, oldest first
+        n = self.cfg.max_scan_points
+        self.slots = np.zeros(n, bool), np.zeros((n, 3)), np.zeros((n, 3)), np.zeros(n)
+        self.Q = np.diag([0.01] * 6 + [0.0001] * 6)
+        self.last_end = 0.0
+        self.last_acc = self.last_gyro = np.zeros(3)
+
+    def set(self, s, P):
+        self.x, self.P = _State(s), np.array(P, np.float64)
+
+    # ---- points
+    def body_cov(self, p):
+        r2 = (p * p).sum(1)
+        d = p / np.sqrt(r2)[:, None]
+        dd = d[:, :, None] * d[:, None, :]
+        s = math.sin(math.radians(self.cfg.angle_cov)) ** 2
+        return self.cfg.ranging_cov**2 * dd + (r2 * s)[:, None, None] * (np.eye(3) - dd)
+
+    def scan(self, xyz):
+        p = np.asarray(xyz, np.float64).T.copy()
+        p[p[:, 2] == 0, 2] = 0.001
+        self.f32 = np.asarray(xyz, np.float32)
+        self.p, self.cov = p, self.body_cov(p)
+        # the residual slots keep what earlier scans left at an index
+        self.valid, self.norm, self.pmean, self.res = (a[: len(p)] for a in self.slots)
+
+    def world_cov(self, x):
+        R, H = x.rot @ x.rot_ext, _hat(self.p)
+        return R @ self.cov @ R.T + H @ self.P[3:6, 3:6] @ H.transpose(0, 2, 1) + self.P[0:3, 0:3]
+
+    def inserted(self):
+        """World points in fp32 (m0 x + (m1 y + (m2 z + t))), keys, covariances."""
+        R = (self.x.rot @ self.x.rot_ext).astype(np.float32)
+        t = (self.x.rot @ self.x.pos_ext + self.x.pos).astype(np.float32)
+        X, Y, Z = self.f32
+        w = np.stack([R[i, 0] * X + (R[i, 1] * Y + (R[i, 2] * Z + t[i])) for i in range(3)], 1).astype(np.float64)
+        return w, self.keys(w), self.world_cov(self.x)
+
+    def keys(self, w):
+        k = np.floor(w / self.cfg.voxel_size).astype(np.int64) + (1 << 20)
+        return (k[:, 0] << 42) | (k[:, 1] << 21) | k[:, 2]
+
+    # ---- map
+    def touch(self, k):
+        v = self.map.pop(k, None)
+        if v is None:
+            v = _Voxel(k, self.groups)
+            self.groups += 1
+            if len(self.map) >= self.cfg.map_capacity:
+                del self.map[next(iter(self.map))]
+        self.map[k] = v
+        return v
+
+    def build(self, xyz):
+        self.scan(xyz)
+        w, keys, cov = self.inserted()
+        order = np.argsort(keys, kind="stable")
+        uniq, first, count = np.unique(keys[order], return_index=True, return_counts=True)
+        seg = dict(zip(uniq.tolist(), zip(first.tolist(), count.tolist())))
+        for k in keys.tolist():
+            self.touch(k)
+        for k, v in self.map.items():
+            a, c = seg[k]
+            at = order[a : a + c]
+            v.n = v.held = c
+            v.pts, v.covs = list(w[at]), list(cov[at])
+            v.mean = w[at].mean(0)
+            self.fit(v)
+
+    def fit(self, v):
+        if v.n < self.cfg.update_size_thresh:
+            return
+        v.init = True
+        p, cov = np.array(v.pts) - v.mean, np.array(v.covs)
+        ev, V = np.linalg.eigh(p.T @ p / v.n)
+        v.plane = bool(ev[0] <= self.cfg.plane_thresh)
+        if not v.plane:
+            return
+        n0 = V[:, 0]
+        for m in (1, 2):
+            em = V[:, m]
+            F = p @ (np.outer(em, n0) + np.outer(n0, em)) / (v.n * (ev[0] - ev[m]))
+            v.tn += float(np.einsum("ni,nij,nj->", F, cov, F))
+        v.tm += float(np.trace(cov.sum(0))) / (v.n * v.n)
+        v.norm = -n0 if v.mean @ n0 > 0 else n0
+
+    def push(self, v, p, c):
+        if v.init and not v.enabled:
+            if v.plane:
+                self.merge(v)
+            return
+        v.mean = v.mean + (p - v.mean) / (v.n + 1.0)
+        v.n += 1
+        v.pts.append(p)
+        v.covs.append(c)
+        v.held += 1
+        if not v.init:
+            return self.fit(v)
+        v.fresh += 1
+        if v.fresh >= self.cfg.update_size_thresh:
+            self.fit(v)
+            v.fresh = 0
+        if v.held >= self.cfg.max_point_thresh:
+            v.enabled, v.held, v.pts, v.covs = False, 0, [], []
+
+    def merge(self, v):
+        for step in (-(1 << 42), -(1 << 21), -1, 1 << 42, 1 << 21, 1):
+            o = self.map.get(v.key + step)
+            if o is None or o.group == v.group or o.enabled or not o.plane:
+                continue
+            if (1.0 - o.norm @ v.norm > self.cfg.merge_thresh_for_angle
+                    or abs(o.norm @ o.mean - v.norm @ v.mean) > self.cfg.merge_thresh_for_distance):
+                continue
+            a, b = v.tn + v.tm, o.tn + o.tm
+            mean = v.tm * o.mean + o.tm * v.mean / (v.tm + o.tm)
+            norm = v.tn * o.norm + o.tn * v.norm / (v.tn + o.tn)
+            norm = -norm if mean @ norm > 0 else norm
+            tn, tm = ((a * a * o.tn + b * b * v.tn) / (a + b) ** 2, (a * a * o.tm + b * b * v.tm) / (a + b) ** 2)
+            o.group = v.group
+            for q in (v, o):
+                q.mean, q.norm, q.tn, q.tm = mean, norm, tn, tm
+
+    def insert(self):
+        w, keys, cov = self.inserted()
+        for k, p, c in zip(keys.tolist(), w, cov):
+            self.push(self.touch(k), p, c)
+
+    def export(self):
+        dbl = np.array([[*v.mean, *v.norm, v.tn, v.tm] for v in reversed(self.map.values())])
+        return {"keys": None, "ints": None, "group": None,
+                "dbl": np.pad(dbl, [(0, self.cfg.map_capacity - len(dbl)), (0, 0)])}
+
+    # ---- filter
+    def observe(self, x):
+        R = x.rot @ x.rot_ext
+        w = self.p @ R.T + (x.rot @ x.pos_ext + x.pos)
+        keys = np.array(list(self.map.keys()), np.int64)
+        order = np.argsort(keys)
+        vox = list(self.map.values())
+        plane, mean, norm = (np.array([getattr(v, f) for v in vox])[order] for f in ("plane", "mean", "norm"))
+        k = self.keys(w)
+        at = np.minimum(np.searchsorted(keys[order], k), len(vox) - 1)
+        hit = keys[order][at] == k
+        on = hit & plane[at]
+        self.valid[hit] = False
+        self.norm[on], self.pmean[on] = norm[at[on]], mean[at[on]]
+        r = ((w - self.pmean) * self.norm).sum(1)
+        self.res[on] = r[on]
+        s = np.einsum("ni,nij,nj->n", self.norm, self.world_cov(x), self.norm)
+        self.valid[on] = (np.abs(r) < 3.0 * np.sqrt(s))[on]
+        v = self.valid
+        n, p = self.norm[v], self.p[v]
+        nr = n @ R
+        info = np.einsum("ni,nij,nj->n", nr, self.cov[v], nr)
+        info = np.where(info < 0.0002, 5000.0, 1.0 / info)
+        J = np.zeros((len(n), 12))
+        J[:, 0:3] = n
+        J[:, 3:6] = -np.einsum("ni,nij->nj", n @ x.rot, _hat(p @ x.rot_ext.T + x.pos_ext))
+        if self.cfg.estimate_ext:
+            J[:, 6:9] = -np.einsum("ni,nij->nj", nr, _hat(p))
+            J[:, 9:12] = n @ x.rot
+        Ji = J * info[:, None]
+        return Ji.T @ J, Ji.T @ self.res[v]
+
+    def jacobian(self, xp, d):
+        J = np.eye(23)
+        J[3:6, 3:6], J[6:9, 6:9] = _jr(d[3:6]), _jr(d[6:9])
+        J[21:23, 21:23] = self.x.nx() @ xp.mx(d[21:23])
+        return J
+
+    def register(self, xyz):
+        self.scan(xyz)
+        xp, Pinv = self.x, np.linalg.inv(self.P)
+        for _ in range(self.cfg.max_iter):
+            H, b = self.observe(self.x)
+            d = self.x.minus(xp)
+            J = self.jacobian(xp, d)
+            JtP = J.T @ Pinv
+            A, c = JtP @ J, JtP @ d
+            A[:12, :12] += H
+            c[:12] += b
+            d = -np.linalg.solve(A, c)
+            self.x = self.x.plus(d)
+            if d.max() < 1e-3:
+                break
+        L = self.jacobian(xp, d)
+        self.P = L @ np.linalg.inv(A) @ L.T
+        self.insert()
+
+    # ---- IMU side
+    def imu_init(self, imu):
+        t, acc, gyro = imu
+        a = acc.mean(0)
+        self.gravity = math.sqrt(float(a @ a))
+        x = _State(state_vector())
+        x.bg = gyro.mean(0)
+        u, v = -a / self.gravity, np.array([0.0, 0.0, -1.0])
+        w, c = np.cross(u, v), float(u @ v)
+        K = _hat(w)
+        x.rot = np.eye(3) + K + K @ K / (1.0 + c)
+        self.x, self.P = x, initial_covariance()
+        self.last_imu = (t[-1], acc[-1], gyro[-1])
+        self.last_end = 1.0
+
+    def predict(self, acc, gyro, dt):
+        x = self.x
+        w = (gyro - x.bg) * dt
+        F, Gm = np.eye(23), np.zeros((23, 12))
+        F[0:3, 12:15] = np.eye(3) * dt
+        F[3:6, 3:6] = _exp(-w)
+        F[3:6, 15:18] = Gm[3:6, 0:3] = -_jr(w) * dt
+        F[12:15, 3:6] = -x.rot @ _hat(acc - x.ba) * dt
+        F[12:15, 18:21] = Gm[12:15, 3:6] = -x.rot * dt
+        F[12:15, 21:23] = x.mx() * dt
+        F[21:23, 21:23] = x.nx() @ x.mx()
+        Gm[15:18, 6:9] = Gm[18:21, 9:12] = np.eye(3) * dt
+        y = _State(x.flat())
+        y.pos, y.rot = x.pos + x.vel * dt, x.rot @ _exp(w)
+        y.vel = x.vel + (x.rot @ (acc - x.ba) + x.g) * dt
+        self.x, self.P = y, F @ self.P @ F.T + Gm @ self.Q @ Gm.T
+
+    def undistort(self, raw, imu, start, end):
+        seq = [self.last_imu] + list(zip(*imu))
+        knots = [(0.0, self.last_acc, self.last_gyro, self.x)]
+        for (t0, a0, g0), (t1, a1, g1) in zip(seq[:-1], seq[1:]):
+            if t1 < self.last_end:
+                continue
+            gyro, acc = 0.5 * (g0 + g1), 0.5 * (a0 + a1) * G / self.gravity
+            self.predict(acc, gyro, t1 - (self.last_end if t0 < self.last_end else t0))
+            self.last_gyro, self.last_acc = gyro - self.x.bg, self.x.rot @ (acc - self.x.ba) + self.x.g
+            knots.append((t1 - start, self.last_acc, self.last_gyro, self.x))
+        self.predict(acc, gyro, end - seq[-1][0])
+        self.last_imu, self.last_end = seq[-1], end
+        x = self.x
+        out = raw[:3].astype(np.float64).T
+        t = raw[3].astype(np.float64) / 1000.0
+        at = len(t) - 1
+        for (t0, _, _, h), (_, acc, gyro, _) in zip(knots[-2::-1], knots[:0:-1]):
+            while t[at] > t0:
+                dt = t[at] - t0
+                p = x.rot_ext @ out[at] + x.pos_ext
+                p = h.rot @ _exp(dt * gyro) @ p + h.pos + dt * h.vel + 0.5 * dt * dt * acc
+                p = x.rot_ext.T @ (x.rot.T @ (p - x.pos) - x.pos_ext)
+                out[at] = p.astype(np.float32)
+                if at == 0:
+                    break
+                at -= 1
+        return out.T.astype(np.float32)
+
+    def filtered(self, xyz):
+        """VoxelGrid: the fp32 mean of each leaf's points, leaves in index order."""
+        if self.cfg.scan_resolution <= 0:
+            return xyz
+        inv = np.float32(1.0) / np.float32(self.cfg.scan_resolution)
+        ijk = np.floor(xyz * inv) - np.floor(xyz.min(1, keepdims=True) * inv)
+        dim = np.floor(xyz.max(1) * inv) - np.floor(xyz.min(1) * inv) + 1
+        lin = (ijk[0] + ijk[1] * float(dim[0]) + ijk[2] * float(dim[0]) * float(dim[1])).astype(np.int64)
+        _, leaf, count = np.unique(lin, return_inverse=True, return_counts=True)
+        out = np.zeros((3, len(count)), np.float32)
+        for a in range(3):
+            np.add.at(out[a], leaf, xyz[a])
+        return out / count.astype(np.float32)
