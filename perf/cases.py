@@ -422,7 +422,7 @@ def _ints(*structs):
     return np.concatenate([np.frombuffer(s, np.int32) for s in structs])
 
 
-MAP_INTS = 11  # counters up to the maintenance flags; the rest describe the replay's schedule
+MAP_INTS = 10  # counters up to the map's size; the rest describe housekeeping and the replay's schedule
 
 
 class _Observe(_Program):
