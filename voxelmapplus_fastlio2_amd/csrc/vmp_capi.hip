@@ -355,8 +355,6 @@ struct vmp_session {
   double* partials = nullptr;
   int32_t* obs_ctr = nullptr;
   int32_t* obs_stat = nullptr;
-  int32_t* live = nullptr;
-  int32_t* nlive = nullptr;
   bool has_points = false;
   bool needs_check = false;  // device buffers bound, checked when the next step starts
   // IMU side: device state, the raw package bound for the next step
@@ -754,7 +752,7 @@ extern "C" int64_t vmp_session_bytes(const vmp_map_cfg* cfg) {
   Sizes z = sizes_for(*cfg);
   int64_t b = 0;
   b += z.hcap * int64_t(sizeof(HashEntry));
-  b += z.pool * int64_t(sizeof(VoxHot) + sizeof(VoxState) + 8 * kPlaneD + 8 * kMomD + 4 + 4);
+  b += z.pool * int64_t(sizeof(VoxHot) + sizeof(VoxState) + 8 * kPlaneD + 8 * kMomD + 4);
   b += z.pool * int64_t(std::max(cfg->update_size_thresh - 1, 1)) * kPendF * 4;
   b += z.qcap * 12;
   b += z.maxn * (3 * 4 + 16);
@@ -829,8 +827,6 @@ extern "C" int vmp_session_create(vmp_ctx* ctx, const vmp_map_cfg* cfg, vmp_sess
   ok &= dalloc(A, &s->partials, size_t(z.max_blocks) * kObsRowMax) == hipSuccess;
   ok &= dalloc(A, &s->obs_ctr, 8) == hipSuccess;
   ok &= dalloc(A, &s->obs_stat, 8) == hipSuccess;
-  ok &= dalloc(A, &s->live, size_t(z.pool)) == hipSuccess;
-  ok &= dalloc(A, &s->nlive, 1) == hipSuccess;
   ok &= dalloc(A, &s->imu, 1) == hipSuccess;
   ok &= dalloc(A, &s->own_t, maxn) == hipSuccess;
   if (cfg->scan_resolution > 0.0) {
@@ -854,9 +850,9 @@ extern "C" int vmp_session_create(vmp_ctx* ctx, const vmp_map_cfg* cfg, vmp_sess
   m.merge_d = cfg->merge_thresh_for_distance;
   m.vs64 = cfg->voxel_size;
   hipStream_t st = ctx->stream;
-  hipLaunchKernelGGL(k_rehash_clear, dim3(grid_for(std::min<int64_t>(z.hcap, 1 << 20), 256)), dim3(256), 0, st, m);
   MapCounters c0{};
   if (hipMemcpyAsync(m.ctr, &c0, sizeof(c0), hipMemcpyHostToDevice, st) != hipSuccess) return fail(VMP_EDEVICE);
+  hipLaunchKernelGGL(k_hash_init, dim3(grid_for(std::min<int64_t>(z.hcap, 1 << 20), 256)), dim3(256), 0, st, m);
   // residual slots start invalid (NaN residual), voxel records empty; all
   // stream-ordered so creating a session does not wait for other streams
   hipLaunchKernelGGL(k_init_slots, dim3(grid_for(maxn, 256)), dim3(256), 0, st, s->slots, maxn);
@@ -1855,77 +1851,117 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode) {
   return hipGetLastError() == hipSuccess ? VMP_OK : VMP_EDEVICE;
 }
 
-// housekeeping between scans: hash rebuild and LRU ring compaction (rare)
-static int maintain(vmp_ctx* ex, vmp_session* s, int32_t* did) {
-  *did = 0;
+// A table is rebuilt once a scan's new keys (at most one per point) could
+// take it past 5/8 full.  It holds at least 2 (capacity + scan points)
+// slots, so that leaves at least (capacity + scan points) / 4 tombstones
+// between two rebuilds of a full map; past 3/4 the probe sequences of the
+// eight-slot bricks grow long.
+static bool wants_rehash(const vmp_session* s) {
+  const int64_t hcap = int64_t(s->map.hmask) + 1;
+  return int64_t(s->h_ctr.used_entries) + int64_t(s->cfg.max_scan_points) > hcap / 8 * 5;
+}
+static bool wants_ring_compaction(const vmp_session* s) {
+  return s->h_ctr.ring_tail - s->h_ctr.ring_head + int64_t(s->cfg.max_scan_points) > s->map.qcap;
+}
+
+// LRU ring compaction of one session, ordered on the context's stream
+// without a wait: a full ring holds one current entry per live voxel, so the
+// host knows the compacted length.
+static int compact_ring(vmp_ctx* ex, vmp_session* s) {
   MapDev& m = s->map;
-  const MapCounters& c = s->h_ctr;
   hipStream_t st = ex->stream;
-  const int64_t hcap = int64_t(m.hmask) + 1;
   const int T = 256;
-  if (int64_t(c.used_entries) + 2 * int64_t(s->cfg.max_scan_points) > hcap / 2) {
-    VMP_HIP(hipMemsetAsync(s->nlive, 0, sizeof(int32_t), st));
-    hipLaunchKernelGGL(k_rehash_collect, dim3(grid_for(m.pool, T)), dim3(T), 0, st, m, s->live, s->nlive);
-    hipLaunchKernelGGL(k_rehash_clear, dim3(grid_for(std::min<int64_t>(hcap, 1 << 20), T)), dim3(T), 0, st, m);
-    MapCounters cc = c;
-    cc.used_entries = 0;
-    cc.tombs = 0;
-    VMP_HIP(hipMemcpyAsync(m.ctr, &cc, sizeof(cc), hipMemcpyHostToDevice, st));
-    hipLaunchKernelGGL(k_rehash_insert, dim3(grid_for(m.pool, T)), dim3(T), 0, st, m, s->live, s->nlive);
-    VMP_HIP(hipMemcpyAsync(&s->h_ctr, m.ctr, sizeof(MapCounters), hipMemcpyDeviceToHost, st));
-    VMP_HIP(hipStreamSynchronize(st));
-    *did |= 1;
-  }
   const int64_t used = s->h_ctr.ring_tail - s->h_ctr.ring_head;
-  if (used + int64_t(s->cfg.max_scan_points) > m.qcap) {
-    RingTmp& t = ex->rt;
-    if (t.cap < used && t.fixed) {
-      s->err = "LRU ring compaction: the ring exceeds the no-allocation scratch";
-      return VMP_ECAPACITY;
-    }
-    if (t.cap < used) {
-      VMP_HIP(hipStreamSynchronize(st));
+  RingTmp& t = ex->rt;
+  if (t.cap < used && t.fixed) {
+    s->err = "LRU ring compaction: the ring exceeds the no-allocation scratch";
+    return VMP_ECAPACITY;
+  }
+  if (t.cap < used) {
+    VMP_HIP(hipStreamSynchronize(st));
+    t.release();
+    const size_t n = size_t(used);
+    bool ok = dalloc(t.allocs, &t.tv, n) == hipSuccess && dalloc(t.allocs, &t.ts, n) == hipSuccess &&
+              dalloc(t.allocs, &t.keep, n) == hipSuccess && dalloc(t.allocs, &t.sel, n) == hipSuccess &&
+              dalloc(t.allocs, &t.cnt, 1) == hipSuccess;
+    t.temp_bytes = 0;
+    if (ok)
+      ok = rocprim::select(nullptr, t.temp_bytes, rocprim::counting_iterator<int32_t>(0), t.keep, t.sel, t.cnt, n,
+                           st) == hipSuccess;
+    if (ok) ok = dalloc(t.allocs, reinterpret_cast<uint8_t**>(&t.temp), t.temp_bytes + 256) == hipSuccess;
+    if (!ok) {
       t.release();
-      const size_t n = size_t(used);
-      bool ok = dalloc(t.allocs, &t.tv, n) == hipSuccess && dalloc(t.allocs, &t.ts, n) == hipSuccess &&
-                dalloc(t.allocs, &t.keep, n) == hipSuccess && dalloc(t.allocs, &t.sel, n) == hipSuccess &&
-                dalloc(t.allocs, &t.cnt, 1) == hipSuccess;
-      t.temp_bytes = 0;
-      if (ok)
-        ok = rocprim::select(nullptr, t.temp_bytes, rocprim::counting_iterator<int32_t>(0), t.keep, t.sel, t.cnt, n,
-                             st) == hipSuccess;
-      if (ok) ok = dalloc(t.allocs, reinterpret_cast<uint8_t**>(&t.temp), t.temp_bytes + 256) == hipSuccess;
-      if (!ok) {
-        t.release();
-        s->err = "LRU ring compaction: device allocation failed";
-        return VMP_ENOMEM;
-      }
-      t.temp_bytes += 256;
-      t.cap = used;
+      s->err = "LRU ring compaction: device allocation failed";
+      return VMP_ENOMEM;
     }
-    hipLaunchKernelGGL(k_ring_mark, dim3(grid_for(used, T)), dim3(T), 0, st, m, s->h_ctr.ring_head, used, t.tv, t.ts,
-                       t.keep);
-    size_t tb = t.temp_bytes;
-    VMP_HIP(rocprim::select(t.temp, tb, rocprim::counting_iterator<int32_t>(0), t.keep, t.sel, t.cnt, size_t(used), st));
-    hipLaunchKernelGGL(k_ring_scatter, dim3(grid_for(used, T)), dim3(T), 0, st, m, t.tv, t.ts, t.sel, t.cnt);
-    int32_t kept = 0;
-    VMP_HIP(hipMemcpyAsync(&kept, t.cnt, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    VMP_HIP(hipStreamSynchronize(st));
-    MapCounters cc = s->h_ctr;
-    cc.ring_head = 0;
-    cc.ring_tail = int64_t(kept);
-    VMP_HIP(hipMemcpyAsync(m.ctr, &cc, sizeof(cc), hipMemcpyHostToDevice, st));
-    VMP_HIP(hipStreamSynchronize(st));
-    s->h_ctr = cc;
-    *did |= 2;
-    if (t.fixed) {
-      // these arrays share the device scratch with the workspace of
-      // vmp_register_scan_noalloc, whose primitives' control words must
-      // start from zero at its next step
-      VMP_HIP(hipMemsetAsync(ex->ws.b.prim, 0, prim_ws_entries(ex->ws.cap_points) * sizeof(int32_t), st));
-    }
+    t.temp_bytes += 256;
+    t.cap = used;
+  }
+  hipLaunchKernelGGL(k_ring_mark, dim3(grid_for(used, T)), dim3(T), 0, st, m, s->h_ctr.ring_head, used, t.tv, t.ts,
+                     t.keep);
+  size_t tb = t.temp_bytes;
+  VMP_HIP(rocprim::select(t.temp, tb, rocprim::counting_iterator<int32_t>(0), t.keep, t.sel, t.cnt, size_t(used), st));
+  hipLaunchKernelGGL(k_ring_scatter, dim3(grid_for(used, T)), dim3(T), 0, st, m, t.tv, t.ts, t.sel, t.cnt);
+  s->h_ctr.ring_head = 0;
+  s->h_ctr.ring_tail = s->h_ctr.size;
+  if (t.fixed) {
+    // these arrays share the device scratch with the workspace of
+    // vmp_register_scan_noalloc, whose primitives' control words must
+    // start from zero at its next step
+    VMP_HIP(hipMemsetAsync(ex->ws.b.prim, 0, prim_ws_entries(ex->ws.cap_points) * sizeof(int32_t), st));
   }
   return VMP_OK;
+}
+
+// Housekeeping of a finished step's sessions (ok[i]: session i's step
+// succeeded; did[i]: 1 hash table rebuilt, 2 ring compacted): the hash
+// rebuilds of all of them in two launches, then the ring compactions, all
+// ordered on the context's stream.  Only a step on borrowed memory (the
+// device scratch that other contexts share) or on another context's
+// sessions, whose next step may run on another stream, waits for them.
+static int maintain(vmp_ctx* ex, vmp_session** ss, int n, const uint8_t* ok, int32_t* did) {
+  hipStream_t st = ex->stream;
+  int rc = VMP_OK;
+  bool wait = false;
+  MaintList l;
+  int rows = 0;
+  int64_t most_h = 0, most_p = 0;
+  hipGetLastError();  // only this function's launches are reported below
+  auto rebuild = [&]() {
+    if (rows == 0) return;
+    const int T = kMapThreads;
+    const int gh = std::min(grid_for(most_h, T), 1024), gp = std::min(grid_for(most_p, T), 1024);
+    hipLaunchKernelGGL(k_rehash_clear, dim3(gh, rows), dim3(T), 0, st, ex->ws.d_maps, l);
+    hipLaunchKernelGGL(k_rehash_insert, dim3(gp, rows), dim3(T), 0, st, ex->ws.d_maps, l);
+    rows = 0;
+    most_h = most_p = 0;
+  };
+  for (int i = 0; i < n; ++i) {
+    did[i] = 0;
+    if (!ok[i] || !wants_rehash(ss[i])) continue;
+    l.s[rows++] = uint16_t(i);
+    most_h = std::max(most_h, int64_t(ss[i]->map.hmask) + 1);
+    most_p = std::max(most_p, int64_t(ss[i]->map.pool));
+    ss[i]->h_ctr.used_entries = int32_t(ss[i]->h_ctr.size);
+    did[i] |= 1;
+    wait |= ex->ws.fixed || ss[i]->ctx != ex;
+    if (rows == kMaintRows) rebuild();
+  }
+  rebuild();
+  for (int i = 0; i < n; ++i) {
+    if (!ok[i] || !wants_ring_compaction(ss[i])) continue;
+    const int r = compact_ring(ex, ss[i]);
+    if (r != VMP_OK) {
+      if (rc == VMP_OK) rc = r;
+      continue;
+    }
+    did[i] |= 2;
+    wait |= ex->ws.fixed || ss[i]->ctx != ex;
+  }
+  vmp_session* s = ss[0];
+  VMP_HIP(hipGetLastError());
+  if (wait) VMP_HIP(hipStreamSynchronize(st));
+  return rc;
 }
 
 static void collect_kernel_timing(vmp_ctx* c) {
@@ -2190,10 +2226,23 @@ static int step_finish(vmp_ctx* c, vmp_obs_stats* ost, vmp_map_stats* mst) {
     }
   }
   int first_err = VMP_OK;
+  uint8_t ok_small[16];
+  int32_t did_small[16];
+  std::vector<uint8_t> ok_big;
+  std::vector<int32_t> did_big;
+  uint8_t* ok = ok_small;  // sessions whose map update succeeded
+  int32_t* did = did_small;
+  if (n > 16) {
+    ok_big.resize(size_t(n));
+    did_big.resize(size_t(n));
+    ok = ok_big.data();
+    did = did_big.data();
+  }
   for (int i = 0; i < n; ++i) {
     vmp_session* si = ss[i];
     const BatchOut& o = c->ws.h_out[i];
     si->h_ctr = o.ctr;
+    ok[i] = 0;
     if ((mode & kStepIeskf) && o.obs[7]) {
       si->err = "hash probe overflow";
       if (first_err == VMP_OK) first_err = VMP_EDEVICE;
@@ -2233,11 +2282,15 @@ static int step_finish(vmp_ctx* c, vmp_obs_stats* ost, vmp_map_stats* mst) {
         mst[i].dropped = m.dropped;
         mst[i].map_size = int32_t(m.size);
       }
-      int32_t did = 0;
-      rc = maintain(c, si, &did);
-      if (mst) mst[i].maintenance = did;
-      if (rc != VMP_OK && first_err == VMP_OK) first_err = rc;
+      ok[i] = 1;
     }
+  }
+  if (mode & kStepMap) {
+    rc = maintain(c, ss, n, ok, did);
+    if (rc != VMP_OK && first_err == VMP_OK) first_err = rc;
+    if (mst)
+      for (int i = 0; i < n; ++i)
+        if (ok[i]) mst[i].maintenance = did[i];
   }
   return first_err;
 }
@@ -2673,6 +2726,7 @@ extern "C" int64_t vmp_map_export(vmp_session* s, int64_t cap, int64_t* keys, in
   std::lock_guard<std::mutex> lk(s->ctx->mu);
   if (hipSetDevice(s->ctx->device) != hipSuccess) return -1;
   const MapDev& m = s->map;
+  if (hipStreamSynchronize(s->ctx->stream) != hipSuccess) return -1;  // a step's housekeeping may still run
   std::vector<VoxState> vs(static_cast<size_t>(m.pool));
   std::vector<double> pl(static_cast<size_t>(m.pool) * kPlaneD);
   if (hipMemcpy(vs.data(), m.vs, sizeof(VoxState) * vs.size(), hipMemcpyDeviceToHost) != hipSuccess) return -1;

@@ -88,38 +88,36 @@ __device__ inline int32_t nbr_at(const MapDev& m, uint64_t vkey, int j, int tag,
 }
 
 // The six face neighbours' voxel ids (-1: none), as lookup_vid gives them;
-// the six home-slot entries are loaded together, and only a collision
-// continues its probe.
+// the six home-slot entries are loaded together, then the next probes of the
+// neighbours that collided, together again.
 __device__ inline void lookup_nbrs6(const MapDev& m, uint64_t vkey, int32_t nv[6]) {
   uint64_t nk[6];
-  uint32_t h[6];
+  HashSeq q[6];
   HashEntry e[6];
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
     nk[j] = key_neighbour_ok(vkey, j) ? key_neighbour(vkey, j) : kKeyEmpty;
-    h[j] = hash_slot(nk[j], m.hmask);
-    e[j] = m.table[h[j]];
+    q[j] = hash_seq(nk[j]);
+    e[j] = m.table[hash_home(q[j], m.hmask)];
+    nv[j] = -1;
   }
+  uint32_t open = 0;  // neighbours whose sequence goes on
 #pragma unroll
   for (int j = 0; j < 6; ++j) {
-    int32_t v = -1;
-    if (nk[j] != kKeyEmpty) {
-      if (e[j].key == nk[j]) {
-        v = e[j].vid;
-      } else if (e[j].key != kKeyEmpty) {
-        uint32_t hh = h[j];
-        for (uint32_t probe = 1; probe <= m.hmask; ++probe) {
-          hh = (hh + 1) & m.hmask;
-          const HashEntry ee = m.table[hh];
-          if (ee.key == nk[j]) {
-            v = ee.vid;
-            break;
-          }
-          if (ee.key == kKeyEmpty) break;
-        }
-      }
+    if (nk[j] == kKeyEmpty) continue;
+    if (e[j].key == nk[j]) nv[j] = e[j].vid;
+    else if (e[j].key != kKeyEmpty) open |= 1u << j;
+  }
+  for (uint32_t probe = 1; open != 0 && probe <= m.hmask; ++probe) {
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+      if (open & (1u << j)) e[j] = m.table[hash_probe(q[j], probe, m.hmask)];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      if (!(open & (1u << j))) continue;
+      if (e[j].key == nk[j]) nv[j] = e[j].vid;
+      if (e[j].key == nk[j] || e[j].key == kKeyEmpty) open &= ~(1u << j);
     }
-    nv[j] = v;
   }
 }
 

@@ -133,17 +133,15 @@ __device__ inline int find_job(kconst<ObsJob>* jobs, int njobs, int blk) {
   return lo;
 }
 
-// Linear probe from slot h, whose entry e was already read; each further
-// entry's key and id are read in one load.
-__device__ inline int32_t hash_resolve(const HashEntry* table, uint32_t mask, uint64_t key, uint32_t h, vmp_u3 e,
-                                       int32_t* err) {
-  for (uint32_t probe = 0;; ++probe) {
+// The probe sequence from the home slot, whose entry e was already read; each
+// further entry's key and id are read in one load.
+__device__ inline int32_t hash_resolve(const HashEntry* table, uint32_t mask, uint64_t key, vmp_u3 e, int32_t* err) {
+  for (uint32_t probe = 0;;) {
     const uint64_t k = uint64_t(e.x) | (uint64_t(e.y) << 32);
     if (k == key) return int32_t(e.z);
     if (k == kKeyEmpty) return -1;
     if (probe == mask) break;
-    h = (h + 1) & mask;
-    e = *as_global(reinterpret_cast<const vmp_u3*>(table + h));
+    e = *as_global(reinterpret_cast<const vmp_u3*>(table + hash_probe(hash_seq(key), ++probe, mask)));
   }
   if (err) atomicOr(err, 1);
   return -1;
@@ -206,7 +204,6 @@ __global__ void __launch_bounds__(kObsThreads) observe_kernel(const ObsJob* __re
     float uh[kObsGroup][3], ul[kObsGroup][3], kl[kObsGroup][3], pw[kObsGroup][3];
     int64_t key[kObsGroup][3];
     uint64_t pk[kObsGroup];
-    uint32_t hs[kObsGroup];
     vmp_u3 he[kObsGroup];
 #pragma unroll
     for (int g = 0; g < kObsGroup; ++g) {
@@ -281,15 +278,15 @@ __global__ void __launch_bounds__(kObsThreads) observe_kernel(const ObsJob* __re
       // (read unconditionally: slot 0 stands in for points without a key, so
       // the loads stay in flight together; every load's whole destination
       // is used, so no register is reused while it is pending)
-      hs[g] = in_range ? hash_slot(pk[g], J.hmask) : 0u;
-      he[g] = *as_global(reinterpret_cast<const vmp_u3*>(J.table + hs[g]));
+      const uint32_t hs = in_range ? hash_home(hash_seq(pk[g]), J.hmask) : 0u;
+      he[g] = *as_global(reinterpret_cast<const vmp_u3*>(J.table + hs));
     }
     int32_t vid[kObsGroup];
     vmp_f4 h0[kObsGroup];
     vmp_f3 h1[kObsGroup];
 #pragma unroll
     for (int g = 0; g < kObsGroup; ++g)
-      vid[g] = pk[g] == kKeyEmpty ? -1 : hash_resolve(J.table, J.hmask, pk[g], hs[g], he[g], J.counters + 4);
+      vid[g] = pk[g] == kKeyEmpty ? -1 : hash_resolve(J.table, J.hmask, pk[g], he[g], J.counters + 4);
 #pragma unroll
     for (int g = 0; g < kObsGroup; ++g) {
       // both halves of the 32 B plane record are loaded together (record 0
