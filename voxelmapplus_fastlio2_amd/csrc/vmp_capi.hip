@@ -553,8 +553,7 @@ static bool ws_layout(vmp_ctx* c, BatchWs& w, size_t n, int ns, size_t pre_cap, 
        dev(&b.cand_start, size_t(ns)) && dev(&b.spl, n);
   ok = ok && dev(&b.seg_ct, n * 7) && dev(&b.seg_nct, n) && dev(&b.seg_nbr, n * 6);
   ok = ok && dev(&b.len_in, n) && dev(&b.len_out, n) && dev(&b.ord_in, n) && dev(&b.ord, n);
-  ok = ok && dev(&b.lv, n * 2) && dev(&b.lv2, n * 2) && dev(&b.lv_cnt, (n * 2 >> 6) + size_t(ns) + 2) &&
-       dev(&b.lv_n, size_t(ns));
+  ok = ok && dev(&b.lv, n * 2) && dev(&b.lv2, n * 2) && dev(&b.lv_cnt, (n * 2 >> 6) + size_t(ns) + 2);
   ok = ok && dev(&b.prim, prim_ws_entries(int64_t(n))) && dev(&b.qc, n * 3);
   // the refitting-voxel list of the replay lives in cand_nbr's memory (24 B
   // per point), which k_spec_eval writes only after the replays
@@ -1765,9 +1764,8 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode) {
           timed_launch(c, kTkRingLive, [&] {
             hipLaunchKernelGGL(k_ring_live, dim3(kLvBlocks, n), dim3(64 * kLvWaves), 0, st, M, S, n, b);
           });
-          hipLaunchKernelGGL(k_ring_pack, dim3(n), dim3(kLpThreads), 0, st, M, S, n, b);
           timed_launch(c, kTkCreateEvict,
-                       [&] { hipLaunchKernelGGL(k_create_evict, dim3(n), dim3(128), 0, st, M, S, n, b); });
+                       [&] { hipLaunchKernelGGL(k_create_evict, dim3(n), dim3(kCeThreads), 0, st, M, S, n, b); });
         }
         hipLaunchKernelGGL(k_create_init, dim3(gn), dim3(T), 0, st, M, S, n, b);
         // replay order by segment length in 6 bits (one radix pass; segments
