@@ -1,9 +1,9 @@
 """LRU evictions of one scan against the oracle: the keys in LRU order after
-every scan, where the evictions are decided all at once (a few, or most of
-the touched old voxels evicted and created again in the scan; the first
-overflow, with room left for some of the creations) and where they are
-decided one at a time (more touched entries, or more points, than the
-all-at-once tables hold)."""
+every scan, with few or most of the touched old voxels evicted and created
+again in the scan, at the first overflow (room left for some of the
+creations), with more touched entries than threads, with a ring whose head
+is mostly stale (more of it read than is prefetched), and with more points
+than the tables in LDS hold."""
 import numpy as np
 import pytest
 
@@ -20,6 +20,7 @@ CASES = {
     "one_over": (3700, 2000, (20.0, 20.0, 2.0), 0.0, 4),
     "many_touched": (45000, 30000, (25.0, 25.0, 2.0), 0.0, 4),
     "many_points": (6600, 263000, (7.0, 7.0, 2.0), 2.0, 3),
+    "stale_ring": (900, 600, (2.0, 2.0, 2.0), 0.0, 40),
 }
 
 
@@ -28,6 +29,8 @@ def scans(name):
     rng = np.random.default_rng(len(name) * 1000 + n)
     for q in range(k):
         pts = rng.uniform(-1.0, 1.0, (n - q, 3)) * half
+        if name == "stale_ring" and q >= k - 2:  # after a long stand: new ground, more voxels than the map has room for
+            pts *= 8.0
         yield state_vector(np.eye(3), [move * q, 0.0, 0.0]), np.ascontiguousarray(pts.T.astype(np.float32))
 
 

@@ -31,7 +31,6 @@
 namespace vmp {
 
 constexpr int kMapThreads = 256;
-constexpr int kHeapCap = 4096;
 constexpr int32_t kNever = 0x7fffffff;
 
 struct MapCounters {
@@ -230,29 +229,13 @@ __device__ inline int wave_fetch_add(int* p, int v) {
   return out;
 }
 
+__device__ inline uint64_t bits_below(int l) { return l == 0 ? 0ull : (~0ull >> (64 - l)); }
+
 // LDS written by some lanes of a wave and read by others of the same wave
 __device__ inline void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Least value over the 64 lanes of a wave (every lane active): row shifts
-// within each 16-lane row, then the row broadcasts, leave it in lane 63.
-__device__ inline uint32_t wave_min_u32(uint32_t v) {
-  constexpr int kId = -1;  // 0xffffffff, the identity of min
-  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(kId, int(v), 0x111, 0xf, 0xf, false)));  // row_shr:1
-  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(kId, int(v), 0x112, 0xf, 0xf, false)));  // row_shr:2
-  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(kId, int(v), 0x114, 0xf, 0xf, false)));  // row_shr:4
-  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(kId, int(v), 0x118, 0xf, 0xf, false)));  // row_shr:8
-  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(kId, int(v), 0x142, 0xa, 0xf, false)));  // row_bcast:15
-  v = min(v, uint32_t(__builtin_amdgcn_update_dpp(kId, int(v), 0x143, 0xc, 0xf, false)));  // row_bcast:31
-  return uint32_t(__builtin_amdgcn_readlane(int(v), 63));
-}
-__device__ inline uint64_t wave_min_u64(uint64_t v) {
-  const uint32_t hi = wave_min_u32(uint32_t(v >> 32));
-  const uint32_t lo = wave_min_u32(uint32_t(v >> 32) == hi ? uint32_t(v) : 0xffffffffu);
-  return (uint64_t(hi) << 32) | lo;
 }
 
 // *inserted = 1 when this call claimed the empty slot (the caller counts
@@ -627,8 +610,8 @@ __global__ void k_create_fast(const MapDev* maps, const SessInfo* si, int nsess,
 }
 
 // Chunks of the ring that k_ring_live compacts for a session: enough for the
-// creations of the scan at a few stale entries per victim, within the
-// session's two entries per point; the ordered pass reads the ring directly
+// creations of most scans at a few stale entries per victim, within the
+// session's two entries per point; k_create_evict reads the ring itself
 // beyond them.
 __device__ inline int64_t lv_chunks(const MapCounters* c, const SessInfo& S) {
   const int64_t used = c->ring_tail - c->ring_head;
@@ -636,13 +619,30 @@ __device__ inline int64_t lv_chunks(const MapCounters* c, const SessInfo& S) {
   return min(min((used + 63) >> 6, (want + 63) >> 6), (int64_t(2) * S.n) >> 6);
 }
 
+// The ring entry `rel` places after the head as (vid, first touch in this
+// scan or kNever, segment, rel); vid -1 if it is past the tail or stale.  An
+// entry is live while its voxel is alive, still carries the entry's stamp
+// and has not been evicted in this scan; no decision of k_create_evict makes
+// another entry live.
+__device__ inline int4 ring_entry(const MapDev& m, int64_t head, int64_t tail, int tag, int64_t rel) {
+  int4 e = make_int4(-1, kNever, -1, int32_t(rel));
+  if (head + rel >= tail) return e;
+  const int64_t ph = (head + rel) % m.qcap;
+  const int32_t v = m.ring_vid[ph];
+  const uint64_t stp = m.ring_stamp[ph];
+  const VoxState& st = m.vs[v];
+  const bool cur = st.tag == tag;
+  if ((st.flags & kAlive) && st.stamp == stp && !(cur && st.evict_t != kNever)) e.x = v;
+  if (cur && st.create_t < 0) e.y = st.first_t;
+  e.z = st.seg;
+  return e;
+}
+
 constexpr int kLvWaves = 4;   // waves per block of k_ring_live
 constexpr int kLvBlocks = 32; // blocks per session
 
-// Liveness of the ring entries ahead of the head (grid: kLvBlocks x
-// sessions), one wave per 64-entry chunk, compacted within the chunk.  An entry is live while its voxel
-// is alive, still carries the entry's stamp and has not been evicted in this
-// scan; nothing the ordered pass changes makes another entry live.
+// The live ring entries ahead of the head (grid: kLvBlocks x sessions), one
+// wave per 64-entry chunk, compacted within the chunk.
 __global__ void __launch_bounds__(64 * kLvWaves) k_ring_live(const MapDev* maps, const SessInfo* si, int nsess,
                                                               BatchBufs b) {
   const int s = blockIdx.y;
@@ -655,69 +655,24 @@ __global__ void __launch_bounds__(64 * kLvWaves) k_ring_live(const MapDev* maps,
   const int64_t head = c->ring_head, tail = c->ring_tail;
   const int tag = c->tag;
   const int lane = threadIdx.x & 63;
-  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
   int4* out0 = b.lv + int64_t(2) * S.off;
   for (int64_t k = int64_t(blockIdx.x) * kLvWaves + (threadIdx.x >> 6); k < nch;
        k += int64_t(gridDim.x) * kLvWaves) {
-    const int64_t idx = head + k * 64 + lane;
-    int32_t v = -1, first = kNever, seg = -1;
-    bool live = false;
-    if (idx < tail) {
-      const int64_t ph = idx % m.qcap;
-      v = m.ring_vid[ph];
-      const uint64_t stp = m.ring_stamp[ph];
-      const VoxState& st = m.vs[v];
-      const bool cur = st.tag == tag;
-      live = (st.flags & kAlive) && st.stamp == stp && !(cur && st.evict_t != kNever);
-      first = (cur && st.create_t < 0) ? st.first_t : kNever;
-      seg = st.seg;
-    }
-    const uint64_t bal = __ballot(live);
-    if (live) out0[k * 64 + __popcll(bal & below)] = make_int4(v, first, seg, int32_t(k * 64 + lane));
+    const int4 e = ring_entry(m, head, tail, tag, k * 64 + lane);
+    const uint64_t bal = __ballot(e.x >= 0);
+    if (e.x >= 0) out0[k * 64 + __popcll(bal & bits_below(lane))] = e;
     if (lane == 0) b.lv_cnt[lv_cnt_base(S.off, s) + k] = __popcll(bal);
   }
 }
 
-constexpr int kCeThreads = 1024;  // k_create_evict block
-constexpr int kCeWaves = kCeThreads / 64;
-
-// The chunks' live entries packed in ring order (a block of kCeThreads):
-// counts scanned per group of 1024 chunks, then one wave copies a chunk.
-// Returns the number of entries.
-__device__ inline int ring_pack(const BatchBufs& b, const SessInfo& S, int s, int64_t nch, int32_t* sh) {
-  const int4* src = b.lv + int64_t(2) * S.off;
-  int4* dst = b.lv2 + int64_t(2) * S.off;
-  const int32_t* cnt = b.lv_cnt + lv_cnt_base(S.off, s);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int32_t base = 0;
-  for (int64_t g0 = 0; g0 < nch; g0 += kCeThreads) {
-    const int32_t cj = g0 + tid < nch ? cnt[g0 + tid] : 0;
-    sh[tid] = cj;
-    __syncthreads();
-    for (int d = 1; d < kCeThreads; d <<= 1) {  // inclusive scan
-      const int32_t v = tid >= d ? sh[tid - d] : 0;
-      __syncthreads();
-      sh[tid] += v;
-      __syncthreads();
-    }
-    for (int q = wave; q < kCeThreads && g0 + q < nch; q += kCeWaves) {
-      const int32_t hi = sh[q], lo = q > 0 ? sh[q - 1] : 0;
-      if (lane < hi - lo) dst[base + lo + lane] = src[(g0 + q) * 64 + lane];
-    }
-    base += sh[kCeThreads - 1];
-    __syncthreads();
-  }
-  return base;
-}
-
-// Ordered creation + eviction, one workgroup per session that may overflow.
-// LRU order is the descending order of last-touch stamps; the ring holds
-// (vid, stamp) in ascending stamp order with stale entries skipped lazily.
-// The victim of each creation is the oldest live voxel not yet touched by an
-// earlier point of this scan; a victim touched later comes back as a new
-// voxel at its first touch (another creation event).
+// Creations and evictions in order, one workgroup per session that may
+// overflow.  LRU order is the descending order of last-touch stamps; the
+// ring holds (vid, stamp) in ascending stamp order with stale entries skipped
+// lazily.  The victim of each creation is the oldest live voxel not yet
+// touched by an earlier point of this scan; a victim touched later comes back
+// as a new voxel at its first touch (another creation event).
 //
-// All decisions at once (evict_parallel).  Let the events (creations and
+// All decisions are taken at once.  Let the events (creations and
 // re-creations) in time order be T_0 < T_1 < ..., Z the creations that still
 // fit under the capacity, f_i the first touch of the live ring entry i in
 // this scan (kNever: none) and r_i the number of victims before i.  The ring
@@ -726,32 +681,33 @@ __device__ inline int ring_pack(const BatchBufs& b, const SessInfo& S, int s, in
 // untouched entry always is, while events are left.  Only the touched
 // entries need deciding, and whether one is a victim changes r of the
 // entries after it and the events after its first touch only.  So: one bit
-// per ring entry (victim) and per point time (event), all touched entries
+// per live entry (victim) and per point time (event), all touched entries
 // evaluated against prefix counts of both, the changed bits flipped, until a
-// round changes none.  Such a state is the sequential result: by induction
-// over i, r_i is right, and a victim behind i returns after the event that
-// reaches i.  2 to 6 rounds settle thousands of events (at most 6 in 2,400
-// random instances, a few dozen to 4,400 of the touched entries victims).
-// For 6,300 evictions of a 60k-point scan 26 us, bound by the chain of round
-// trips and barriers; one at a time (about 1 us for each step of up to 64)
-// with the packing of the ring entries 181 us.
+// round changes none.
 //
-// One at a time (the rest of the kernel), for sessions beyond evict_parallel's
-// tables and the rare one whose prefetched ring chunks run out: wave 0
-// decides.  It holds 64-entry windows of the live ring entries and of
-// the creation events, and 128 entries of the free list, in its lanes, and
-// takes them from LDS stream buffers that wave 1 fills from global memory
-// ahead of it, so the deciding wave waits on no global load while its own
-// stores drain.  While the next creations precede every pending
-// re-creation, up to 64 of them take their victims in one step.
-constexpr int kStreamSlots = 8;  // chunks of each stream buffered in LDS
-constexpr int kProdBurst = 4;    // chunks of each stream the producer loads per round trip
-// Waits for every vector memory operation of the wave.  The decider's rare
-// paths (direct ring reads, creations below capacity) end with it: their
-// global loads are then complete on every path into the decision loop, so
-// the loop's common path (LDS only) carries no wait on the scattered stores
-// of earlier steps (stores and loads share one counter on this target).
-__device__ __forceinline__ void drain_vm() { __builtin_amdgcn_s_waitcnt(0); }
+// Such a state is the sequential result: by induction over i, r_i is right,
+// and a victim behind i returns after the event that reaches i.  And the
+// rounds end: once the entries before i are settled, one behind i that is
+// wrongly held a victim with a first touch before T_(Z + r_i) is dropped by
+// the next round if no other such entry has an earlier first touch, and
+// without such entries i itself is right.  2 to 6 rounds settle thousands of
+// events (at most 6 in 2,400 random instances, with a few dozen to 4,400 of
+// the touched entries among the victims).
+//
+// For 6,300 evictions of a 60k-point scan 30 us, bound by the chain of round
+// trips and barriers; one decision after the other (about 1 us for each step
+// of up to 64 of them) took 181 us.
+constexpr int kCeThreads = 1024;  // k_create_evict block
+constexpr int kCeWaves = kCeThreads / 64;
+constexpr int kEvWords = 4096;    // words of each bit table that fit in LDS (262,144 bits)
+constexpr int kEvUnroll = 8;      // ring chunks a wave loads per round trip
+constexpr uint64_t kCandWrong = uint64_t(1) << 31;  // above the 26 bits of a live entry's index
+struct EvTables {
+  uint64_t* ev;  // bit t: an event at point time t
+  uint64_t* vw;  // bit i: live entry i is a victim
+  int32_t* evp;  // bits set before each word
+  int32_t* vp;
+};
 
 // marks an evicted voxel in its record (one lane); cur: the record already
 // carries this scan's fields
@@ -766,166 +722,124 @@ __device__ inline void evict_write(const MapDev& m, int tag, int32_t victim, boo
   }
 }
 
-constexpr int kEvWords = 4096;  // 64-bit words of point times, and of ring entries (262,144 each)
-constexpr int kEvCand = 4096;   // touched ring entries to decide
-constexpr int kEvRounds = 64;   // then the one-at-a-time decisions take over
-constexpr int kEvUnroll = 8;    // ring chunks a wave loads per round trip
-struct EvLds {
-  uint64_t ev[kEvWords];   // bit t: an event at point time t
-  uint64_t vw[kEvWords];   // bit l of word k: live entry l of ring chunk k is a victim
-  int32_t evp[kEvWords];   // bits set before each word
-  int32_t vp[kEvWords];
-  int32_t cf[kEvCand];     // touched entries: first touch, and chunk * 64 + entry
-  int32_t cp[kEvCand];
-};
-struct SeqLds {
-  uint64_t heap[kHeapCap];     // (first touch << 32) | evicted vid
-  int32_t heap_seg[kHeapCap];  // the key's segment in this scan
-  int4 live[kStreamSlots][64];
-  int32_t cre[kStreamSlots][128];
-  int32_t free[kStreamSlots][64];
-  int32_t seq[3];  // chunks produced per stream
-  int32_t use[3];  // first chunk per stream the decider still reads
-  int32_t done;
-};
-__device__ inline uint64_t bits_below(int l) { return l == 0 ? 0ull : (~0ull >> (64 - l)); }
-
-// exclusive prefix counts of the set bits of w[0 .. n), n <= kEvWords, into
-// p; returns the total (a block of kCeThreads, four words each)
-static_assert(4 * kCeThreads >= kEvWords, "four words per thread");
-__device__ inline int bits_scan(const uint64_t* w, int n, int32_t* p, int32_t* wsum) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int v[4], sum = 0;
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    v[u] = 4 * tid + u < n ? __popcll(w[4 * tid + u]) : 0;
-    sum += v[u];
-  }
-  int incl = sum;
-  for (int o = 1; o < 64; o <<= 1) {
-    const int x = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += x;
-  }
-  if (lane == 63) wsum[wave] = incl;
-  __syncthreads();
-  int run = incl - sum, total = 0;
-#pragma unroll
-  for (int q = 0; q < kCeWaves; ++q) {
-    const int x = wsum[q];
-    run += q < wave ? x : 0;
-    total += x;
-  }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    if (4 * tid + u < n) p[4 * tid + u] = run;
-    run += v[u];
-  }
-  __syncthreads();
-  return total;
+// a bit table's word: in LDS, or in global memory, where the flips are
+// device-scope atomics that plain loads could miss
+template <bool kLds>
+__device__ inline uint64_t ev_word(const uint64_t* p) {
+  return kLds ? *p : __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// false: nothing was changed, and the decisions are taken one at a time
-__device__ inline bool evict_parallel(const MapDev& m, const SessInfo& S, int s, const BatchBufs& b, EvLds& L) {
+// exclusive prefix counts of the set bits of w[0 .. n) into p; returns the
+// total (a block of kCeThreads, four words each per pass)
+template <bool kLds>
+__device__ inline int bits_scan(const uint64_t* w, int n, int32_t* p, int32_t* wsum) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  int carry = 0;
+  for (int i0 = 0; i0 < n; i0 += 4 * kCeThreads) {
+    const int i = i0 + 4 * tid;
+    int v[4], sum = 0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      v[u] = i + u < n ? __popcll(ev_word<kLds>(w + i + u)) : 0;
+      sum += v[u];
+    }
+    int incl = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int x = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += x;
+    }
+    if (lane == 63) wsum[wave] = incl;
+    __syncthreads();
+    int run = carry + incl - sum;
+#pragma unroll
+    for (int q = 0; q < kCeWaves; ++q) {
+      const int x = wsum[q];
+      run += q < wave ? x : 0;
+      carry += x;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (i + u < n) p[i + u] = run;
+      run += v[u];
+    }
+    __syncthreads();
+  }
+  return carry;
+}
+
+// The decisions over nlive packed live entries (b.lv2, at 2 * off): the
+// events into b.co, the victims into b.ev_vid and their records, the
+// session's counters.  With too few victims in the whole ring the scan
+// touches more new voxels than the LRU can evict: error 4, nothing changed.
+template <bool kLds>
+__device__ inline void evict_decide(const MapDev& m, const SessInfo& S, const BatchBufs& b, int nlive, int Z,
+                                    const EvTables& T, int32_t* wsum, int* ncand) {
   MapCounters* c = m.ctr;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int clo = S.cre_lo, ncre_ev = S.cre_hi - clo, off = S.off;
-  const int nw = (S.n + 63) >> 6;
-  const int64_t nch64 = lv_chunks(c, S);
-  if (nw > kEvWords || nch64 > kEvWords) return false;
-  const int nch = int(nch64);
-  const int64_t size = c->size, cap = m.capacity;
-  const int Z = int(max(int64_t(0), cap - size));  // below ncre_ev: the session is not a fast one
-  const int4* lv = b.lv + int64_t(2) * off;
-  const int32_t* lcnt = b.lv_cnt + lv_cnt_base(off, s);
-  __shared__ int32_t wsum[kCeWaves], wu[kCeWaves], wt[kCeWaves];
-  __shared__ int ncand, last_rel;
-  for (int i = tid; i < nw; i += kCeThreads) L.ev[i] = 0;
-  if (tid == 0) ncand = 0;
+  const int nw = (S.n + 63) >> 6, nk = (nlive + 63) >> 6;
+  const int4* lv = b.lv2 + int64_t(2) * off;
+  uint64_t* cand = b.cand_in + off;  // touched entries: (first touch << 32) | entry
+  auto flip = [](uint64_t* p, int bit) {
+    atomicXor(reinterpret_cast<unsigned long long*>(p), 1ull << bit);
+  };
+  for (int i = tid; i < nw; i += kCeThreads) T.ev[i] = 0;
+  if (tid == 0) *ncand = 0;
   __syncthreads();
   for (int r = tid; r < ncre_ev; r += kCeThreads) {
     const int t = b.cre_t[clo + r];
-    atomicOr(reinterpret_cast<unsigned long long*>(&L.ev[t >> 6]), 1ull << (t & 63));
+    flip(T.ev + (t >> 6), t & 63);
   }
-  // ---- the ring's chunks, up to where the untouched entries alone could
-  //      serve every creation and every return of a touched one before them
-  int k0 = 0, nu = 0, nt = 0;
-  while (k0 < nch) {
-    const int kw = k0 + wave * kEvUnroll;
-    int cn[kEvUnroll], f[kEvUnroll];
-#pragma unroll
-    for (int u = 0; u < kEvUnroll; ++u) {  // every load of the round first
-      const int k = min(kw + u, nch - 1);
-      cn[u] = lcnt[k];
-      f[u] = lv[k * 64 + lane].y;
+  for (int k = wave; k < nk; k += kCeWaves) {
+    const int i = 64 * k + lane;
+    const int f = i < nlive ? lv[i].y : kNever;
+    const uint64_t bt = __ballot(f != kNever), bu = __ballot(i < nlive && f == kNever);
+    if (lane == 0) T.vw[k] = bu;
+    if (bt) {
+      int base = 0;
+      if (lane == 0) base = atomicAdd(ncand, __popcll(bt));
+      base = __builtin_amdgcn_readfirstlane(base);
+      if (f != kNever) cand[base + __popcll(bt & bits_below(lane))] = (uint64_t(uint32_t(f)) << 32) | uint32_t(i);
     }
-    int su = 0, stt = 0;
-#pragma unroll
-    for (int u = 0; u < kEvUnroll; ++u) {
-      if (kw + u >= nch) break;
-      const bool in = lane < cn[u];
-      const uint64_t bt = __ballot(in && f[u] != kNever), bu = __ballot(in && f[u] == kNever);
-      if (lane == 0) L.vw[kw + u] = bu;
-      su += __popcll(bu);
-      if (bt) {
-        const int n = __popcll(bt);
-        stt += n;
-        int base = 0;
-        if (lane == 0) base = atomicAdd(&ncand, n);
-        base = __builtin_amdgcn_readfirstlane(base);
-        const int at = base + __popcll(bt & bits_below(lane));
-        if (((bt >> lane) & 1ull) && at < kEvCand) {
-          L.cf[at] = f[u];
-          L.cp[at] = (kw + u) * 64 + lane;
-        }
+  }
+  __syncthreads();
+  const int nt = *ncand;
+  auto victim_bit = [&](int i) { return (ev_word<kLds>(T.vw + (i >> 6)) >> (i & 63)) & 1ull; };
+  auto rank = [&](int i) { return T.vp[i >> 6] + __popcll(ev_word<kLds>(T.vw + (i >> 6)) & bits_below(i & 63)); };
+  auto events_before = [&](int t) {
+    return T.evp[t >> 6] + __popcll(ev_word<kLds>(T.ev + (t >> 6)) & bits_below(t & 63));
+  };
+  int nev, nvict;
+  while (true) {
+    nev = bits_scan<kLds>(T.ev, nw, T.evp, wsum);
+    nvict = bits_scan<kLds>(T.vw, nk, T.vp, wsum);
+    // every evaluation of a round precedes its flips: a wrong bit is noted in
+    // the entry's bit 31 (its own thread flips it after the barrier)
+    int wrong = 0;
+    for (int q = tid; q < nt; q += kCeThreads) {
+      const uint64_t cq = cand[q];
+      const int f = int(cq >> 32), i = int(uint32_t(cq));
+      if (int(events_before(f) >= Z + rank(i) + 1) != int(victim_bit(i))) {
+        cand[q] = cq | kCandWrong;
+        wrong = 1;
       }
     }
-    if (lane == 0) {
-      wu[wave] = su;
-      wt[wave] = stt;
-    }
-    __syncthreads();
-    for (int q = 0; q < kCeWaves; ++q) {
-      nu += wu[q];
-      nt += wt[q];
-    }
-    k0 += kCeWaves * kEvUnroll;
-    __syncthreads();
-    if (nu >= ncre_ev - Z + nt) break;
-  }
-  const int nk = min(k0, nch);
-  if (nt > kEvCand) return false;
-  __syncthreads();
-  // ---- rounds
-  int nev = 0, nvict = 0;
-  bool settled = false;
-  for (int it = 0; it < kEvRounds && !settled; ++it) {
-    nev = bits_scan(L.ev, nw, L.evp, wsum);
-    nvict = bits_scan(L.vw, nk, L.vp, wsum);
-    uint32_t flip = 0;
-#pragma unroll
-    for (int u = 0; u < kEvCand / kCeThreads; ++u) {
-      const int q = tid + u * kCeThreads;
-      if (q >= nt) break;
-      const int f = L.cf[q], p = L.cp[q];
-      const uint64_t w = L.vw[p >> 6];
-      const int r = L.vp[p >> 6] + __popcll(w & bits_below(p & 63));
-      const int before = L.evp[f >> 6] + __popcll(L.ev[f >> 6] & bits_below(f & 63));
-      const bool victim = before >= Z + r + 1;
-      if (victim != (((w >> (p & 63)) & 1ull) != 0)) flip |= 1u << u;
-    }
-    settled = !__syncthreads_or(int(flip));
-#pragma unroll
-    for (int u = 0; u < kEvCand / kCeThreads; ++u) {
-      if (!(flip & (1u << u))) continue;
-      const int q = tid + u * kCeThreads;
-      const int f = L.cf[q], p = L.cp[q];
-      atomicXor(reinterpret_cast<unsigned long long*>(&L.vw[p >> 6]), 1ull << (p & 63));
-      atomicXor(reinterpret_cast<unsigned long long*>(&L.ev[f >> 6]), 1ull << (f & 63));
+    if (!__syncthreads_or(wrong)) break;
+    for (int q = tid; wrong && q < nt; q += kCeThreads) {
+      uint64_t cq = cand[q];
+      if (!(cq & kCandWrong)) continue;
+      cand[q] = cq &= ~kCandWrong;
+      const int f = int(cq >> 32), i = int(uint32_t(cq));
+      flip(T.vw + (i >> 6), i & 63);
+      flip(T.ev + (f >> 6), f & 63);
     }
     __syncthreads();
   }
   const int need = nev - Z;  // one victim per event from the Z-th on
-  if (!settled || nvict < need || nev > S.n) return false;
+  if (nvict < need || nev > S.n) {
+    if (tid == 0) atomicOr(&c->error, 4);
+    return;
+  }
   // ---- the events in order: the j-th takes the j-th free slot
   const int ftop = c->free_top, bump = c->bump;
   int err = 0;
@@ -934,45 +848,44 @@ __device__ inline bool evict_parallel(const MapDev& m, const SessInfo& S, int s,
     if (vid >= m.pool) err = 8;
     return vid;
   };
-  auto event_at = [&](int t) { return L.evp[t >> 6] + __popcll(L.ev[t >> 6] & bits_below(t & 63)); };
   for (int r = tid; r < ncre_ev; r += kCeThreads) {
     const int t = b.cre_t[clo + r], seg = b.cre_seg[clo + r];
-    const int j = event_at(t);
+    const int j = events_before(t);
     b.co[off + j] = make_int4(slot_of(j), seg, t, -1);
   }
   for (int q = tid; q < nt; q += kCeThreads) {
-    const int p = L.cp[q];
-    if (!((L.vw[p >> 6] >> (p & 63)) & 1ull)) continue;
-    const int4 e = lv[p];
-    const int j = event_at(e.y);
+    const int i = int(uint32_t(cand[q]));
+    if (!victim_bit(i)) continue;
+    const int4 e = lv[i];
+    const int j = events_before(e.y);
     b.co[off + j] = make_int4(slot_of(j), e.z, e.y, e.x);
   }
   if (err) atomicOr(&c->error, err);
   __syncthreads();
   // ---- the victims in order: the r-th goes at the event Z + r
   const int tag = c->tag;
-  for (int kk = wave; kk < nk; kk += kCeWaves) {
-    const uint64_t w = L.vw[kk];
-    if (L.vp[kk] >= need) break;
-    const int r = L.vp[kk] + __popcll(w & bits_below(lane));
-    if (!((w >> lane) & 1ull) || r >= need) continue;
-    const int4 e = lv[kk * 64 + lane];
+  int last = -1;
+  for (int k = wave; k < nk; k += kCeWaves) {
+    if (T.vp[k] >= need) break;
+    const int i = 64 * k + lane;
+    const int r = rank(i);
+    if (!victim_bit(i) || r >= need) continue;
+    const int4 e = lv[i];
     const int t = b.co[off + Z + r].z;
     evict_write(m, tag, e.x, e.y != kNever, t);
     b.ev_vid[off + r] = e.x;
-    if (r == need - 1) last_rel = e.w;
+    if (r == need - 1) last = e.w;
   }
-  __syncthreads();
-  if (tid == 0) {
-    c->size = size + Z;
+  __syncthreads();  // every read of the counters precedes their update
+  if (last >= 0) {  // the thread of the last victim
+    c->size += Z;
     c->group_counter += uint64_t(nev);
     c->free_top = max(0, ftop - nev);
     c->bump = bump + max(0, nev - ftop);
-    c->ring_head += last_rel + 1;
+    c->ring_head += last + 1;
     c->ncre = nev;
     c->nevict = need;
   }
-  return true;
 }
 
 __global__ void __launch_bounds__(kCeThreads) k_create_evict(const MapDev* maps, const SessInfo* si, int nsess,
@@ -980,429 +893,80 @@ __global__ void __launch_bounds__(kCeThreads) k_create_evict(const MapDev* maps,
   const int s = blockIdx.x;
   if (s >= nsess) return;
   const MapDev m = maps[s];
-  MapCounters* c = m.ctr;
+  const MapCounters* c = m.ctr;
   if (c->fast) return;
-  __shared__ __align__(16) unsigned char lds[sizeof(EvLds) > sizeof(SeqLds) ? sizeof(EvLds) : sizeof(SeqLds)];
+  __shared__ uint64_t s_ev[kEvWords], s_vw[kEvWords];
+  __shared__ int32_t s_evp[kEvWords], s_vp[kEvWords];
+  __shared__ int32_t wsum[kCeWaves], wt[kCeWaves];
+  __shared__ int ncand;
   const SessInfo S = si[s];
-  if (evict_parallel(m, S, s, b, *reinterpret_cast<EvLds*>(lds))) return;
-  const int clo = S.cre_lo, ncre_ev = S.cre_hi - clo;
-  const int off = S.off;
-  const int64_t npre = lv_chunks(c, S);
-  __syncthreads();
-  const int nlive = ring_pack(b, S, s, npre, reinterpret_cast<int32_t*>(lds));
-  const int ftop0 = c->free_top;
-  // streams: 0 packed live ring entries, 1 creation events (time, segment),
-  // 2 the free list from its top down; 64 entries per chunk
-  const int nwin = (nlive + 63) >> 6, ncch = (ncre_ev + 63) >> 6, nfch = (ftop0 + 63) >> 6;
-  SeqLds& L = *reinterpret_cast<SeqLds*>(lds);
-  uint64_t* heap = L.heap;
-  int32_t* heap_seg = L.heap_seg;
-  auto& s_live = L.live;
-  auto& s_cre = L.cre;
-  auto& s_free = L.free;
-  auto& s_seq = L.seq;
-  auto& s_use = L.use;
-  int32_t& s_done = L.done;
-  const int lane = threadIdx.x & 63;
-  if (threadIdx.x < 3) {
-    s_seq[threadIdx.x] = 0;
-    s_use[threadIdx.x] = 0;
-  }
-  if (threadIdx.x == 0) s_done = 0;
-  __syncthreads();
-  if (threadIdx.x >= 128) return;
-
-  if (threadIdx.x >= 64) {
-    // ---- stream producer: keeps each stream up to kStreamSlots chunks
-    //      ahead of the decider (skipping chunks it no longer needs), up to
-    //      kProdBurst chunks of each stream per round trip, and stops when
-    //      the decider is done or every chunk is out
-    const int4* lvs = b.lv2 + int64_t(2) * off;
-    const __attribute__((address_space(1))) int32_t* fl = as_global(m.freelist);
-    int p0 = 0, p1 = 0, p2 = 0;
-    while (__hip_atomic_load(&s_done, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == 0) {
-      const int u0 = __hip_atomic_load(&s_use[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      const int u1 = __hip_atomic_load(&s_use[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      const int u2 = __hip_atomic_load(&s_use[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      p0 = max(p0, u0);
-      p1 = max(p1, u1);
-      p2 = max(p2, u2);
-      const int n0 = max(0, min(kProdBurst, min(nwin, u0 + kStreamSlots) - p0));
-      const int n1 = max(0, min(kProdBurst, min(ncch, u1 + kStreamSlots) - p1));
-      const int n2 = max(0, min(kProdBurst, min(nfch, u2 + kStreamSlots) - p2));
-      int4 e[kProdBurst];
-      int32_t ct[kProdBurst], cs[kProdBurst], fv[kProdBurst];
-#pragma unroll
-      for (int k = 0; k < kProdBurst; ++k) {  // every load of the round first
-        const int i0 = 64 * (p0 + k) + lane, i1 = 64 * (p1 + k) + lane, i2 = 64 * (p2 + k) + lane;
-        e[k] = make_int4(-1, kNever, -1, 0);
-        ct[k] = kNever;
-        cs[k] = -1;
-        fv[k] = -1;
-        if (k < n0 && i0 < nlive) e[k] = lvs[i0];
-        if (k < n1 && i1 < ncre_ev) {
-          ct[k] = b.cre_t[clo + i1];
-          cs[k] = b.cre_seg[clo + i1];
-        }
-        if (k < n2 && i2 < ftop0) fv[k] = fl[ftop0 - 1 - i2];
-      }
-#pragma unroll
-      for (int k = 0; k < kProdBurst; ++k) {
-        if (k < n0) s_live[(p0 + k) % kStreamSlots][lane] = e[k];
-        if (k < n1) {
-          s_cre[(p1 + k) % kStreamSlots][lane] = ct[k];
-          s_cre[(p1 + k) % kStreamSlots][64 + lane] = cs[k];
-        }
-        if (k < n2) s_free[(p2 + k) % kStreamSlots][lane] = fv[k];
-      }
-      p0 += n0;
-      p1 += n1;
-      p2 += n2;
-      if (lane == 0) {
-        __hip_atomic_store(&s_seq[0], p0, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-        __hip_atomic_store(&s_seq[1], p1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-        __hip_atomic_store(&s_seq[2], p2, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-      if (p0 >= nwin && p1 >= ncch && p2 >= nfch) break;
-      if (n0 + n1 + n2 == 0) __builtin_amdgcn_s_sleep(2);
-    }
-    return;
-  }
-
-  // ---- the decider (wave 0)
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int off = S.off, ncre_ev = S.cre_hi - S.cre_lo;
+  const int Z = int(max(int64_t(0), int64_t(m.capacity) - c->size));  // below ncre_ev: the session is not a fast one
+  // ---- the live entries from the head on, packed in ring order, up to
+  //      where the untouched ones alone could serve every creation and every
+  //      return of a touched one before them (creations and touched old
+  //      voxels have distinct first points, so that is at most 2 n entries)
+  const int64_t nch = lv_chunks(c, S);
+  const int64_t head = c->ring_head, tail = c->ring_tail, used = tail - head;
   const int tag = c->tag;
-  const int64_t cap = m.capacity;
-  int hn = 0;
-  int64_t size = c->size;
-  uint64_t gc = c->group_counter;
-  int ftop = ftop0, bump = c->bump;
-  int64_t ptr = c->ring_head;
-  const int64_t tail = c->ring_tail;
-  const int64_t head0 = ptr;
-  // ring window: per lane an entry's vid, liveness, first touch in this scan
-  // (kNever if untouched), segment, ring position - head0, and whether the
-  // voxel state carries this tag; wend is the ring position after the
-  // window.  The live entries of the first npre ring chunks come packed, 64
-  // per window; the ring is read directly after them.
-  int64_t wend = head0;
-  int lw = 0;  // next packed window
-  int32_t l_vid = -1, l_first = kNever, l_seg = -1, l_rel = 0;
-  bool l_live = false, l_cur = false;
-  // creation chunk cq in lanes; free-list chunks fq, fq + 1 (allocation
-  // indices 64 fq ... 64 fq + 127, allocation a taking freelist[ftop0 - 1 - a])
-  int cq = -1, fq = -1;
-  int32_t c_t = kNever, c_seg = -1, f_lo = -1, f_hi = -1;
-  int ci = 0, nco = 0, nev = 0;
-  int err = 0;
-  const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-
-  auto await = [&](int st, int need) {  // until chunk need - 1 of stream st is out
-    while (__hip_atomic_load(&s_seq[st], __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < need)
-      __builtin_amdgcn_s_sleep(1);
-  };
-  auto release = [&](int st, int first) {
-    if (lane == 0) __hip_atomic_store(&s_use[st], first, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  };
-  auto load_ring = [&]() {  // the next window, from ptr on
-    if (lw < nwin) {
-      release(0, lw);
-      await(0, lw + 1);
-      const int4 e = s_live[lw % kStreamSlots][lane];
-      l_vid = e.x;
-      l_first = e.y;
-      l_seg = e.z;
-      l_rel = e.w;
-      l_live = e.x >= 0;
-      l_cur = e.y != kNever;  // a live voxel carries this tag iff touched in this scan
-      wend = head0 + __builtin_amdgcn_readlane(e.w, min(63, nlive - 64 * lw - 1)) + 1;
-      ++lw;
-      return;
-    }
-    const int64_t rbase = max(ptr, head0 + 64 * npre);
-    ptr = rbase;
-    wend = min<int64_t>(rbase + 64, tail);
-    const int64_t idx = rbase + lane;
-    l_vid = -1;
-    l_live = false;
-    l_cur = false;
-    l_first = kNever;
-    l_seg = -1;
-    l_rel = int32_t(idx - head0);
-    if (idx < tail) {
-      const int64_t ph = idx % m.qcap;
-      const int32_t v = *as_global(m.ring_vid + ph);
-      const uint64_t stp = *as_global(m.ring_stamp + ph);
-      const auto* st = as_global(m.vs + v);
-      l_vid = v;
-      l_cur = st->tag == tag;
-      l_live = (st->flags & kAlive) && st->stamp == stp && !(l_cur && st->evict_t != kNever);
-      l_first = (l_cur && st->create_t < 0) ? st->first_t : kNever;
-      l_seg = st->seg;
-    }
-    drain_vm();
-  };
-  auto load_cre = [&]() {  // the chunk of creation ci
-    cq = ci >> 6;
-    release(1, cq);
-    await(1, cq + 1);
-    c_t = s_cre[cq % kStreamSlots][lane];
-    c_seg = s_cre[cq % kStreamSlots][64 + lane];
-  };
-  // make the lanes hold the next k free-list entries (k <= 64, k <= ftop)
-  auto load_free = [&](int k) {
-    const int a = ftop0 - ftop;
-    if (fq >= 0 && a >= 64 * fq && a + k <= 64 * fq + 128) return;
-    fq = a >> 6;
-    release(2, fq);
-    await(2, min(fq + 2, nfch));
-    f_lo = s_free[fq % kStreamSlots][lane];
-    f_hi = fq + 1 < nfch ? s_free[(fq + 1) % kStreamSlots][lane] : -1;
-  };
-  auto free_at = [&](int a) {  // entry of allocation a (inside the window), per lane
-    const int q = a - 64 * fq;
-    const int32_t x = __shfl(f_lo, q & 63, 64), y = __shfl(f_hi, q & 63, 64);
-    return q < 64 ? x : y;
-  };
-  auto free_at_u = [&](int a) {  // the same for an allocation uniform over the wave
-    const int q = a - 64 * fq;
-    return q < 64 ? __builtin_amdgcn_readlane(f_lo, q) : __builtin_amdgcn_readlane(f_hi, q - 64);
-  };
-  // pending re-creations, (first touch << 32) | evicted vid, in slots
-  // [0, hn) of heap (segment in heap_seg); slot i belongs to lane i & 63,
-  // which keeps the least key of its slots (lmin, at lpos), so the earliest
-  // one is a wave minimum away
-  int th = kNever;  // time of the earliest pending re-creation
-  uint64_t lmin = ~0ull;
-  int lpos = -1;
-  auto lane_rescan = [&](bool me) {
-    if (me) {
-      lmin = ~0ull;
-      lpos = -1;
-      for (int i = lane; i < hn; i += 64) {
-        const uint64_t k = heap[i];
-        if (k < lmin) {
-          lmin = k;
-          lpos = i;
-        }
+  const int4* lvc = b.lv + int64_t(2) * off;
+  const int32_t* lcnt = b.lv_cnt + lv_cnt_base(off, s);
+  int4* packed = b.lv2 + int64_t(2) * off;
+  const int lim = 2 * S.n;
+  int nl = 0, nt = 0;
+  for (int64_t k0 = 0; 64 * k0 < used; k0 += kCeWaves * kEvUnroll) {
+    const int64_t kw = k0 + wave * kEvUnroll;
+    int4 e[kEvUnroll];
+    if (kw + kEvUnroll <= nch) {  // compacted ahead: every load of the round first
+      int cn[kEvUnroll];
+#pragma unroll
+      for (int u = 0; u < kEvUnroll; ++u) {
+        cn[u] = lcnt[kw + u];
+        e[u] = lvc[(kw + u) * 64 + lane];
       }
-    }
-  };
-  // a re-creation at first touch f of the evicted voxel v (segment sg)
-  auto heap_push = [&](int32_t f, int32_t v, int32_t sg) {
-    const uint64_t key = (uint64_t(uint32_t(f)) << 32) | uint32_t(v);
-    if (lane == (hn & 63)) {
-      heap[hn] = key;
-      heap_seg[hn] = sg;
-      if (key < lmin) {
-        lmin = key;
-        lpos = hn;
-      }
-    }
-    ++hn;
-    th = min(th, f);
-  };
-
-  while (true) {
-    if (ci < ncre_ev && (ci >> 6) != cq) load_cre();
-    const int d = ci & 63;  // creation ci sits in lane d of its chunk
-    const int t_s = ci < ncre_ev ? __builtin_amdgcn_readlane(c_t, d) : kNever;
-    const int t_h = th;
-    if (t_s == kNever && t_h == kNever) break;
-    if (t_s < t_h) {
-      // ---- bulk: creations that need no victim (below capacity, where no
-      //      re-created key can be pending)
-      if (size < cap && hn == 0) {
-        const int mm = int(min<int64_t>(cap - size, int64_t(ncre_ev - ci)));
-        for (int j0 = 0; j0 < mm; j0 += 64) {
-          const int j = j0 + lane;
-          if (j < mm) {
-            const int fj = ftop - 1 - j;  // the same allocation order as one by one
-            const int32_t vid = fj >= 0 ? *as_global(m.freelist + fj) : bump + (j - ftop);
-            if (vid >= m.pool) err |= 8;
-            b.co[off + nco + j] = make_int4(vid, b.cre_seg[clo + ci + j], b.cre_t[clo + ci + j], -1);
-          }
-        }
-        drain_vm();
-        if (__ballot(err != 0)) {
-          err |= 8;
-          break;
-        }
-        if (mm <= ftop) ftop -= mm;
-        else {
-          bump += mm - ftop;
-          ftop = 0;
-        }
-        ci += mm;
-        nco += mm;
-        gc += uint64_t(mm);
-        size += mm;
-        continue;
-      }
-      // ---- bulk: creations before the next re-creation take their victims
-      //      from the live ring entries ahead.  An entry first touched before
-      //      t_s is passed over by all of them (creation times only grow);
-      //      an untouched one is the victim of whichever creation reaches
-      //      it; the first entry touched after t_s ("hard") ends the step,
-      //      as the victim of the next creation if that comes before the
-      //      entry's first touch (its key then returns at that touch).
-      if (size >= cap && ptr < tail) {
-        if (ptr >= wend) load_ring();
-        const bool ahead = l_live && head0 + l_rel >= ptr;
-        const uint64_t hard = __ballot(ahead && l_first != kNever && l_first > t_s);
-        const int tpos = hard ? __ffsll((unsigned long long)hard) - 1 : 64;
-        const uint64_t usable = __ballot(ahead && l_first == kNever) & (tpos >= 64 ? ~0ull : ((1ull << tpos) - 1));
-        const int ncr = __popcll(__ballot(lane >= d && c_t < t_h));  // creations of this chunk before t_h
-        const int nu = __popcll(usable);
-        int mm = min(nu, ncr);
-        int32_t hf = kNever, hv = -1, hs = -1;
-        if (mm == nu && nu < ncr && tpos < 64) {
-          hf = __builtin_amdgcn_readlane(l_first, tpos);
-          if (__builtin_amdgcn_readlane(c_t, d + nu) < hf) {
-            hv = __builtin_amdgcn_readlane(l_vid, tpos);
-            hs = __builtin_amdgcn_readlane(l_seg, tpos);
-            ++mm;
-          }
-        }
-        const uint64_t vmask = usable | (hv >= 0 ? (1ull << tpos) : 0ull);
-        if (mm > 0) {
-          // the r-th entry of vmask is the victim of creation ci + r
-          const bool mine = ((vmask >> lane) & 1ull) != 0;
-          const int r = __popcll(vmask & below);
-          const bool act = mine && r < mm;
-          const int src = d + (act ? r : 0);
-          const int t = __shfl(c_t, src, 64);
-          const int sg = __shfl(c_seg, src, 64);
-          const int nf = min(mm, ftop);  // victims' slots from the free list, then the bump
-          if (nf > 0) load_free(nf);
-          const int a0 = ftop0 - ftop;  // allocation index of creation ci
-          const int32_t fv = nf > 0 ? free_at(a0 + min(act ? r : 0, nf - 1)) : -1;
-          if (act) {
-            const int32_t vid = r < ftop ? fv : bump + (r - ftop);
-            if (vid >= m.pool) err |= 8;
-            b.co[off + nco + r] = make_int4(vid, sg, t, -1);
-            evict_write(m, tag, l_vid, l_cur, t);
-            b.ev_vid[off + nev + r] = l_vid;
-            l_live = false;
-          }
-          if (__ballot(err != 0)) {
-            err |= 8;
-            break;
-          }
-          // the ring position after the mm-th victim (the lane of vmask's mm-th bit)
-          const uint64_t lastb = __ballot(mine && r == mm - 1);
-          ptr = head0 + __builtin_amdgcn_readlane(l_rel, __ffsll((unsigned long long)lastb) - 1) + 1;
-          if (hv >= 0) {
-            if (hn >= kHeapCap) {
-              err |= 16;
-              break;
-            }
-            heap_push(hf, hv, hs);
-          }
-          if (mm <= ftop) ftop -= mm;
-          else {
-            bump += mm - ftop;
-            ftop = 0;
-          }
-          ci += mm;
-          nco += mm;
-          nev += mm;
-          gc += uint64_t(mm);
-          continue;
-        }
-        // no victim left in the window: the rest was touched before t_s
-        ptr = wend;
-        continue;
-      }
-    }
-    // ---- single step: the earliest event, then its victim if over capacity
-    int t, seg, prev;
-    if (t_s < t_h) {
-      t = t_s;
-      seg = __builtin_amdgcn_readlane(c_seg, d);
-      prev = -1;
-      ++ci;
-    } else {  // the earliest pending re-creation leaves its slot to the last one
-      const uint64_t top = wave_min_u64(lmin);
-      const int w = __ffsll((unsigned long long)__ballot(lmin == top)) - 1;  // keys are unique (vid)
-      const int gp = __builtin_amdgcn_readlane(lpos, w);
-      t = int(top >> 32);
-      prev = int32_t(top & 0xffffffffu);  // evicted incarnation of this key
-      seg = heap_seg[gp];
-      const int last = hn - 1, lo = last & 63;
-      wave_lds_sync();
-      if (lane == lo && last != gp) {
-        heap[gp] = heap[last];
-        heap_seg[gp] = heap_seg[last];
-      }
-      wave_lds_sync();
-      --hn;
-      lane_rescan(lane == w || lane == lo);
-      th = hn > 0 ? int(wave_min_u64(lmin) >> 32) : kNever;
-    }
-    int32_t vid;
-    if (ftop > 0) {
-      load_free(1);
-      vid = free_at_u(ftop0 - ftop);
-      --ftop;
+#pragma unroll
+      for (int u = 0; u < kEvUnroll; ++u)
+        if (lane >= cn[u]) e[u] = make_int4(-1, kNever, -1, 0);
     } else {
-      vid = bump++;
+#pragma unroll
+      for (int u = 0; u < kEvUnroll; ++u) e[u] = ring_entry(m, head, tail, tag, (kw + u) * 64 + lane);
     }
-    if (vid >= m.pool) {
-      err |= 8;
-      break;
+    int su = 0, stt = 0;
+#pragma unroll
+    for (int u = 0; u < kEvUnroll; ++u) {
+      su += __popcll(__ballot(e[u].x >= 0));
+      stt += __popcll(__ballot(e[u].x >= 0 && e[u].y != kNever));
     }
-    if (lane == 0) b.co[off + nco] = make_int4(vid, seg, t, prev);
-    ++gc;
-    ++nco;
-    ++size;
-    if (size > cap) {
-      int32_t victim = -1, vfirst = kNever, vseg = -1;
-      bool vcur = false;
-      while (true) {
-        if (ptr >= tail) {
-          err |= 4;
-          break;
-        }
-        if (ptr >= wend) load_ring();
-        const uint64_t bal = __ballot(l_live && head0 + l_rel >= ptr && l_first > t);
-        if (bal) {
-          const int w = __ffsll((unsigned long long)bal) - 1;
-          victim = __builtin_amdgcn_readlane(l_vid, w);
-          vfirst = __builtin_amdgcn_readlane(l_first, w);
-          vseg = __builtin_amdgcn_readlane(l_seg, w);
-          vcur = __builtin_amdgcn_readlane(int(l_cur), w) != 0;
-          ptr = head0 + __builtin_amdgcn_readlane(l_rel, w) + 1;
-          if (lane == w) l_live = false;
-          break;
-        }
-        ptr = wend;
-      }
-      if (victim < 0) break;
-      if (lane == 0) {
-        evict_write(m, tag, victim, vcur, t);
-        b.ev_vid[off + nev] = victim;
-      }
-      ++nev;
-      --size;
-      if (vfirst != kNever) {  // the key comes back later in this scan
-        if (hn >= kHeapCap) {
-          err |= 16;
-          break;
-        }
-        heap_push(vfirst, victim, vseg);
-      }
+    if (lane == 0) {
+      wsum[wave] = su;
+      wt[wave] = stt;
     }
+    __syncthreads();
+    int at = nl;
+    for (int q = 0; q < kCeWaves; ++q) {
+      at += q < wave ? wsum[q] : 0;
+      nl += wsum[q];
+      nt += wt[q];
+    }
+#pragma unroll
+    for (int u = 0; u < kEvUnroll; ++u) {
+      const uint64_t bal = __ballot(e[u].x >= 0);
+      const int i = at + __popcll(bal & bits_below(lane));
+      if (e[u].x >= 0 && i < lim) packed[i] = e[u];
+      at += __popcll(bal);
+    }
+    __syncthreads();
+    if (nl - nt >= ncre_ev - Z + nt) break;
   }
-  if (lane == 0) {
-    c->size = size;
-    c->group_counter = gc;
-    c->free_top = ftop;
-    c->bump = bump;
-    c->ring_head = ptr;
-    c->ncre = nco;
-    c->nevict = nev;
-    if (err) atomicOr(&c->error, err);
-    __hip_atomic_store(&s_done, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  const int nlive = min(nl, lim);
+  const int nw = (S.n + 63) >> 6, nk = (nlive + 63) >> 6;
+  if (nw <= kEvWords && nk <= kEvWords) {
+    evict_decide<true>(m, S, b, nlive, Z, EvTables{s_ev, s_vw, s_evp, s_vp}, wsum, &ncand);
+  } else {  // the tables of a larger scan in the candidate stage's scratch, free until then
+    uint64_t* ev = reinterpret_cast<uint64_t*>(b.cand_nbr + size_t(off) * 6);
+    int32_t* evp = reinterpret_cast<int32_t*>(ev + nw + nk);
+    evict_decide<false>(m, S, b, nlive, Z, EvTables{ev, ev + nw, evp, evp + nw}, wsum, &ncand);
   }
 }
 
