@@ -309,7 +309,7 @@ int vmp_autotune_observe(vmp_session* s, int32_t reps, int32_t* best_ppt, float*
  * session falls in); either may be NULL. */
 int vmp_autotune_observe_batch(vmp_session** s, int32_t n, int32_t reps, int32_t* table, float* cand_ms);
 
-/* Device events around the last call's kernels (for roofline timing). */
+/* Stage times of the last completed step, from the device's clock (-1: none yet). */
 int vmp_session_timing(vmp_session* s, double* observe_ms, double* map_ms, int32_t* observe_launches);
 /* Per-launch HIP-event timing of the observe kernel and of the map-update
  * pipeline, accumulated until the next vmp_session_set_timing call.

@@ -14,9 +14,19 @@ __device__ inline void load_state(const vmp_state& src, vmp_state& dst, int lane
   for (int i = lane; i < 36; i += 64) d[i] = s[i];
 }
 
-__global__ void k_obs_prep(FilterDev** fs) {
+// before an observe pass of its own: the pass's parameters and cleared counters
+__global__ void k_obs_prep(FilterDev** fs, int32_t** obs_ctr) {
   FilterDev* f = fs[blockIdx.x];
+  if (threadIdx.x < 8) obs_ctr[blockIdx.x][threadIdx.x] = 0;
   if (threadIdx.x == 0) make_obs_params(f->x, f->P, f->cfg, f->obs_prm);
+}
+// the same at a given state, which becomes the session's
+__global__ void k_obs_prep_at(FilterDev* f, vmp_state x, int32_t* obs_ctr) {
+  if (threadIdx.x < 8) obs_ctr[threadIdx.x] = 0;
+  if (threadIdx.x == 0) {
+    f->x = x;
+    make_obs_params(x, f->P, f->cfg, f->obs_prm);
+  }
 }
 __global__ void k_upd_prep(FilterDev** fs) {
   FilterDev* f = fs[blockIdx.x];
@@ -66,8 +76,10 @@ __global__ void k_zero_lists(int32_t** lists, int n) {
 // factor runs in the first wave's lanes; the inverse's product W^T W is
 // spread over all the workgroup's waves.
 constexpr int kBeginEndThreads = 256;
-__global__ void __launch_bounds__(kBeginEndThreads) k_ieskf_begin(FilterDev** fs, int32_t** obs_ctr) {
+__global__ void __launch_bounds__(kBeginEndThreads) k_ieskf_begin(FilterDev** fs, int32_t** obs_ctr,
+                                                                  uint64_t* clk) {
   FilterDev* f = fs[blockIdx.x];
+  if (blockIdx.x == 0 && threadIdx.x == 0) clk[0] = wall_clock64();
   if (threadIdx.x < 8) obs_ctr[blockIdx.x][threadIdx.x] = 0;  // counters of the first observe pass
   __shared__ vmp_state sx;
   const int lane = threadIdx.x;

@@ -47,7 +47,6 @@ struct ImuDev {
   double q[4];     // diagonal of Q by block: ng, na, nbg, nba
   int32_t npose;   // entries of the pose table
   int32_t pad;
-  ImuPkg pkg;      // the package being processed
   double pose[kMaxImu + 1][kPoseD];
   double pose_min[kMaxImu + 1];  // min of the offsets from entry i to the second to last
 };
@@ -62,6 +61,7 @@ struct ImuCfgDev {
 // one session of the preprocessing stage
 struct PreJob {
   ImuDev* imu;
+  const ImuPkg* pkg;
   FilterDev* f;
   const float* x;  // raw points, ascending time
   const float* y;
@@ -422,6 +422,7 @@ k_imu_predict(const PreJob* jobs, int nsess) {
   if (int(blockIdx.x) >= nsess) return;
   const PreJob Jb = jobs[blockIdx.x];
   ImuDev* im = Jb.imu;
+  const ImuPkg* pkg = Jb.pkg;
   FilterDev* f = Jb.f;
   const int lane = threadIdx.x;  // phases A-C and the set-up run on the first wave's lanes
   __shared__ PredShared S;
@@ -429,13 +430,13 @@ k_imu_predict(const PreJob* jobs, int nsess) {
   load_state(f->x, S.sx, lane);
   if (lane < 4) S.q[lane] = im->q[lane];
   __syncthreads();
-  const int m = im->pkg.m;
+  const int m = pkg->m;
   const double lce = im->last_cloud_end;
-  const double cstart = im->pkg.cloud_start;
+  const double cstart = pkg->cloud_start;
   // active IMU pairs (head k-1 or last_imu, tail k) are those whose tail is
   // not before the last scan end: a prefix of the ascending samples is skipped
   int k0 = 0;
-  while (k0 < m && im->pkg.s[k0][0] < lce) ++k0;
+  while (k0 < m && pkg->s[k0][0] < lce) ++k0;
   const int nsteps = (m - k0) + 1;  // the pairs, then the step to the sweep's end
   if (lane == 0) {
     double Bx[6];
@@ -476,23 +477,23 @@ k_imu_predict(const PreJob* jobs, int nsess) {
     if (k < k0) {
       for (int c = 0; c < 3; ++c) acc[c] = gyro[c] = 0.0;
     } else {
-      const double* hs = k == 0 ? nullptr : im->pkg.s[k - 1];
+      const double* hs = k == 0 ? nullptr : pkg->s[k - 1];
       for (int c = 0; c < 3; ++c) {
         const double ha = k == 0 ? im->last_imu_acc[c] : hs[1 + c];
         const double hgy = k == 0 ? im->last_imu_gyro[c] : hs[4 + c];
-        gyro[c] = 0.5 * (hgy + im->pkg.s[k][4 + c]);
-        acc[c] = 0.5 * (ha + im->pkg.s[k][1 + c]);
+        gyro[c] = 0.5 * (hgy + pkg->s[k][4 + c]);
+        acc[c] = 0.5 * (ha + pkg->s[k][1 + c]);
         acc[c] = acc[c] * 9.81 / im->gravity_norm;
       }
     }
     if (st < nsteps - 1) {
-      const double ht = k == 0 ? im->last_imu_t : im->pkg.s[k - 1][0];
-      tt = im->pkg.s[k][0];
+      const double ht = k == 0 ? im->last_imu_t : pkg->s[k - 1][0];
+      tt = pkg->s[k][0];
       dt = ht < lce ? tt - lce : tt - ht;
     } else {
-      const double imu_end = m > 0 ? im->pkg.s[m - 1][0] : im->last_imu_t;
+      const double imu_end = m > 0 ? pkg->s[m - 1][0] : im->last_imu_t;
       tt = 0.0;
-      dt = im->pkg.cloud_end - imu_end;
+      dt = pkg->cloud_end - imu_end;
     }
   };
   int np = 1;  // pose table entries
@@ -613,13 +614,13 @@ k_imu_predict(const PreJob* jobs, int nsess) {
   if (lane == 0) {
     f->x = S.sx;
     if (m > 0) {
-      im->last_imu_t = im->pkg.s[m - 1][0];
+      im->last_imu_t = pkg->s[m - 1][0];
       for (int c = 0; c < 3; ++c) {
-        im->last_imu_acc[c] = im->pkg.s[m - 1][1 + c];
-        im->last_imu_gyro[c] = im->pkg.s[m - 1][4 + c];
+        im->last_imu_acc[c] = pkg->s[m - 1][1 + c];
+        im->last_imu_gyro[c] = pkg->s[m - 1][4 + c];
       }
     }
-    im->last_cloud_end = im->pkg.cloud_end;
+    im->last_cloud_end = pkg->cloud_end;
     im->npose = np;
     // running minimum of the offsets of the interval heads (entries 0..np-2)
     double mn = 1e300;

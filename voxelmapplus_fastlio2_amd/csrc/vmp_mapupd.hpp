@@ -349,8 +349,9 @@ __device__ inline void write_hot(const MapDev& m, int32_t vid, uint32_t flags) {
 
 #define VMP_GRID_LOOP(i, n) for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < (n); i += gridDim.x * blockDim.x)
 
-__global__ void k_begin_scan(const MapDev* maps, int nsess) {
+__global__ void k_begin_scan(const MapDev* maps, int nsess, uint64_t* clk) {
   if (threadIdx.x != 0 || int(blockIdx.x) >= nsess) return;
+  if (blockIdx.x == 0) clk[1] = wall_clock64();
   MapCounters* c = maps[blockIdx.x].ctr;
   c->tag += 1;
   c->fast = 0;
@@ -1878,18 +1879,6 @@ __global__ void k_lru_append(const MapDev* maps, const SessInfo* si, int nsess, 
     m.ring_vid[ph] = vid;
     m.ring_stamp[ph] = uint64_t(m.ctr->point_base + t);
   }
-}
-
-// the scan's counter updates: the LRU appends, the points, and the evicted
-// voxels that k_evict_finalize pushed above the free-list top (nothing
-// after k_evict_finalize reads free_top; nevict stays 0 in a scan without
-// points)
-__global__ void k_end_scan(const MapDev* maps, const SessInfo* si, int nsess) {
-  if (threadIdx.x != 0 || int(blockIdx.x) >= nsess) return;
-  MapCounters* c = maps[blockIdx.x].ctr;
-  c->ring_tail += c->nlru;
-  c->point_base += si[blockIdx.x].n;
-  c->free_top += c->nevict;
 }
 
 // start of each session's candidates in the sorted candidate list, and

@@ -426,9 +426,16 @@ __global__ void __launch_bounds__(kObsThreads) observe_kernel(const ObsJob* __re
 
 // Reduce the partial rows of every job (one workgroup per session) in a fixed
 // order: row b is added by thread b mod 256, threads are combined wave by
-// wave.  Writes H (12x12 column-major, symmetric), b and the counters.
+// wave.  Writes H (12x12 column-major, symmetric), b and the counters, for one
+// job also to the host (out: pinned memory), with the signal word `sig` set
+// to `want` behind them.
+struct ObsOut {
+  double H[144], b[12];
+  int32_t ctr[8];
+};
 template <int NJ>
-__global__ void __launch_bounds__(kObsThreads) k_obs_reduce(const ObsJob* __restrict__ jobs) {
+__global__ void __launch_bounds__(kObsThreads) k_obs_reduce(const ObsJob* __restrict__ jobs, ObsOut* out,
+                                                            int32_t* sig, int32_t want) {
   constexpr int NH = NJ * (NJ + 1) / 2;
   constexpr int NACC = NH + NJ;
   constexpr int ROW = obs_row<NJ>();
@@ -465,9 +472,22 @@ __global__ void __launch_bounds__(kObsThreads) k_obs_reduce(const ObsJob* __rest
       v = red[0][o];
     }
     J.out[tid] = v;
+    if (out) out->H[tid] = v;
   }
-  if (tid < 12) J.out[144 + tid] = tid < NJ ? red[0][NH + tid] : 0.0;
+  if (tid < 12) {
+    const double v = tid < NJ ? red[0][NH + tid] : 0.0;
+    J.out[144 + tid] = v;
+    if (out) out->b[tid] = v;
+  }
   if (tid < 4) J.counters[tid] = int32_t(red[0][NACC + tid]);
+  if (!out) return;
+  if (tid < 4) out->ctr[tid] = int32_t(red[0][NACC + tid]);
+  else if (tid < 8) out->ctr[tid] = J.counters[tid];
+  __syncthreads();
+  if (tid == 0) {
+    __threadfence_system();
+    if (sig) __hip_atomic_store(sig, want, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 }  // namespace vmp
