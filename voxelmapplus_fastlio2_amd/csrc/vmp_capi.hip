@@ -1800,12 +1800,16 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
         // the work evenly over waves, every segment replays on its own
         hipLaunchKernelGGL(k_seg_lenkeys, dim3(gn), dim3(T), 0, st, M, S, b, lbits, long_seg);
         if (!sort_pairs(b.len_in, b.ord_in, b.len_out, b.ord, lbits + 1)) return VMP_EDEVICE;
-        // the moment path: a voxel per wave up to wave_max refitting voxels
-        // (a grid of up to 4096 waves strides over them), else for the long
-        // segments only and 64 voxels per wave for the rest; the light path
-        // covers the voxels that do not refit
+        // the moment path: a voxel per wave up to wave_max refitting voxels,
+        // else for the long segments only and 64 voxels per wave for the
+        // rest; the light path covers the voxels that do not refit.  The
+        // waves stride over the voxels: up to 2,048 (what the card holds at
+        // this kernel's registers), a quarter as many as points for small
+        // scans (a wave per 64 points left 88 voxels of a 2,003-point scan
+        // to 32 waves, three refits after one another: 68 us against 24).
+        const int heavy_blocks = std::max(1, std::min((ntot + 15) / 16, 512));
         timed_launch(c, kTkReplayHeavy, [&] {
-          hipLaunchKernelGGL(k_replay_heavy_wave, dim3(std::min(gn, 1024)), dim3(T), 0, st, M, S, b, wave_max);
+          hipLaunchKernelGGL(k_replay_heavy_wave, dim3(heavy_blocks), dim3(T), 0, st, M, S, b, wave_max);
           hipLaunchKernelGGL(k_replay_heavy, dim3(std::min(gn, 256)), dim3(T), 0, st, M, S, b, wave_max);
         });
         timed_launch(c, kTkReplayLight, [&] { hipLaunchKernelGGL(k_replay_light, dim3(gn), dim3(T), 0, st, M, S, b); });
