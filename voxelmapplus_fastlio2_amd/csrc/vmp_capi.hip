@@ -951,6 +951,7 @@ extern "C" int vmp_session_create(vmp_ctx* ctx, const vmp_map_cfg* cfg, vmp_sess
   f0.x.g[2] = -kGravity;
   for (int i = 0; i < 23; ++i) f0.P[i * 23 + i] = 1.0;
   if (hipMemcpyAsync(s->f, &f0, sizeof(f0), hipMemcpyHostToDevice, st) != hipSuccess) return fail(VMP_EDEVICE);
+  hipLaunchKernelGGL(k_filter_init, dim3(1), dim3(64), 0, st, s->f);
   if (hipMemsetAsync(s->obs_ctr, 0, 8 * sizeof(int32_t), st) != hipSuccess) return fail(VMP_EDEVICE);
   if (hipMemsetAsync(s->imu, 0, sizeof(ImuDev), st) != hipSuccess) return fail(VMP_EDEVICE);
   if (hipMemsetAsync(s->obs_stat, 0, 8 * sizeof(int32_t), st) != hipSuccess) return fail(VMP_EDEVICE);

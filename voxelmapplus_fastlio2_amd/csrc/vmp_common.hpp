@@ -240,29 +240,22 @@ __host__ __device__ inline void d33_to_cm(const D33& A, double* cm) {
     for (int r = 0; r < 3; ++r) cm[c * 3 + r] = A.m[r * 3 + c];
 }
 
-// r_wl = rot * rot_ext, p_wl = rot * pos_ext + pos (lio_builder.cpp:252-253)
-__host__ __device__ inline void state_lidar_pose(const vmp_state& x, D33& r_wl, D3& p_wl) {
-  D33 rot = d33_from_cm(x.rot), ext = d33_from_cm(x.rot_ext);
-  r_wl = d33_mul(rot, ext);
-  D3 pe{{x.pos_ext[0], x.pos_ext[1], x.pos_ext[2]}};
-  D3 a = d33_mulv(rot, pe);
-  for (int i = 0; i < 3; ++i) p_wl.v[i] = a.v[i] + x.pos[i];
-}
-
 __host__ __device__ inline void split_f32(double v, float& hi, float& lo) {
   hi = float(v);
   lo = float(v - double(hi));
 }
 
-__host__ __device__ inline void sym6_from_P(const double* P, int o, float out[6]) {
-  // P column-major 23x23, block (o..o+2, o..o+2)
-  auto at = [&](int r, int c) { return P[(o + c) * 23 + (o + r)]; };
-  out[0] = float(at(0, 0));
-  out[1] = float(at(0, 1));
-  out[2] = float(at(0, 2));
-  out[3] = float(at(1, 1));
-  out[4] = float(at(1, 2));
-  out[5] = float(at(2, 2));
+// 1 / sqrt(x) and 1 / x for normal x > 0: the hardware's estimate (about 23
+// bits) and one third-order step
+__device__ inline double rsqrt_pos(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+__device__ inline double rcp_pos(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
 }
 
 // sin^2 of the angular resolution (commons.cpp:26-28)
@@ -271,52 +264,81 @@ __host__ __device__ inline float angle_s2(const vmp_map_cfg& cfg) {
   return float(sa * sa);
 }
 
-__host__ __device__ inline void make_obs_params(const vmp_state& x, const double* P, const vmp_map_cfg& cfg,
-                                                ObsParams& o) {
-  D33 r;
-  D3 p;
-  state_lidar_pose(x, r, p);
-  for (int i = 0; i < 9; ++i) o.r_wl[i] = r.m[i];
-  for (int i = 0; i < 3; ++i) o.p_wl[i] = p.v[i];
-  for (int i = 0; i < 9; ++i) split_f32(r.m[i], o.Rh[i], o.Rl[i]);
-  for (int i = 0; i < 3; ++i) {
-    o.anchor[i] = int64_t(floor(p.v[i] / cfg.voxel_size));
-    double loc = p.v[i] - double(o.anchor[i]) * cfg.voxel_size;
-    split_f32(loc, o.th[i], o.tl[i]);
+// entry k of a symmetric 3x3's upper triangle: its row and column
+__host__ __device__ constexpr int sym6_row(int k) { return k < 3 ? 0 : (k < 5 ? 1 : 2); }
+__host__ __device__ constexpr int sym6_col(int k) { return k < 3 ? k : (k < 5 ? k - 2 : 2); }
+
+// The parameters of an observe pass at state x, by the lanes of one wave: an
+// entry of the rotations each (0-8), of the translations (16-18), of P's two
+// blocks (32-43), the scalars (63).  P: column-major, at least its first six
+// columns; s2: angle_s2(cfg).  One lane forming all of them took 2.3 us at
+// the end of every filter iteration.
+__device__ inline void make_obs_params(const vmp_state& x, const double* P, const vmp_map_cfg& cfg, float s2,
+                                       int active, ObsParams& o, int lane) {
+  const double *R = x.rot, *E = x.rot_ext;  // column-major
+  if (lane < 9) {
+    const int i = lane / 3, j = lane % 3;
+    double r = R[i] * E[3 * j];
+    r += R[3 + i] * E[3 * j + 1];
+    r += R[6 + i] * E[3 * j + 2];
+    o.r_wl[lane] = r;
+    split_f32(r, o.Rh[lane], o.Rl[lane]);
+    o.rwl32[lane] = float(r);
+    o.rot[lane] = float(R[3 * j + i]);
+    o.ext_R[lane] = float(E[3 * j + i]);
+  } else if (lane >= 16 && lane < 19) {
+    const int i = lane - 16;
+    double p = R[i] * x.pos_ext[0];
+    p += R[3 + i] * x.pos_ext[1];
+    p += R[6 + i] * x.pos_ext[2];
+    p = p + x.pos[i];
+    o.p_wl[i] = p;
+    o.anchor[i] = int64_t(floor(p / cfg.voxel_size));
+    split_f32(p - double(o.anchor[i]) * cfg.voxel_size, o.th[i], o.tl[i]);
+    o.ext_t[i] = float(x.pos_ext[i]);
+  } else if (lane >= 32 && lane < 44) {
+    const int k = (lane - 32) % 6, b = lane < 38 ? 3 : 0;
+    const float v = float(P[(b + sym6_col(k)) * 23 + b + sym6_row(k)]);
+    if (b) o.Prr[k] = v;
+    else o.Ppp[k] = v;
+  } else if (lane == 63) {
+    o.vs = float(cfg.voxel_size);
+    o.inv_vs = float(1.0 / cfg.voxel_size);
+    o.vs64 = cfg.voxel_size;
+    o.s2 = s2;
+    o.rv = float(cfg.ranging_cov * cfg.ranging_cov);
+    o.estimate_ext = cfg.estimate_ext;
+    o.active = active;
   }
-  D33 rot = d33_from_cm(x.rot), ext = d33_from_cm(x.rot_ext);
-  for (int i = 0; i < 9; ++i) {
-    o.rot[i] = float(rot.m[i]);
-    o.rwl32[i] = float(r.m[i]);
-    o.ext_R[i] = float(ext.m[i]);
-  }
-  for (int i = 0; i < 3; ++i) o.ext_t[i] = float(x.pos_ext[i]);
-  sym6_from_P(P, 3, o.Prr);
-  sym6_from_P(P, 0, o.Ppp);
-  o.vs = float(cfg.voxel_size);
-  o.inv_vs = float(1.0 / cfg.voxel_size);
-  o.vs64 = cfg.voxel_size;
-  o.s2 = angle_s2(cfg);
-  o.rv = float(cfg.ranging_cov * cfg.ranging_cov);
-  o.estimate_ext = cfg.estimate_ext;
-  o.active = 1;
 }
 
-__host__ __device__ inline void make_upd_params(const vmp_state& x, const double* P, const vmp_map_cfg& cfg,
-                                                UpdParams& u) {
-  D33 r;
-  D3 p;
-  state_lidar_pose(x, r, p);
-  for (int i = 0; i < 9; ++i) {
-    u.m[i] = float(r.m[i]);  // (rot*rot_ext).cast<float>()
-    u.rwl32[i] = float(r.m[i]);
+// the insertion's parameters at state x, likewise
+__device__ inline void make_upd_params(const vmp_state& x, const double* P, const vmp_map_cfg& cfg, float s2,
+                                       UpdParams& u, int lane) {
+  const double *R = x.rot, *E = x.rot_ext;
+  if (lane < 9) {
+    const int i = lane / 3, j = lane % 3;
+    double r = R[i] * E[3 * j];
+    r += R[3 + i] * E[3 * j + 1];
+    r += R[6 + i] * E[3 * j + 2];
+    u.m[lane] = float(r);  // (rot*rot_ext).cast<float>()
+    u.rwl32[lane] = float(r);
+  } else if (lane >= 16 && lane < 19) {
+    const int i = lane - 16;
+    double p = R[i] * x.pos_ext[0];
+    p += R[3 + i] * x.pos_ext[1];
+    p += R[6 + i] * x.pos_ext[2];
+    u.t[i] = float(p + x.pos[i]);
+  } else if (lane >= 32 && lane < 44) {
+    const int k = (lane - 32) % 6, b = lane < 38 ? 3 : 0;
+    const float v = float(P[(b + sym6_col(k)) * 23 + b + sym6_row(k)]);
+    if (b) u.Prr[k] = v;
+    else u.Ppp[k] = v;
+  } else if (lane == 63) {
+    u.s2 = s2;
+    u.rv = float(cfg.ranging_cov * cfg.ranging_cov);
+    u.vs64 = cfg.voxel_size;
   }
-  for (int i = 0; i < 3; ++i) u.t[i] = float(p.v[i]);
-  sym6_from_P(P, 3, u.Prr);
-  sym6_from_P(P, 0, u.Ppp);
-  u.s2 = angle_s2(cfg);
-  u.rv = float(cfg.ranging_cov * cfg.ranging_cov);
-  u.vs64 = cfg.voxel_size;
 }
 
 // -------------------------------------------------- FP32 point helpers -----

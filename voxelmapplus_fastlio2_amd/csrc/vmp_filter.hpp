@@ -18,19 +18,26 @@ __device__ inline void load_state(const vmp_state& src, vmp_state& dst, int lane
 __global__ void k_obs_prep(FilterDev** fs, int32_t** obs_ctr) {
   FilterDev* f = fs[blockIdx.x];
   if (threadIdx.x < 8) obs_ctr[blockIdx.x][threadIdx.x] = 0;
-  if (threadIdx.x == 0) make_obs_params(f->x, f->P, f->cfg, f->obs_prm);
+  make_obs_params(f->x, f->P, f->cfg, f->s2, 1, f->obs_prm, threadIdx.x);
 }
 // the same at a given state, which becomes the session's
 __global__ void k_obs_prep_at(FilterDev* f, vmp_state x, int32_t* obs_ctr) {
   if (threadIdx.x < 8) obs_ctr[threadIdx.x] = 0;
+  __shared__ vmp_state sx;  // (the lanes index into it)
   if (threadIdx.x == 0) {
+    sx = x;
     f->x = x;
-    make_obs_params(x, f->P, f->cfg, f->obs_prm);
   }
+  __syncthreads();
+  make_obs_params(sx, f->P, f->cfg, f->s2, 1, f->obs_prm, threadIdx.x);
 }
 __global__ void k_upd_prep(FilterDev** fs) {
   FilterDev* f = fs[blockIdx.x];
-  if (threadIdx.x == 0) make_upd_params(f->x, f->P, f->cfg, f->upd_prm);
+  make_upd_params(f->x, f->P, f->cfg, f->s2, f->upd_prm, threadIdx.x);
+}
+// a new session's constants
+__global__ void k_filter_init(FilterDev* f) {
+  if (threadIdx.x == 0) f->s2 = angle_s2(f->cfg);
 }
 
 struct Diag23 {
@@ -97,8 +104,8 @@ __global__ void __launch_bounds__(kBeginEndThreads) k_ieskf_begin(FilterDev** fs
   if (lane == 0) {
     f->iters = 0;
     f->active = 1;
-    make_obs_params(sx, f->P, f->cfg, f->obs_prm);
   }
+  if (lane >= 64 && lane < 128) make_obs_params(sx, f->P, f->cfg, f->s2, 1, f->obs_prm, lane - 64);
 }
 
 // one IESKF iteration after an observe pass (ieskf.cpp:133-149)
@@ -136,6 +143,8 @@ k_ieskf_step(FilterDev** fs, const ObsJob* __restrict__ jobs, int32_t** obs_ctr,
   for (int i = lane; i < 529; i += kStepThreads) Pi[i] = f->Pinv[i];
   if (lane < 6 * 23) Pc[lane] = f->P[lane];
   if (lane == 0) scfg = f->cfg;
+  const int it0 = f->iters;
+  const float ss2 = f->s2;
   {
     const ObsJob& J = jobs[blockIdx.x];
     const auto part = as_global(J.partials);
@@ -205,34 +214,32 @@ k_ieskf_step(FilterDev** fs, const ObsJob* __restrict__ jobs, int32_t** obs_ctr,
   if (lane < 23) {
     const int r = lane;
     double t[23];
-    // JtPi[r][c] = sum_k J[k][r] Pi[k][c]; a block row sums its nonzero terms
-    // in ascending k (the zero terms of the dense sum add nothing)
-    if (r >= 3 && r < 6) {
-#pragma unroll
-      for (int c = 0; c < 23; ++c) {
-        double s = jb.a[0 * 3 + (r - 3)] * Pi[3 * 23 + c];
-        s += jb.a[1 * 3 + (r - 3)] * Pi[4 * 23 + c];
-        s += jb.a[2 * 3 + (r - 3)] * Pi[5 * 23 + c];
-        t[c] = s;
-      }
-    } else if (r >= 6 && r < 9) {
-#pragma unroll
-      for (int c = 0; c < 23; ++c) {
-        double s = jb.b[0 * 3 + (r - 6)] * Pi[6 * 23 + c];
-        s += jb.b[1 * 3 + (r - 6)] * Pi[7 * 23 + c];
-        s += jb.b[2 * 3 + (r - 6)] * Pi[8 * 23 + c];
-        t[c] = s;
-      }
+    // JtPi[r][c] = sum_k J[k][r] Pi[k][c]: the (up to three) nonzero terms in
+    // ascending k, every row in the same instructions (rows of the identity
+    // take zero factors for the rest, which add nothing)
+    double j0 = 1.0, j1 = 0.0, j2 = 0.0;
+    int k0 = r, k1 = r, k2 = r;
+    if (r >= 3 && r < 9) {
+      const double* blk = r < 6 ? jb.a : jb.b;
+      const int q = (r - 3) % 3;
+      k0 = r < 6 ? 3 : 6;
+      k1 = k0 + 1;
+      k2 = k0 + 2;
+      j0 = blk[q];
+      j1 = blk[3 + q];
+      j2 = blk[6 + q];
     } else if (r >= 21) {
+      k0 = 21;
+      k1 = 22;
+      j0 = jb.c[r - 21];
+      j1 = jb.c[2 + r - 21];
+    }
 #pragma unroll
-      for (int c = 0; c < 23; ++c) {
-        double s = jb.c[0 * 2 + (r - 21)] * Pi[21 * 23 + c];
-        s += jb.c[1 * 2 + (r - 21)] * Pi[22 * 23 + c];
-        t[c] = s;
-      }
-    } else {
-#pragma unroll
-      for (int c = 0; c < 23; ++c) t[c] = Pi[r * 23 + c];
+    for (int c = 0; c < 23; ++c) {
+      double s = j0 * Pi[k0 * 23 + c];
+      s += j1 * Pi[k1 * 23 + c];
+      s += j2 * Pi[k2 * 23 + c];
+      t[c] = s;
     }
     // H_[r][c] = sum_k JtPi[r][k] J[k][c]
 #pragma unroll
@@ -276,16 +283,19 @@ k_ieskf_step(FilterDev** fs, const ObsJob* __restrict__ jobs, int32_t** obs_ctr,
   if (lane < 23) f->delta[lane] = dl[lane];
   state_plus_par(sx, dl, lane);
   load_state(sx, f->x, lane);
+  // converged: signed maxCoeff (ieskf.cpp:148)
+  double mx = dl[0];
+#pragma unroll
+  for (int k = 1; k < 23; ++k) mx = mx > dl[k] ? mx : dl[k];
+  const int iters = it0 + 1;
+  const int active = (mx < 0.001 || iters >= scfg.max_iter) ? 0 : 1;
+  if (lane >= 64 && lane < 128) make_obs_params(sx, Pc, scfg, ss2, active, f->obs_prm, lane - 64);
   if (lane == 0) {
-    f->iters += 1;
-    double mx = dl[0];
-    for (int k = 1; k < 23; ++k) mx = mx > dl[k] ? mx : dl[k];
-    if (mx < 0.001 || f->iters >= scfg.max_iter) f->active = 0;  // signed maxCoeff (ieskf.cpp:148)
-    make_obs_params(sx, Pc, scfg, f->obs_prm);
-    f->obs_prm.active = f->active;
+    f->iters = iters;
+    f->active = active;
     int32_t* so = stat_out[blockIdx.x];
     int32_t* oc = obs_ctr[blockIdx.x];
-    if (f->iters == 1)
+    if (iters == 1)
       for (int k = 4; k < 8; ++k) so[k] = 0;
     int32_t cnt[4];  // hits, plane hits, effective, fallbacks of this pass
     for (int k = 0; k < 4; ++k) cnt[k] = int32_t(red[NACC + k]);
@@ -365,10 +375,8 @@ __global__ void __launch_bounds__(kBeginEndThreads) k_ieskf_end(FilterDev** fs) 
     f->P[c * 23 + r] = s;  // column-major
   }
   __syncthreads();
-  if (lane == 0) {
-    make_upd_params(sx, f->P, f->cfg, f->upd_prm);
-    f->active = 0;
-  }
+  if (lane < 64) make_upd_params(sx, f->P, f->cfg, f->s2, f->upd_prm, lane);
+  if (lane == 64) f->active = 0;
 }
 
 }  // namespace vmp

@@ -25,9 +25,10 @@ struct FilterDev {
   ObsParams obs_prm;
   UpdParams upd_prm;
   vmp_map_cfg cfg;
+  float s2;        // angle_s2(cfg), set at the session's creation
   int32_t iters;
   int32_t active;
-  int32_t pad[2];
+  int32_t pad;
 };
 
 // ------------------------------------------------------- SO3 in FP64 ------
@@ -183,58 +184,19 @@ __device__ inline void s2_minus_d(const double* g, const double* og, double* out
   }
 }
 
-// x += d (ieskf.cpp:11-21)
-__device__ inline void state_plus(vmp_state& x, const double d[23]) {
-  for (int i = 0; i < 3; ++i) x.pos[i] += d[i];
-  d33_to_cm(d33_mul(d33_from_cm(x.rot), so3_exp_d(d + 3)), x.rot);
-  d33_to_cm(d33_mul(d33_from_cm(x.rot_ext), so3_exp_d(d + 6)), x.rot_ext);
-  for (int i = 0; i < 3; ++i) {
-    x.pos_ext[i] += d[9 + i];
-    x.vel[i] += d[12 + i];
-    x.bg[i] += d[15 + i];
-    x.ba[i] += d[18 + i];
-  }
-  double B[6];
-  getBx_d(x.g, B);
-  const double w[3] = {B[0] * d[21] + B[1] * d[22], B[2] * d[21] + B[3] * d[22], B[4] * d[21] + B[5] * d[22]};
-  const D33 E = so3_exp_d(w);
-  double g2[3];
-  for (int i = 0; i < 3; ++i) g2[i] = E.m[i * 3] * x.g[0] + E.m[i * 3 + 1] * x.g[1] + E.m[i * 3 + 2] * x.g[2];
-  for (int i = 0; i < 3; ++i) x.g[i] = g2[i];
-}
-
 // blocks of J (and L): right Jacobians of the two rotations, S2 block
 struct JacBlocks {
   double a[9], b[9], c[4];
 };
-__device__ inline void jac_blocks(const vmp_state& x, const vmp_state& xp, const double d[23], JacBlocks& J) {
-  // right Jacobian = leftJacobian(w)^T
-  const D33 A = d33_t(left_jac_d(d + 3)), B = d33_t(left_jac_d(d + 6));
-  for (int i = 0; i < 9; ++i) {
-    J.a[i] = A.m[i];
-    J.b[i] = B.m[i];
-  }
-  double N[6], M[6];
-  getNx_d(x.g, N);
-  getMx_d(xp.g, d + 21, M);
-  for (int r = 0; r < 2; ++r)
-    for (int c = 0; c < 2; ++c) J.c[r * 2 + c] = N[r * 3] * M[c] + N[r * 3 + 1] * M[2 + c] + N[r * 3 + 2] * M[4 + c];
-}
-// element (r, c) of the 23x23 J built from the blocks
-__device__ inline double jac_at(const JacBlocks& J, int r, int c) {
-  if (r >= 3 && r < 6 && c >= 3 && c < 6) return J.a[(r - 3) * 3 + (c - 3)];
-  if (r >= 6 && r < 9 && c >= 6 && c < 9) return J.b[(r - 6) * 3 + (c - 6)];
-  if (r >= 21 && c >= 21) return J.c[(r - 21) * 2 + (c - 21)];
-  return r == c ? 1.0 : 0.0;
-}
-
 // ---- Cholesky factorisation, solve and inverse of a symmetric positive
 //      definite 23x23 on rows held in lanes ---------------------------------
 // Lane i (< 23) holds row i of the matrix in a[0..22]; values cross lanes by
 // readlane (uniform index), so nothing goes through LDS and no barrier is
 // needed.  The factorisation is right-looking (column k scaled, then the
 // trailing lower triangle updated in ascending column order); divisions by a
-// diagonal element are products with its reciprocal (kept per lane in dinv).
+// diagonal element are products with its reciprocal (kept per lane in dinv),
+// which comes from a reciprocal square root (a square root and a division in
+// every column's chain took about 1.4 us more per factorisation).
 __device__ inline double rl64(double v, int src) {
   const long long x = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_readlane(int(x), src);
@@ -248,8 +210,10 @@ __device__ inline void chol_rows(double (&a)[23], double& dinv, int lane) {
   dinv = 0.0;
 #pragma unroll
   for (int k = 0; k < 23; ++k) {
-    const double d = sqrt(rl64(a[k], k));
-    const double inv = 1.0 / d;
+    const double v = rl64(a[k], k);
+    const double inv = rsqrt_pos(v);
+    double d = v * inv;
+    d = fma(fma(-d, d, v), 0.5 * inv, d);
     if (lane == k) {
       a[k] = d;
       dinv = inv;
@@ -337,35 +301,36 @@ __device__ inline void chol_inverse_rows(const double (&a)[23], double dinv, dou
   __syncthreads();  // S may be reused by the caller
 }
 
-// ---- lane-parallel pieces of the state algebra (inputs in LDS) ----------
-// x - xp split over three lanes: rotation, extrinsic rotation, gravity chart
-__device__ inline void state_minus_par(const vmp_state& x, const vmp_state& o, double* d, int lane) {
-  if (lane == 0) {
-    so3_log_d(d33_mul(d33_t(d33_from_cm(o.rot)), d33_from_cm(x.rot)), d + 3);
-  } else if (lane == 1) {
-    so3_log_d(d33_mul(d33_t(d33_from_cm(o.rot_ext)), d33_from_cm(x.rot_ext)), d + 6);
-  } else if (lane == 2) {
+// ---- pieces of the state algebra on the waves of a workgroup of at least
+//      three (inputs in LDS): the two rotations on two lanes of the first
+//      wave, in the same instructions; the gravity part on the second, the
+//      vector parts on the third.  On one wave the three kinds ran one after
+//      the other (3.0, 4.3 and 3.5 us of a filter iteration, about half now).
+constexpr int kVecPart[5] = {0, 9, 12, 15, 18};  // offsets of pos, pos_ext, vel, bg, ba in the error state
+__device__ inline double* state_vec(vmp_state& x, int part) {
+  return part == 0 ? x.pos : (part == 1 ? x.pos_ext : (part == 2 ? x.vel : (part == 3 ? x.bg : x.ba)));
+}
+// d = x - xp
+__device__ inline void state_minus_par(vmp_state& x, vmp_state& o, double* d, int tid) {
+  if (tid < 2) {
+    const double* a = tid == 0 ? o.rot : o.rot_ext;
+    const double* b = tid == 0 ? x.rot : x.rot_ext;
+    so3_log_d(d33_mul(d33_t(d33_from_cm(a)), d33_from_cm(b)), d + 3 + 3 * tid);
+  } else if (tid == 64) {
     s2_minus_d(x.g, o.g, d + 21);
-  } else if (lane == 3) {
-    for (int i = 0; i < 3; ++i) {
-      d[i] = x.pos[i] - o.pos[i];
-      d[9 + i] = x.pos_ext[i] - o.pos_ext[i];
-      d[12 + i] = x.vel[i] - o.vel[i];
-      d[15 + i] = x.bg[i] - o.bg[i];
-      d[18 + i] = x.ba[i] - o.ba[i];
-    }
+  } else if (tid >= 128 && tid < 143) {
+    const int part = (tid - 128) / 3, i = (tid - 128) % 3;
+    d[kVecPart[part] + i] = state_vec(x, part)[i] - state_vec(o, part)[i];
   }
   __syncthreads();
 }
 __device__ inline void jac_blocks_par(const vmp_state& x, const vmp_state& xp, const double* d, JacBlocks& J,
-                                      int lane) {
-  if (lane == 0) {
-    const D33 A = d33_t(left_jac_d(d + 3));
-    for (int i = 0; i < 9; ++i) J.a[i] = A.m[i];
-  } else if (lane == 1) {
-    const D33 B = d33_t(left_jac_d(d + 6));
-    for (int i = 0; i < 9; ++i) J.b[i] = B.m[i];
-  } else if (lane == 2) {
+                                      int tid) {
+  if (tid < 2) {  // right Jacobian = leftJacobian(w)^T
+    const D33 A = d33_t(left_jac_d(d + 3 + 3 * tid));
+    double* out = tid == 0 ? J.a : J.b;
+    for (int i = 0; i < 9; ++i) out[i] = A.m[i];
+  } else if (tid == 64) {
     double N[6], M[6];
     getNx_d(x.g, N);
     getMx_d(xp.g, d + 21, M);
@@ -374,12 +339,12 @@ __device__ inline void jac_blocks_par(const vmp_state& x, const vmp_state& xp, c
   }
   __syncthreads();
 }
-__device__ inline void state_plus_par(vmp_state& x, const double* d, int lane) {
-  if (lane == 0) {
-    d33_to_cm(d33_mul(d33_from_cm(x.rot), so3_exp_d(d + 3)), x.rot);
-  } else if (lane == 1) {
-    d33_to_cm(d33_mul(d33_from_cm(x.rot_ext), so3_exp_d(d + 6)), x.rot_ext);
-  } else if (lane == 2) {
+// x += d (ieskf.cpp:11-21)
+__device__ inline void state_plus_par(vmp_state& x, const double* d, int tid) {
+  if (tid < 2) {
+    double* R = tid == 0 ? x.rot : x.rot_ext;
+    d33_to_cm(d33_mul(d33_from_cm(R), so3_exp_d(d + 3 + 3 * tid)), R);
+  } else if (tid == 64) {
     double B[6];
     getBx_d(x.g, B);
     const double w[3] = {B[0] * d[21] + B[1] * d[22], B[2] * d[21] + B[3] * d[22], B[4] * d[21] + B[5] * d[22]};
@@ -387,59 +352,10 @@ __device__ inline void state_plus_par(vmp_state& x, const double* d, int lane) {
     double g2[3];
     for (int i = 0; i < 3; ++i) g2[i] = E.m[i * 3] * x.g[0] + E.m[i * 3 + 1] * x.g[1] + E.m[i * 3 + 2] * x.g[2];
     for (int i = 0; i < 3; ++i) x.g[i] = g2[i];
-  } else if (lane == 3) {
-    for (int i = 0; i < 3; ++i) {
-      x.pos[i] += d[i];
-      x.pos_ext[i] += d[9 + i];
-      x.vel[i] += d[12 + i];
-      x.bg[i] += d[15 + i];
-      x.ba[i] += d[18 + i];
-    }
+  } else if (tid >= 128 && tid < 143) {
+    const int part = (tid - 128) / 3, i = (tid - 128) % 3;
+    state_vec(x, part)[i] += d[kVecPart[part] + i];
   }
-  __syncthreads();
-}
-
-// Gauss-Jordan inverse with partial pivoting of the 23x23 row-major M (LDS),
-// one wave; result in Inv (LDS).  W is a 23x46 LDS workspace, fac 23 doubles.
-__device__ inline void gj_inverse(const double* M, double* Inv, double (*W)[47], double* fac, int lane) {
-  constexpr int n = 23;
-  for (int idx = lane; idx < n * 2 * n; idx += 64) {
-    const int r = idx / (2 * n), c = idx % (2 * n);
-    W[r][c] = c < n ? M[r * n + c] : (c - n == r ? 1.0 : 0.0);
-  }
-  __syncthreads();
-  for (int k = 0; k < n; ++k) {
-    double v = (lane >= k && lane < n) ? fabs(W[lane][k]) : -1.0;
-    int pi = lane;
-    for (int o = 32; o > 0; o >>= 1) {
-      const double ov = __shfl_xor(v, o, 64);
-      const int op = __shfl_xor(pi, o, 64);
-      if (ov > v || (ov == v && op < pi)) {
-        v = ov;
-        pi = op;
-      }
-    }
-    if (pi != k) {
-      for (int c = lane; c < 2 * n; c += 64) {
-        const double t = W[k][c];
-        W[k][c] = W[pi][c];
-        W[pi][c] = t;
-      }
-    }
-    __syncthreads();
-    const double d = W[k][k];
-    __syncthreads();
-    for (int c = lane; c < 2 * n; c += 64) W[k][c] = W[k][c] / d;
-    __syncthreads();
-    if (lane < n) fac[lane] = W[lane][k];
-    __syncthreads();
-    for (int idx = lane; idx < n * 2 * n; idx += 64) {
-      const int r = idx / (2 * n), c = idx % (2 * n);
-      if (r != k) W[r][c] -= fac[r] * W[k][c];
-    }
-    __syncthreads();
-  }
-  for (int idx = lane; idx < n * n; idx += 64) Inv[idx] = W[idx / n][n + idx % n];
   __syncthreads();
 }
 

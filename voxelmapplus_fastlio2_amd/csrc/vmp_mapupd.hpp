@@ -280,19 +280,6 @@ __host__ __device__ constexpr int s6(int a, int b) {
   return a <= b ? (a == 0 ? b : (a == 1 ? 2 + b : 5)) : (b == 0 ? a : (b == 1 ? 2 + a : 5));
 }
 
-// 1 / sqrt(x) and 1 / x for normal x > 0: the hardware's estimate (about 23
-// bits) and one third-order step
-__device__ inline double rsqrt_pos(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
-}
-__device__ inline double rcp_pos(double x) {
-  const double y = __builtin_amdgcn_rcp(x);
-  const double e = fma(-x, y, 1.0);
-  return fma(y, fma(e, e, e), y);
-}
-
 // One Jacobi rotation in the plane (p, q): apq becomes zero, apr and aqr are
 // the elements coupling p and q to the third axis, vp and vq the columns of V.
 // The angle comes from cos and sin of twice the angle, two reciprocal square
