@@ -602,7 +602,7 @@ def kernel_rooflines(tt, kt, stats, N, scans):
         "k_imu_predict": (stats["pred_bytes"], f"{PRED_BYTES} B + {PRED_SAMPLE_BYTES} B x IMU samples"),
         "k_candidates": (CAND_VOXEL_BYTES * stats["touched"], f"{CAND_VOXEL_BYTES} B x touched voxels"),
         "k_ins_keys": (INS_BYTES_POINT * stats["points"], f"{INS_BYTES_POINT} B x points"),
-        "k_replay_heavy": (REFIT_BYTES * stats["refits"], f"{REFIT_BYTES} B x refits (k_replay_heavy_wave and "
+        "k_replay_heavy": (REFIT_BYTES * stats["refits"], f"{REFIT_BYTES} B x refits (k_replay on those voxels and "
                            "k_replay_heavy together)"),
         "k_merge_replay": (MERGE_BYTES * stats["merge_evals"], f"{MERGE_BYTES} B x merge() evaluations"),
         "k_create_evict": (LRU_BYTES * (stats["created"] + stats["evicted"]), f"{LRU_BYTES} B x (creations + evictions)"),

@@ -321,8 +321,10 @@ int vmp_session_timing_totals(vmp_session* s, double* obs_ms, int64_t* obs_launc
  * reference counterpart): milliseconds and launches of, in this order,
  * k_ins_keys, k_create_evict, k_replay_heavy, k_replay_light,
  * k_merge_replay, k_candidates, k_ring_live, k_ieskf_step, k_undistort,
- * k_imu_predict, k_spec_eval.  Returns the number of kernels (up to cap
- * entries are written). */
+ * k_imu_predict, k_spec_eval.  (k_replay runs once for both replay paths;
+ * while timing is on it is launched for each, as k_replay_heavy with the
+ * per-lane kernel of that name, and as k_replay_light.)  Returns the number of
+ * kernels (up to cap entries are written). */
 int32_t vmp_ctx_kernel_times(vmp_ctx* ctx, int32_t cap, double* total_ms, int64_t* launches);
 
 #ifdef __cplusplus

@@ -119,7 +119,7 @@ struct BatchOut {
 };
 constexpr int kFinishThreads = 256;
 // End of a step, a block per session: the map update's counters advance (the
-// LRU appends, the points, and the evicted voxels that k_evict_finalize
+// LRU appends, the points, and the evicted voxels that k_finalize
 // pushed above the free-list top; nevict stays 0 in a scan without points),
 // the results go to the host, and the last block to finish (counted in
 // *done) sets the signal word the host waits for.  One launch in place of
@@ -139,7 +139,7 @@ __global__ void __launch_bounds__(kFinishThreads) k_finish(const MapDev* maps, c
       o.clk[2] = wall_clock64();
     }
     if (map_step) {
-      c->ring_tail += c->nlru;
+      c->ring_tail += c->nseg;
       c->point_base += si[s].n;
       c->free_top += c->nevict;
     }
@@ -624,7 +624,7 @@ static bool ws_layout(vmp_ctx* c, BatchWs& w, size_t n, int ns, size_t pre_cap, 
        dev(&b.cand_spec, n) &&
        dev(&b.cand_start, size_t(ns)) && dev(&b.spl, n);
   ok = ok && dev(&b.seg_ct, n * 7) && dev(&b.seg_nct, n) && dev(&b.seg_nbr, n * 6);
-  ok = ok && dev(&b.len_in, n) && dev(&b.len_out, n) && dev(&b.ord_in, n) && dev(&b.ord, n);
+  ok = ok && dev(&b.seg_cls, n) && dev(&b.seg_old, n);
   ok = ok && dev(&b.lv, n * 2) && dev(&b.lv2, n * 2) && dev(&b.lv_cnt, (n * 2 >> 6) + size_t(ns) + 2);
   ok = ok && dev(&b.prim, prim_ws_entries(int64_t(n))) && dev(&b.qc, n * 3);
   // the refitting-voxel list of the replay lives in cand_nbr's memory (24 B
@@ -669,12 +669,11 @@ static bool ws_layout(vmp_ctx* c, BatchWs& w, size_t n, int ns, size_t pre_cap, 
   ok = ok && host(&w.h_out, sizeof(BatchOut) * S) && host(&w.h_motion, sizeof(MotionRec) * S) &&
        host(&w.h_vg, sizeof(VgJob) * S) && host(&w.h_vgst, sizeof(int32_t) * kVgStat * S);
   if (!ok) return false;
-  size_t t[4] = {0, 0, 0, 0};
+  size_t t[3] = {0, 0, 0};
   rocprim::radix_sort_pairs(nullptr, t[0], b.skey_in, b.skey_out, b.sval_in, b.sval_out, n, 0, 64, c->stream);
   rocprim::radix_sort_keys(nullptr, t[1], b.cand_in, b.cand_out, n, 0, 64, c->stream);
   rocprim::select(nullptr, t[2], rocprim::counting_iterator<int32_t>(0), b.flags, b.sel, b.cnt, n, c->stream);
-  rocprim::radix_sort_pairs(nullptr, t[3], b.len_in, b.len_out, b.ord_in, b.ord, n, 0, 32, c->stream);
-  w.temp_bytes = *std::max_element(t, t + 4) + 256;
+  w.temp_bytes = *std::max_element(t, t + 3) + 256;
   uint8_t* temp = nullptr;
   if (!dev(&temp, w.temp_bytes)) return false;
   w.temp = temp;
@@ -1723,11 +1722,9 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
     for (int i = 0; i < n; ++i)
       while ((int64_t(1) << tbits) < int64_t(ss[i]->n)) ++tbits;
     b.cand_sshift = 25 + tbits;
-    // the stage's launches; `lbits` etc. depend only on the step's shape
-    int lbits = 1;  // replay order by segment length, capped at 6 bits
-    while ((int64_t(1) << lbits) <= int64_t(ntot) && lbits < 6) ++lbits;
-    // long segments sort first only below the length clamp (2^lbits - 2)
-    const int long_seg = c->replay_long_seg < (1 << lbits) - 1 ? c->replay_long_seg : 0;
+    // the stage's launches; what they are given depends only on the step's
+    // shape and the context's settings
+    const int long_seg = c->replay_long_seg;
     const int wave_max = c->replay_wave_max;
     // every session's counters are the ones its last step returned (a step
     // on this context starts only after the previous one finished), and a
@@ -1760,20 +1757,22 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
       return rocprim::radix_sort_pairs(w.temp, tb, kin, kout, vin, vout, size_t(ntot), 0, bits, st) == hipSuccess;
     };
     auto map_stage = [&]() -> int {
-      hipLaunchKernelGGL(k_begin_scan, dim3(n), dim3(1), 0, st, M, n, w.d_clk);
+      timed_launch(c, kTkInsKeys, [&] {
+        hipLaunchKernelGGL(k_ins_keys, dim3(std::max(gn, 1)), dim3(T), 0, st, M, S, n, b, w.d_clk);
+      });
       if (ntot > 0) {
-        timed_launch(c, kTkInsKeys, [&] { hipLaunchKernelGGL(k_ins_keys, dim3(gn), dim3(T), 0, st, M, S, n, b); });
         // one stable radix sort over (session, hash slot): every key's points
         // become a contiguous segment in point order, sessions stay in order
         if (!sort_pairs(b.skey_in, b.sval_in, b.skey_out, b.sval_out, hbits + sbits)) return VMP_EDEVICE;
-        hipLaunchKernelGGL(k_seg_heads, dim3(gn), dim3(T), 0, st, M, S, n, b);
-        // the library's compaction also clears the flags it reads, computes
-        // the per-session ranges in its last tile and (creation events)
-        // splits each event into its time and segment
+        // the library's compaction finds the segment heads in the keys, also
+        // clears the flags it reads, computes the per-session ranges in its
+        // last tile and (creation events) splits each event into its time and
+        // segment
         if (prim) {
-          select_stable(st, ntot, PredFlagClear{b.flags}, OutIndex{b.sel}, b.prim, b.cnt + 0,
+          select_stable(st, ntot, PredHead{b.skey_out}, OutIndex{b.sel}, b.prim, b.cnt + 0,
                         TailRanges{M, S, n, b.sel, 0, w.d_sfirst, ntot});
         } else {
+          hipLaunchKernelGGL(k_seg_heads, dim3(gn), dim3(T), 0, st, b);
           if (!select_flags(b.flags, b.sel, b.cnt + 0)) return VMP_EDEVICE;
           hipLaunchKernelGGL(k_ranges, dim3(grid_for(n, 64)), dim3(64), 0, st, M, S, n, b.sel, b.cnt + 0, 0);
           hipLaunchKernelGGL(k_fill_i32, dim3(gn), dim3(T), 0, st, b.flags, 0, ntot);
@@ -1787,7 +1786,6 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
           hipLaunchKernelGGL(k_ranges, dim3(grid_for(n, 64)), dim3(64), 0, st, M, S, n, b.sel, b.cnt + 1, 1);
           hipLaunchKernelGGL(k_cre_split, dim3(gn), dim3(T), 0, st, S, n, b);
         }
-        hipLaunchKernelGGL(k_create_fast, dim3(gn), dim3(T), 0, st, M, S, n, b);
         if (!all_fast) {
           timed_launch(c, kTkRingLive, [&] {
             hipLaunchKernelGGL(k_ring_live, dim3(kLvBlocks, n), dim3(64 * kLvWaves), 0, st, M, S, n, b);
@@ -1795,12 +1793,7 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
           timed_launch(c, kTkCreateEvict,
                        [&] { hipLaunchKernelGGL(k_create_evict, dim3(n), dim3(kCeThreads), 0, st, M, S, n, b); });
         }
-        hipLaunchKernelGGL(k_create_init, dim3(gn), dim3(T), 0, st, M, S, n, b);
-        // replay order by segment length in 6 bits (one radix pass; segments
-        // of 62 points and more share the first key): the order only spreads
-        // the work evenly over waves, every segment replays on its own
-        hipLaunchKernelGGL(k_seg_lenkeys, dim3(gn), dim3(T), 0, st, M, S, b, lbits, long_seg);
-        if (!sort_pairs(b.len_in, b.ord_in, b.len_out, b.ord, lbits + 1)) return VMP_EDEVICE;
+        hipLaunchKernelGGL(k_create_init, dim3(gn), dim3(T), 0, st, M, S, n, b, long_seg);
         // the moment path: a voxel per wave up to wave_max refitting voxels,
         // else for the long segments only and 64 voxels per wave for the
         // rest; the light path covers the voxels that do not refit.  The
@@ -1808,12 +1801,26 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
         // this kernel's registers), a quarter as many as points for small
         // scans (a wave per 64 points left 88 voxels of a 2,003-point scan
         // to 32 waves, three refits after one another: 68 us against 24).
-        const int heavy_blocks = std::max(1, std::min((ntot + 15) / 16, 512));
-        timed_launch(c, kTkReplayHeavy, [&] {
-          hipLaunchKernelGGL(k_replay_heavy_wave, dim3(heavy_blocks), dim3(T), 0, st, M, S, b, wave_max);
-          hipLaunchKernelGGL(k_replay_heavy, dim3(std::min(gn, 256)), dim3(T), 0, st, M, S, b, wave_max);
-        });
-        timed_launch(c, kTkReplayLight, [&] { hipLaunchKernelGGL(k_replay_light, dim3(gn), dim3(T), 0, st, M, S, b); });
+        // One launch for both paths, two when each is timed.
+        const int hb = std::max(1, std::min((ntot + 15) / 16, 512));
+        const bool lanes = ntot > wave_max;  // more refitting voxels than waves may be given
+        auto replay = [&](int heavy, int light) {
+          hipLaunchKernelGGL(k_replay, dim3(heavy + light), dim3(T), 0, st, M, S, b, wave_max, heavy);
+        };
+        auto replay_lanes = [&] {
+          if (lanes)
+            hipLaunchKernelGGL(k_replay_heavy, dim3(std::min(gn, 256)), dim3(T), 0, st, M, S, b, wave_max, long_seg);
+        };
+        if (c->timing) {
+          timed_launch(c, kTkReplayHeavy, [&] {
+            replay(hb, 0);
+            replay_lanes();
+          });
+          timed_launch(c, kTkReplayLight, [&] { replay(0, gn); });
+        } else {
+          replay(hb, gn);
+          replay_lanes();
+        }
         if (!(mode & kStepBuild)) {
           timed_launch(c, kTkCandidates, [&] { hipLaunchKernelGGL(k_candidates, dim3(gn), dim3(T), 0, st, M, S, b); });
           // the call at point time t is made by the voxel that received point
@@ -1844,22 +1851,20 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
         }
         // (the library's compaction of the creation events left the flags cleared)
         if (!prim) hipLaunchKernelGGL(k_fill_i32, dim3(gn), dim3(T), 0, st, b.flags, 0, ntot);
-        hipLaunchKernelGGL(k_finalize_segs, dim3(gn), dim3(T), 0, st, M, S, b);
-        hipLaunchKernelGGL(k_evict_finalize, dim3(gn), dim3(T), 0, st, M, S, n, b);
+        hipLaunchKernelGGL(k_finalize, dim3(gn), dim3(T), 0, st, M, S, n, b, all_fast ? 0 : 1);
+        const OutLru lru{M, S, n};
         if (prim) {
-          select_stable(st, ntot, PredFlag{b.flags}, OutIndex{b.sel}, b.prim, b.cnt + 2,
-                        TailRanges{M, S, n, b.sel, 2, w.d_sfirst, ntot});
+          select_stable(st, ntot, PredFlag{b.flags}, lru, b.prim, b.cnt + 2);
         } else {
           if (!select_flags(b.flags, b.sel, b.cnt + 2)) return VMP_EDEVICE;
-          hipLaunchKernelGGL(k_ranges, dim3(grid_for(n, 64)), dim3(64), 0, st, M, S, n, b.sel, b.cnt + 2, 2);
+          hipLaunchKernelGGL(k_lru_append, dim3(gn), dim3(T), 0, st, lru, b);
         }
-        hipLaunchKernelGGL(k_lru_append, dim3(gn), dim3(T), 0, st, M, S, n, b);
       }
       return VMP_OK;
     };
     const int64_t key[3] = {int64_t(ntot), int64_t(n),
                             int64_t(hbits) | (int64_t(sbits) << 8) | (int64_t(tbits) << 16) |
-                                (int64_t(lbits) << 24) | (int64_t(all_fast) << 32) |
+                                (int64_t(all_fast) << 24) |
                                 (int64_t(mode & kStepBuild) << 32) |
                                 (int64_t(long_seg) << 36) | (int64_t(wave_max) << 42)};
     hipGraphExec_t mexec = (c->use_graph && c->use_map_graph && !c->timing) ? map_graph(c, key, map_stage) : nullptr;

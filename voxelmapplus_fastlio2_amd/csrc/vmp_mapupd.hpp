@@ -48,7 +48,7 @@ struct MapCounters {
   int32_t nseg, ncreate_ev, ncre, nevict, ncand;
   int32_t refits, merge_calls, merge_evals, merges, dropped;
   int32_t fast;            // 1: this scan's creations took the parallel (no-eviction) path
-  int32_t nlru;            // voxels appended to the LRU queue by this scan
+  int32_t pad1;
   int32_t merge_windows;   // windows of the merge replay
   int32_t merge_requeued;  // window entries sent back for re-evaluation
   int32_t merge_max_acting;  // most acting entries in one window of the merge replay
@@ -87,7 +87,6 @@ struct SessInfo {
   int32_t is_build;
   int32_t seg_lo, seg_hi;  // its segments in the batch segment list
   int32_t cre_lo, cre_hi;  // its creation events in the batch creation list
-  int32_t lru_lo, lru_hi;  // its LRU appends in the batch append list
   int32_t spl_lo, spl_hi;  // its acting merge candidates in the compacted list
   int32_t ftop0, bump0;    // free-list top and bump pointer before its fast creations
 };
@@ -104,7 +103,8 @@ struct BatchBufs {
   int32_t* sval_out;
   int32_t* flags;      // scratch flag / value array
   int32_t* sel;        // compaction output (ascending global indices)
-  int32_t* cnt;        // counts: [0] segments, [1] creation events, [2] LRU appends
+  int32_t* cnt;        // counts: [0] segments, [1] creation events, [2] LRU appends,
+                       // [5] refitting voxels, [6] the long ones of these
   int32_t* seg_start;  // segment -> first sorted position
   int32_t* seg_end;
   int32_t* seg_sess;
@@ -130,11 +130,9 @@ struct BatchBufs {
   int32_t* seg_ct;     // per segment: its candidate times (up to 7, ascending)
   int32_t* seg_nct;
   int32_t* seg_nbr;    // per segment: the six neighbour voxels (current incarnation, -1 none)
-  int4* hlist;         // refitting voxels as (vid, start, length, session), see k_seg_lenkeys
-  uint32_t* len_in;    // replay order: segments by descending length
-  uint32_t* len_out;
-  int32_t* ord_in;
-  int32_t* ord;
+  int4* hlist;         // refitting voxels as (vid, start, length, session), see k_create_init
+  uint32_t* seg_cls;   // per segment: how its voxel replays (replay_class)
+  int32_t* seg_old;    // per segment: its voxel before this scan's creations (-1: none)
   // per acting candidate (its index in spl, the first pre_cap of them): for
   // each record r (its six eligible neighbours, then itself) and each
   // neighbour j of r (j = 6: r itself), the voxel X there at the candidate's
@@ -157,7 +155,7 @@ struct BatchBufs {
   // per point in key-sorted order: its insertion point relative to its
   // voxel's centre (fp32, as the replays fold it in), its index in the scan
   // and its fp32 world covariance, (q.x, q.y, q.z, index bits, C0..C5, -, -),
-  // formed once by k_seg_heads
+  // formed once by k_seg_info
   float4* qc;
 };
 __host__ __device__ inline int64_t lv_cnt_base(int off, int s) { return (int64_t(2) * off >> 6) + s; }
@@ -373,13 +371,11 @@ __device__ inline void write_hot(const MapDev& m, int32_t vid, uint32_t flags) {
 
 #define VMP_GRID_LOOP(i, n) for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < (n); i += gridDim.x * blockDim.x)
 
-__global__ void k_begin_scan(const MapDev* maps, int nsess, uint64_t* clk) {
-  if (threadIdx.x != 0 || int(blockIdx.x) >= nsess) return;
-  if (blockIdx.x == 0) clk[1] = wall_clock64();
-  MapCounters* c = maps[blockIdx.x].ctr;
+// what a session's counters start a scan from
+__device__ inline void begin_scan(MapCounters* c) {
   c->tag += 1;
   c->fast = 0;
-  c->nseg = c->ncreate_ev = c->ncre = c->nevict = c->ncand = c->nlru = 0;
+  c->nseg = c->ncreate_ev = c->ncre = c->nevict = c->ncand = 0;
   c->refits = c->merge_calls = c->merge_evals = c->merges = c->dropped = 0;
   c->merge_windows = c->merge_requeued = c->merge_max_acting = 0;
 }
@@ -391,7 +387,7 @@ __global__ void k_fill_i32(int32_t* p, int32_t v, int n) {
 // eviction in this scan) takes its new voxels from the free-list top down,
 // then from the bump pointer.  Its counters advance as soon as its creation
 // count is known; the free-list top and bump pointer they started from stay
-// in S for k_create_fast.  Other sessions keep fast = 0 and go through
+// in S for k_create_init.  Other sessions keep fast = 0 and go through
 // k_create_evict.
 __device__ inline void create_fast_counters(const MapDev& m, SessInfo& S, int nc) {
   MapCounters* c = m.ctr;
@@ -414,7 +410,7 @@ __device__ inline void create_fast_counters(const MapDev& m, SessInfo& S, int nc
 }
 
 // per-session [lo, hi) of an ascending list of n global indices
-// which: 0 segments, 1 creation events, 2 LRU appends
+// which: 0 segments, 1 creation events
 __device__ inline void session_range(const MapDev* maps, SessInfo* si, int s, const int32_t* list, int n,
                                      int which) {
   auto lb = [&](int v) {
@@ -432,15 +428,11 @@ __device__ inline void session_range(const MapDev* maps, SessInfo* si, int s, co
     si[s].seg_lo = lo;
     si[s].seg_hi = hi;
     c->nseg = hi - lo;
-  } else if (which == 1) {
+  } else {
     si[s].cre_lo = lo;
     si[s].cre_hi = hi;
     c->ncreate_ev = hi - lo;
     create_fast_counters(maps[s], si[s], hi - lo);
-  } else {
-    si[s].lru_lo = lo;
-    si[s].lru_hi = hi;
-    c->nlru = hi - lo;
   }
 }
 __global__ void k_ranges(const MapDev* maps, SessInfo* si, int nsess, const int32_t* list, const int32_t* count,
@@ -456,7 +448,7 @@ __global__ void k_ranges(const MapDev* maps, SessInfo* si, int nsess, const int3
 // count) and its counter.  Sessions starting at or past nitems (empty
 // trailing sessions) start at the count.
 __device__ inline int32_t* range_lo(SessInfo& S, int which) {
-  return which == 0 ? &S.seg_lo : (which == 1 ? &S.cre_lo : &S.lru_lo);
+  return which == 0 ? &S.seg_lo : &S.cre_lo;
 }
 struct TailRanges {
   const MapDev* maps;
@@ -488,20 +480,26 @@ struct TailRanges {
       if (which == 0) {
         si[s].seg_hi = hi;
         c->nseg = hi - lo;
-      } else if (which == 1) {
+      } else {
         si[s].cre_hi = hi;
         c->ncreate_ev = hi - lo;
         create_fast_counters(maps[s], si[s], hi - lo);
-      } else {
-        si[s].lru_hi = hi;
-        c->nlru = hi - lo;
       }
     }
   }
 };
 
 // ------------------------------------------------------------------ K1 ----
-__global__ void k_ins_keys(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b) {
+// The map stage's first kernel: also starts every session's counters (this
+// kernel itself touches their error and used_entries only), the stage's
+// clock, and the counts and flags of the later passes.
+__global__ void k_ins_keys(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b, uint64_t* clk) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    clk[1] = wall_clock64();
+    b.cnt[5] = 0;
+    b.cnt[6] = 0;
+  }
+  VMP_GRID_LOOP(s, nsess) begin_scan(maps[s].ctr);
   VMP_UNIFORM_LOOP(g, valid, b.ntot) {
     int ins = 0;
     const int s = valid ? sess_of(si, nsess, g) : 0;
@@ -523,28 +521,94 @@ __global__ void k_ins_keys(const MapDev* maps, const SessInfo* si, int nsess, Ba
     else atomicOr(&m.ctr->error, 2);
     b.skey_in[g] = (uint64_t(s) << b.hbits) | uint64_t(uint32_t(e < 0 ? 0 : e));
     b.sval_in[g] = g;
+    b.flags[g] = 0;
     }
     wave_fetch_add(&maps[s].ctr->used_entries, ins);
   }
 }
 
 // ------------------------------------------------------------------ K3 ----
-// Segment heads of the key-sorted points, and the replays' input of every
-// point in that order (so a voxel's points are contiguous): the point
-// relative to its voxel's centre, its world covariance (calcBodyCov's z = 0
-// -> 0.001 applies to the covariance only, commons.cpp:20-23) and its index
-// in the scan, (q.x, q.y, q.z, index bits, C0..C5, -, -).  The transform and
-// the key are k_ins_keys' expressions, so the voxel is the one the point was
-// keyed to.
-__global__ void k_seg_heads(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) {  // refitting voxels, counted by k_seg_lenkeys
-    b.cnt[5] = 0;
-    b.cnt[6] = 0;
-  }
+// Segment heads: a key-sorted point whose key differs from the one before it
+// (a key holds its session, so sessions begin segments too).
+struct PredHead {
+  const uint64_t* key;
+  __device__ int32_t operator()(int i) const { return i == 0 || key[i] != key[i - 1] ? 1 : 0; }
+};
+__global__ void k_seg_heads(BatchBufs b) {
+  const PredHead head{b.skey_out};
+  VMP_GRID_LOOP(j, b.ntot) b.flags[j] = head(j);
+}
+
+// Whether this scan's walk of a voxel reaches a refit (updatePlane with
+// n >= update_size_thresh, voxel_map.cpp:42-95), from counts alone: an
+// uninitialised voxel refits when n reaches the threshold, an initialised
+// enabled one when newly_add does, before the walk stops at the freeze
+// point (n >= max_point_thresh); a build refits every voxel with enough
+// points once at the end.
+__device__ inline bool walk_refits(int n0, int newly0, uint32_t flags, int len, int upd, int mx, bool build) {
+  if (build) return n0 + len >= upd;
+  if ((flags & kInit) && !(flags & kEnable)) return false;
+  if (!(flags & kInit)) return len > upd - n0 - 1;
+  const int jr = upd - newly0 - 1;                  // walk index of the next refit
+  const int f = mx - n0 - 1 > 0 ? mx - n0 - 1 : 0;  // walk index of the freeze point
+  return jr < (len < f + 1 ? len : f + 1);
+}
+
+// How a voxel's points of this scan replay: 0 not at all (no voxel), class 1
+// frozen before the scan (counted only), 2 .. kClsHeavy - 1 the light walk of
+// class - 1 points (clamped), kClsHeavy and above the moment path, by length.
+constexpr uint32_t kClsHeavy = 64;
+constexpr int kClsBits = 6;
+__device__ inline uint32_t replay_class(const MapDev& m, int n0, int newly0, uint32_t flags, int len, bool build) {
+  if (walk_refits(n0, newly0, flags, len, m.upd_pt, m.max_pt, build))
+    return kClsHeavy + min(uint32_t(len), kClsHeavy - 1);
+  if (!build && (flags & kInit) && !(flags & kEnable)) return 1;
+  return 1 + min(uint32_t(len), kClsHeavy - 2);
+}
+
+// ------------------------------------------------------------------ K4 ----
+// Item j: segment j's record (the existing voxel's fields of this scan, its
+// replay class; a creation event at the first point of a segment without a
+// voxel), and the replays' input of sorted point j (so a voxel's points are
+// contiguous): the point relative to its voxel's centre, its world covariance
+// (calcBodyCov's z = 0 -> 0.001 applies to the covariance only,
+// commons.cpp:20-23) and its index in the scan, (q.x, q.y, q.z, index bits,
+// C0..C5, -, -).  The transform and the key are k_ins_keys' expressions, so
+// the voxel is the one the point was keyed to.
+__global__ void k_seg_info(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b) {
+  const int nseg = b.cnt[0];
   VMP_GRID_LOOP(j, b.ntot) {
+    if (j < nseg) {
+      const int q = j;
+      const int start = b.sel[q];
+      const int s = sess_of(si, nsess, start);
+      const SessInfo& S = si[s];
+      const int lim = S.off + S.n;
+      const int end = (q + 1 < nseg && b.sel[q + 1] < lim) ? b.sel[q + 1] : lim;
+      const MapDev m = maps[s];
+      const uint32_t e = uint32_t(b.skey_out[start] & ((uint64_t(1) << b.hbits) - 1));
+      const int first = b.sval_out[start] - S.off;
+      b.seg_start[q] = start;
+      b.seg_end[q] = end;
+      b.seg_sess[q] = s;
+      b.seg_entry[q] = int32_t(e);
+      const int32_t vid = m.table[e].vid;
+      b.seg_vid[q] = vid;
+      b.seg_old[q] = vid;
+      uint32_t cls = 0;
+      if (vid >= 0) {  // this scan's fields (three vector stores)
+        VoxState* st = m.vs + vid;
+        cls = replay_class(m, st->n, st->newly_add, st->flags, end - start, S.is_build != 0);
+        st_global2(&st->merge_pos, kNever, -2);
+        st_global4(&st->tag, m.ctr->tag, -1, kNever, -1);
+        st_global4(&st->prev_vid, -1, first, q, kNever);
+      } else {
+        b.flags[S.off + first] = q + 1;  // creation event at its first point (array cleared before)
+      }
+      b.seg_cls[q] = cls;
+    }
     const int s = sess_of(si, nsess, j);
     const SessInfo& S = si[s];
-    b.flags[j] = (j == S.off || b.skey_out[j] != b.skey_out[j - 1]) ? 1 : 0;
     const double vs64 = maps[s].vs64;
     const UpdParams& P = *S.prm;
     const int i = b.sval_out[j] - S.off;
@@ -562,35 +626,6 @@ __global__ void k_seg_heads(const MapDev* maps, const SessInfo* si, int nsess, B
     b.qc[3 * size_t(j)] = make_float4(qv[0], qv[1], qv[2], __int_as_float(i));
     b.qc[3 * size_t(j) + 1] = make_float4(C[0], C[1], C[2], C[3]);
     b.qc[3 * size_t(j) + 2] = make_float4(C[4], C[5], 0.0f, 0.0f);
-  }
-}
-
-// ------------------------------------------------------------------ K4 ----
-__global__ void k_seg_info(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b) {
-  const int nseg = b.cnt[0];
-  VMP_GRID_LOOP(q, nseg) {
-    const int start = b.sel[q];
-    const int s = sess_of(si, nsess, start);
-    const SessInfo& S = si[s];
-    const int lim = S.off + S.n;
-    const int end = (q + 1 < nseg && b.sel[q + 1] < lim) ? b.sel[q + 1] : lim;
-    const MapDev m = maps[s];
-    const uint32_t e = uint32_t(b.skey_out[start] & ((uint64_t(1) << b.hbits) - 1));
-    const int first = b.sval_out[start] - S.off;
-    b.seg_start[q] = start;
-    b.seg_end[q] = end;
-    b.seg_sess[q] = s;
-    b.seg_entry[q] = int32_t(e);
-    const int32_t vid = m.table[e].vid;
-    b.seg_vid[q] = vid;
-    if (vid >= 0) {  // this scan's fields (three vector stores)
-      VoxState* st = m.vs + vid;
-      st_global2(&st->merge_pos, kNever, -2);
-      st_global4(&st->tag, m.ctr->tag, -1, kNever, -1);
-      st_global4(&st->prev_vid, -1, first, q, kNever);
-    } else {
-      b.flags[S.off + first] = q + 1;  // creation event at its first point (array cleared before)
-    }
   }
 }
 
@@ -619,21 +654,6 @@ struct OutCre {
 };
 
 // ------------------------------------------------------------------ K5 ----
-// Parallel creation for sessions whose LRU cannot overflow in this scan
-// (fast, set with their counters where the creation events were counted).
-__global__ void k_create_fast(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b) {
-  const int nc = b.cnt[1];
-  VMP_GRID_LOOP(r, nc) {
-    const int s = sess_of(si, nsess, b.sel[r]);
-    const MapDev m = maps[s];
-    if (!m.ctr->fast) continue;
-    const int rl = r - si[s].cre_lo;
-    const int ftop = si[s].ftop0, bump = si[s].bump0;
-    const int32_t vid = rl < ftop ? m.freelist[ftop - 1 - rl] : bump + (rl - ftop);
-    b.co[si[s].off + rl] = make_int4(vid, b.cre_seg[r], b.cre_t[r], -1);
-  }
-}
-
 // Chunks of the ring that k_ring_live compacts for a session: enough for the
 // creations of most scans at a few stale entries per victim, within the
 // session's two entries per point; k_create_evict reads the ring itself
@@ -995,45 +1015,124 @@ __global__ void __launch_bounds__(kCeThreads) k_create_evict(const MapDev* maps,
   }
 }
 
-// Initialise created voxels and point their hash slots at them.
-__global__ void k_create_init(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b) {
-  VMP_GRID_LOOP(p, b.ntot) {
-    const int s = sess_of(si, nsess, p);
-    const MapDev m = maps[s];
-    const int r = p - si[s].off;
-    const int ncre = m.ctr->ncre;
-    if (r >= ncre) continue;
-    const int4 co = b.co[p];
-    const int32_t vid = co.x;
-    const int q = co.y;
-    if (vid < 0 || vid >= m.pool || q < 0) continue;  // error already flagged
-    const int32_t e = b.seg_entry[q];
-    VoxState st;
-    st.key = m.table[e].key;
-    st.group_id = m.ctr->group_counter - uint64_t(ncre) + uint64_t(r);
-    st.stamp = 0;
-    st.n = 0;
-    st.newly_add = 0;
-    st.flags = kEnable | kAlive;
-    st.pad = 0;
-    st.tag = m.ctr->tag;
-    st.create_t = co.z;
-    st.evict_t = kNever;
-    st.freeze_t = -1;
-    st.prev_vid = co.w;
-    st.first_t = co.z;
-    st.seg = q;
-    st.merge_pos = kNever;
-    st.dirty_t = -2;
-    st.taint_t = kNever;
-    m.vs[vid] = st;
-    // the plane record and the moments are not cleared here: the voxel has
-    // points in this scan, and the replay starts a voxel with n = 0 from zero
-    VoxHot h{};
-    h.flags = kEnable | kAlive;
-    m.hot[vid] = h;
-    m.table[e].vid = vid;
-    b.seg_vid[q] = vid;
+// Initialise created voxels and point their hash slots at them; a session
+// whose LRU cannot overflow in this scan (fast, set with its counters where
+// the creation events were counted) takes its voxel ids here.  Then every
+// segment has its voxel and its replay class, and the refitting voxels are
+// listed as (vid, start, length, session) records: all of them from the front
+// of hlist (cnt[5] counts them) and, from its back, those with at least
+// long_seg points (cnt[6]; 0 lists none).  The two parts cannot meet: a long
+// segment holds two points or more.  A segment is listed by the thread of its
+// creation, or by its own if its voxel was there before and stays; the two
+// read nothing that the other writes (seg_old and the evict time).
+__global__ void __launch_bounds__(kMapThreads) k_create_init(const MapDev* maps, const SessInfo* si, int nsess,
+                                                             BatchBufs b, int long_seg) {
+  constexpr int kW = kMapThreads / 64;
+  __shared__ int woff[2][kW];
+  __shared__ int bbase[2];
+  const int nseg = b.cnt[0];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  VMP_UNIFORM_LOOP(p, valid, b.ntot) {
+    int4 rec[2] = {make_int4(-1, 0, 0, 0), make_int4(-1, 0, 0, 0)};
+    if (valid) {
+      const int s = sess_of(si, nsess, p);
+      const SessInfo& S = si[s];
+      const MapDev m = maps[s];
+      const int r = p - S.off;
+      const int ncre = m.ctr->ncre;
+      if (r < ncre) {
+        int4 co;
+        if (m.ctr->fast) {
+          const int k = S.cre_lo + r, ftop = S.ftop0;
+          co = make_int4(r < ftop ? m.freelist[ftop - 1 - r] : S.bump0 + (r - ftop), b.cre_seg[k], b.cre_t[k], -1);
+        } else {
+          co = b.co[p];
+        }
+        const int32_t vid = co.x;
+        const int q = co.y;
+        if (vid >= 0 && vid < m.pool && q >= 0) {  // else the error is already flagged
+          const int32_t e = b.seg_entry[q];
+          const int start = b.seg_start[q], len = b.seg_end[q] - start;
+          VoxState st;
+          st.key = m.table[e].key;
+          st.group_id = m.ctr->group_counter - uint64_t(ncre) + uint64_t(r);
+          st.stamp = 0;
+          st.n = 0;
+          st.newly_add = 0;
+          st.flags = kEnable | kAlive;
+          st.pad = 0;
+          st.tag = m.ctr->tag;
+          st.create_t = co.z;
+          st.evict_t = kNever;
+          st.freeze_t = -1;
+          st.prev_vid = co.w;
+          st.first_t = co.z;
+          st.seg = q;
+          st.merge_pos = kNever;
+          st.dirty_t = -2;
+          st.taint_t = kNever;
+          m.vs[vid] = st;
+          // the plane record and the moments are not cleared here: the voxel
+          // has points in this scan, and the replay starts a voxel with n = 0
+          // from zero
+          VoxHot h{};
+          h.flags = kEnable | kAlive;
+          m.hot[vid] = h;
+          m.table[e].vid = vid;
+          b.seg_vid[q] = vid;
+          const uint32_t cls = replay_class(m, 0, 0, kEnable | kAlive, len, S.is_build != 0);
+          b.seg_cls[q] = cls;
+          if (cls >= kClsHeavy) rec[0] = make_int4(vid, start, len, s);
+        }
+      }
+      // the merge stage's per-point slots start empty (k_candidates fills
+      // them; k_create_evict kept its touched entries in cand_in before)
+      b.cand_in[p] = ~0ull;
+      b.cand_spec[p] = 0;
+      int2* tn = reinterpret_cast<int2*>(b.tnbr + size_t(p) * 6);
+      tn[0] = make_int2(0, 0);
+      tn[1] = make_int2(0, 0);
+      tn[2] = make_int2(0, 0);
+      if (p < nseg) {
+        const int32_t vid = b.seg_old[p];
+        if (vid >= 0) {
+          const int qs = b.seg_sess[p];
+          const MapDev qm = maps[qs];
+          const bool stays = qm.ctr->fast || qm.vs[vid].evict_t == kNever;
+          if (stays && b.seg_cls[p] >= kClsHeavy)
+            rec[1] = make_int4(vid, b.seg_start[p], b.seg_end[p] - b.seg_start[p], qs);
+        }
+      }
+    }
+    // the block's share of each list, wave by wave
+    const bool hv[2] = {rec[0].x >= 0, rec[1].x >= 0};
+    const bool lg[2] = {hv[0] && long_seg > 0 && rec[0].z >= long_seg, hv[1] && long_seg > 0 && rec[1].z >= long_seg};
+    const uint64_t bh[2] = {__ballot(hv[0]), __ballot(hv[1])}, bl[2] = {__ballot(lg[0]), __ballot(lg[1])};
+    if (lane == 0) {
+      woff[0][wv] = __popcll(bh[0]) + __popcll(bh[1]);
+      woff[1][wv] = __popcll(bl[0]) + __popcll(bl[1]);
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      int run = 0;
+      for (int w = 0; w < kW; ++w) {
+        const int c = woff[threadIdx.x][w];
+        woff[threadIdx.x][w] = run;
+        run += c;
+      }
+      bbase[threadIdx.x] = run ? atomicAdd(&b.cnt[5 + threadIdx.x], run) : 0;
+    }
+    __syncthreads();
+    const uint64_t below = bits_below(lane);
+    int h0 = bbase[0] + woff[0][wv], l0 = bbase[1] + woff[1][wv];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if (hv[k]) b.hlist[h0 + __popcll(bh[k] & below)] = rec[k];
+      if (lg[k]) b.hlist[b.ntot - 1 - (l0 + __popcll(bl[k] & below))] = rec[k];
+      h0 += __popcll(bh[k]);
+      l0 += __popcll(bl[k]);
+    }
+    __syncthreads();
   }
 }
 
@@ -1202,21 +1301,6 @@ __device__ inline void refit(const MapDev& m, Moments& M, int n, uint32_t& flags
   refit_apply(refit_eval(m, M, n, center), flags, pl);
 }
 
-// Whether this scan's walk of a voxel reaches a refit (updatePlane with
-// n >= update_size_thresh, voxel_map.cpp:42-95), from counts alone: an
-// uninitialised voxel refits when n reaches the threshold, an initialised
-// enabled one when newly_add does, before the walk stops at the freeze
-// point (n >= max_point_thresh); a build refits every voxel with enough
-// points once at the end.
-__device__ inline bool walk_refits(int n0, int newly0, uint32_t flags, int len, int upd, int mx, bool build) {
-  if (build) return n0 + len >= upd;
-  if ((flags & kInit) && !(flags & kEnable)) return false;
-  if (!(flags & kInit)) return len > upd - n0 - 1;
-  const int jr = upd - newly0 - 1;                  // walk index of the next refit
-  const int f = mx - n0 - 1 > 0 ? mx - n0 - 1 : 0;  // walk index of the freeze point
-  return jr < (len < f + 1 ? len : f + 1);
-}
-
 // The whole walk of a voxel in this scan from counts alone (the state
 // machine of the lane walk in k_replay_heavy, voxel_map.cpp:42-95): the
 // walk index of the refit that initialises the voxel, then of the first
@@ -1263,79 +1347,7 @@ __device__ inline WalkPlan walk_plan(int n0, int newly0, uint32_t flags, int len
   return p;
 }
 
-// Replay order: the voxels that refit first (the moment path), then the
-// rest, each part by descending segment length so waves walk segments of
-// similar length; slots past the segment count sort last.  Lengths are
-// clamped below 2^lbits - 1; the class is bit lbits.  Also lists the
-// refitting voxels as (vid, start, length, session) records for the
-// per-wave replay: all of them from the front of hlist (cnt[5] counts them)
-// and, from its back, those with at least long_seg points (cnt[6]; 0 lists
-// none).  The two parts cannot meet: a long segment holds two points or
-// more.  Both counts are cleared by k_seg_heads.
-__global__ void __launch_bounds__(kMapThreads) k_seg_lenkeys(const MapDev* maps, const SessInfo* si, BatchBufs b,
-                                                             int lbits, int long_seg) {
-  constexpr int kW = kMapThreads / 64;
-  __shared__ int woff[2][kW];
-  __shared__ int bbase[2];
-  const int nseg = b.cnt[0];
-  const uint32_t top = uint32_t((uint64_t(1) << lbits) - 1);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  VMP_UNIFORM_LOOP(q, valid, b.ntot) {
-    uint32_t key = (1u << lbits) | top;
-    int heavy = 0, lng = 0, start = 0, len = 0, s = 0;
-    int32_t vid = -1;
-    if (valid && q < nseg) {
-      start = b.seg_start[q];
-      len = b.seg_end[q] - start;
-      vid = b.seg_vid[q];
-      if (vid >= 0) {
-        s = b.seg_sess[q];
-        const MapDev m = maps[s];
-        const VoxState& st = m.vs[vid];
-        heavy = walk_refits(st.n, st.newly_add, st.flags, len, m.upd_pt, m.max_pt, si[s].is_build != 0) ? 1 : 0;
-      }
-      lng = heavy & int(long_seg > 0 && len >= long_seg);
-      key = (uint32_t(1 - heavy) << lbits) | (top - min(uint32_t(len), top - 1));
-    }
-    if (valid) {
-      b.len_in[q] = key;
-      b.ord_in[q] = q;
-      // the merge stage's per-point slots start empty (k_candidates fills them)
-      b.cand_in[q] = ~0ull;
-      b.cand_spec[q] = 0;
-      int2* tn = reinterpret_cast<int2*>(b.tnbr + size_t(q) * 6);
-      tn[0] = make_int2(0, 0);
-      tn[1] = make_int2(0, 0);
-      tn[2] = make_int2(0, 0);
-    }
-    const uint64_t bh = __ballot(heavy), bl = __ballot(lng);
-    if (lane == 0) {
-      woff[0][wv] = __popcll(bh);
-      woff[1][wv] = __popcll(bl);
-    }
-    __syncthreads();
-    if (threadIdx.x < 2) {  // the block's share of each list, wave by wave
-      int run = 0;
-      for (int w = 0; w < kW; ++w) {
-        const int c = woff[threadIdx.x][w];
-        woff[threadIdx.x][w] = run;
-        run += c;
-      }
-      bbase[threadIdx.x] = run ? atomicAdd(&b.cnt[5 + threadIdx.x], run) : 0;
-    }
-    __syncthreads();
-    if (heavy) {
-      const uint64_t below = (uint64_t(1) << lane) - 1;
-      const int4 rec = make_int4(vid, start, len, s);
-      b.hlist[bbase[0] + woff[0][wv] + __popcll(bh & below)] = rec;
-      if (lng) b.hlist[b.ntot - 1 - (bbase[1] + woff[1][wv] + __popcll(bl & below))] = rec;
-    }
-    __syncthreads();
-  }
-}
-
-// The voxels that refit in this scan (the first cnt[5] of the replay
-// order) replay their pending points and then their points of this scan in
+// The voxels that refit in this scan replay their pending points and then their points of this scan in
 // order through the pushPoint state machine, with FP64 moments and refits
 // from them, in one of two forms that give the same bits:
 //  - one wave per voxel (heavy_wave): lane c keeps moment c (lanes 0-4 also
@@ -1381,11 +1393,9 @@ __device__ inline void write_hot_pl(const MapDev& m, int32_t vid, uint32_t flags
   m.hot[vid] = h;
 }
 
-__device__ inline void heavy_lane(const MapDev& m, const SessInfo& S, const BatchBufs& b, int q, int32_t vid,
+__device__ inline void heavy_lane(const MapDev& m, const SessInfo& S, const BatchBufs& b, int32_t vid, int start, int end,
                                   int& refits, int& calls, int& dropped) {
   if (vid >= 0) {
-    const int start = b.seg_start[q];
-    const int end = b.seg_end[q];
     VoxState st = m.vs[vid];
     double* pl = m.plane + size_t(vid) * kPlaneD;
     double* mo = m.mom + size_t(vid) * kMomD;
@@ -1667,12 +1677,44 @@ __device__ inline void heavy_wave(const MapDev& m, bool build, const BatchBufs& 
   }
 }
 
+// Orders a block's items by class, descending (n items per class counted in
+// LDS, then placed by a scan), so that the lanes of a wave walk voxels with
+// similar numbers of points; items of class 0 come last.  Returns the item
+// that this thread takes.  An order over all segments took a histogram and a
+// radix pass, 14 us.  The order decides nothing else, every voxel replays on
+// its own.
+struct SortLds {
+  int cnt[kClsHeavy];
+  int item[kMapThreads];
+};
+__device__ inline int block_order(uint32_t cls, SortLds& L) {
+  const int tid = threadIdx.x;
+  __syncthreads();
+  if (tid < int(kClsHeavy)) L.cnt[tid] = 0;
+  __syncthreads();
+  const int k = int(kClsHeavy - 1 - cls);
+  const int r = atomicAdd(&L.cnt[k], 1);
+  __syncthreads();
+  if (tid < 64) {
+    const int c = L.cnt[tid];
+    int incl = c;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int u = __shfl_up(incl, o, 64);
+      if (tid >= o) incl += u;
+    }
+    L.cnt[tid] = incl - c;
+  }
+  __syncthreads();
+  L.item[L.cnt[k] + r] = tid;
+  __syncthreads();
+  return L.item[tid];
+}
+
 // One wave per voxel of hlist: every refitting voxel when there are at most
 // wave_max of them, else the long ones (cnt[6], at hlist's back).  A
 // one-session step reads its map's record without waiting for the list.
-__global__ void __launch_bounds__(kMapThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_replay_heavy_wave(const MapDev* maps, const SessInfo* si, BatchBufs b, int wave_max) {
-  __shared__ HeavyLds lds[kMapThreads / 64];
+__device__ inline void replay_waves(const MapDev* maps, const SessInfo* si, const BatchBufs& b, int wave_max,
+                                    int block, int nblocks, HeavyLds* lds) {
   constexpr int kWpb = kMapThreads / 64;
   const int nh = b.cnt[5];
   const bool all = nh <= wave_max;
@@ -1680,7 +1722,7 @@ k_replay_heavy_wave(const MapDev* maps, const SessInfo* si, BatchBufs b, int wav
   const int wv = threadIdx.x >> 6;
   const MapDev m0 = maps[0];
   const bool build0 = si[0].is_build != 0;
-  for (int u = blockIdx.x * kWpb + wv; u < nw; u += gridDim.x * kWpb) {
+  for (int u = block * kWpb + wv; u < nw; u += nblocks * kWpb) {
     int refits = 0, calls = 0, dropped = 0;
     const int4 r = b.hlist[all ? u : b.ntot - 1 - u];
     MapDev m;
@@ -1699,37 +1741,48 @@ k_replay_heavy_wave(const MapDev* maps, const SessInfo* si, BatchBufs b, int wav
   }
 }
 
-// The rest of the refitting voxels, one per lane.
-__global__ void __launch_bounds__(kMapThreads) k_replay_heavy(const MapDev* maps, const SessInfo* si, BatchBufs b,
-                                                              int wave_max) {
+// The rest of the refitting voxels, one per lane (a kernel of its own: the
+// walk takes all the registers of a wave per SIMD, and together with
+// heavy_wave it spilled).  Left out where a scan has no more than wave_max
+// points.
+__global__ void __launch_bounds__(kMapThreads)
+k_replay_heavy(const MapDev* maps, const SessInfo* si, BatchBufs b, int wave_max, int long_seg) {
+  __shared__ SortLds sort;
   const int nh = b.cnt[5];
-  const int nw = nh <= wave_max ? nh : b.cnt[6];
-  VMP_UNIFORM_LOOP(i, valid, nh - nw) {
+  if (nh <= wave_max) return;
+  for (int i0 = blockIdx.x * kMapThreads; i0 < nh; i0 += gridDim.x * kMapThreads) {
+    const int i = i0 + int(threadIdx.x);
+    int len = i < nh ? b.hlist[i].z : 0;
+    if (long_seg > 0 && len >= long_seg) len = 0;  // replayed by a wave
+    const int j = i0 + block_order(min(uint32_t(len), kClsHeavy - 1), sort);
+    int4 r = j < nh ? b.hlist[j] : make_int4(-1, 0, 0, 0);
+    if (long_seg > 0 && r.z >= long_seg) r.x = -1;
     int refits = 0, calls = 0, dropped = 0;
-    const int q = valid ? b.ord[nw + i] : 0;
-    const int s = valid ? b.seg_sess[q] : 0;
-    heavy_lane(maps[s], si[s], b, q, valid ? b.seg_vid[q] : -1, refits, calls, dropped);
-    const MapDev& m = maps[s];
+    const MapDev& m = maps[r.w];
+    heavy_lane(m, si[r.w], b, r.x, r.y, r.y + r.z, refits, calls, dropped);
     wave_fetch_add(&m.ctr->refits, refits);
     wave_fetch_add(&m.ctr->merge_calls, calls);
     wave_fetch_add(&m.ctr->dropped, dropped);
   }
 }
 
-// The other voxels (from cnt[5] on): frozen ones count their points as
-// merge() calls or drops; the rest add points without reaching a refit, so
-// only the count, the running mean and the freeze state change, and each
-// point (relative to the voxel centre, with its world cov) joins the pending
-// list that the voxel's next refit folds into the moments.
-__global__ void __launch_bounds__(kMapThreads) k_replay_light(const MapDev* maps, const SessInfo* si, BatchBufs b) {
-  const int nseg = b.cnt[0], nh = b.cnt[5];
+// The other voxels: frozen ones count their points as merge() calls or drops;
+// the rest add points without reaching a refit, so only the count, the
+// running mean and the freeze state change, and each point (relative to the
+// voxel centre, with its world cov) joins the pending list that the voxel's
+// next refit folds into the moments.
+__device__ inline void replay_light(const MapDev* maps, const SessInfo* si, const BatchBufs& b, int block,
+                                    int nblocks, SortLds& sort) {
+  const int nseg = b.cnt[0];
   // a one-session step reads its map's record once, before the voxels
   const MapDev m0 = maps[0];
   const int build0 = si[0].is_build;
-  VMP_UNIFORM_LOOP(qi, valid, nseg - nh) {
+  for (int q0 = block * kMapThreads; q0 < nseg; q0 += nblocks * kMapThreads) {
     int calls = 0, dropped = 0;
-    const int q = valid ? b.ord[nh + qi] : 0;
-    const int32_t vid = valid ? b.seg_vid[q] : -1;
+    const uint32_t cls = q0 + int(threadIdx.x) < nseg ? b.seg_cls[q0 + threadIdx.x] : 0;
+    const int q = min(q0 + block_order(cls >= kClsHeavy ? 0u : cls, sort), nseg - 1);
+    const bool mine = q0 + sort.item[threadIdx.x] < nseg && b.seg_cls[q] < kClsHeavy;
+    const int32_t vid = mine ? b.seg_vid[q] : -1;
     const int start = b.seg_start[q], end = b.seg_end[q];
     MapDev m;
     int s, is_build;
@@ -1738,7 +1791,7 @@ __global__ void __launch_bounds__(kMapThreads) k_replay_light(const MapDev* maps
       m = m0;
       is_build = build0;
     } else {
-      s = valid ? b.seg_sess[q] : 0;
+      s = mine ? b.seg_sess[q] : 0;
       m = maps[s];
       is_build = si[s].is_build;
     }
@@ -1844,6 +1897,19 @@ __global__ void __launch_bounds__(kMapThreads) k_replay_light(const MapDev* maps
   }
 }
 
+// Both in one launch: blocks below hblocks take refitting voxels, the others
+// those that do not refit, so the light walks fill in where the long chains of the
+// refits leave the card idle.
+__global__ void __launch_bounds__(kMapThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_replay(const MapDev* maps, const SessInfo* si, BatchBufs b, int wave_max, int hblocks) {
+  __shared__ HeavyLds lds[kMapThreads / 64];
+  __shared__ SortLds sort;
+  if (int(blockIdx.x) < hblocks)
+    replay_waves(maps, si, b, wave_max, blockIdx.x, hblocks, lds);
+  else
+    replay_light(maps, si, b, int(blockIdx.x) - hblocks, int(gridDim.x) - hblocks, sort);
+}
+
 }  // namespace vmp
 
 #include "vmp_merge.hpp"
@@ -1851,15 +1917,21 @@ __global__ void __launch_bounds__(kMapThreads) k_replay_light(const MapDev* maps
 namespace vmp {
 
 // ------------------------------------------------------------------ K9 ----
-__global__ void k_finalize_segs(const MapDev* maps, const SessInfo* si, BatchBufs b) {
+// The scan's last fields of every touched voxel and the marks of their LRU
+// appends, then (sessions that evict) the evicted voxels' slots: hash
+// tombstones and the free list.
+__global__ void k_finalize(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b, int evict) {
   const int nseg = b.cnt[0];
   VMP_GRID_LOOP(q, nseg) {
     const int32_t vid = b.seg_vid[q];
-    if (vid < 0) continue;
     const int s = b.seg_sess[q];
     const MapDev m = maps[s];
-    VoxState& st = m.vs[vid];
     const int last_t = b.sval_out[b.seg_end[q] - 1] - si[s].off;
+    // LRU append marker (array cleared before); a segment left without a
+    // voxel by an error appends an entry that no voxel's stamp can match
+    b.flags[si[s].off + last_t] = vid < 0 ? -1 : vid + 1;
+    if (vid < 0) continue;
+    VoxState& st = m.vs[vid];
     const bool calls = st.merge_pos != kNever;
     const bool frozen_plane = (st.flags & kPlane) && !(st.flags & kEnable) && (st.flags & kInit);
     // a dirtying event is resolved by a later (evaluated) merge() call
@@ -1867,11 +1939,8 @@ __global__ void k_finalize_segs(const MapDev* maps, const SessInfo* si, BatchBuf
     if (dirty) st.flags |= kDirty;
     else st.flags &= ~kDirty;
     st.stamp = uint64_t(m.ctr->point_base + last_t);
-    b.flags[si[s].off + last_t] = vid + 1;  // LRU append marker (array cleared before)
   }
-}
-
-__global__ void k_evict_finalize(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b) {
+  if (!evict) return;
   VMP_GRID_LOOP(p, b.ntot) {
     const int s = sess_of(si, nsess, p);
     const MapDev m = maps[s];
@@ -1891,18 +1960,23 @@ __global__ void k_evict_finalize(const MapDev* maps, const SessInfo* si, int nse
   }
 }
 
-__global__ void k_lru_append(const MapDev* maps, const SessInfo* si, int nsess, BatchBufs b) {
-  const int nsel = b.cnt[2];
-  VMP_GRID_LOOP(r, nsel) {
-    const int g = b.sel[r];
+// LRU queue append, as the output of the compaction of the marks: one entry
+// per segment, so a session's first is its first segment's number.
+struct OutLru {
+  const MapDev* maps;
+  const SessInfo* si;
+  int nsess;
+  __device__ void operator()(int r, int g, int32_t v) const {
     const int s = sess_of(si, nsess, g);
-    const MapDev m = maps[s];
-    const int t = g - si[s].off;
-    const int32_t vid = b.flags[g] - 1;
-    const int64_t ph = (m.ctr->ring_tail + (r - si[s].lru_lo)) % m.qcap;
-    m.ring_vid[ph] = vid;
-    m.ring_stamp[ph] = uint64_t(m.ctr->point_base + t);
+    const MapDev& m = maps[s];
+    const int64_t ph = (m.ctr->ring_tail + (r - si[s].seg_lo)) % m.qcap;
+    m.ring_vid[ph] = v < 0 ? 0 : v - 1;
+    m.ring_stamp[ph] = v < 0 ? ~uint64_t(0) : uint64_t(m.ctr->point_base + (g - si[s].off));
   }
+};
+__global__ void k_lru_append(OutLru out, BatchBufs b) {
+  const int nsel = b.cnt[2];
+  VMP_GRID_LOOP(r, nsel) out(r, b.sel[r], b.flags[b.sel[r]]);
 }
 
 // start of each session's candidates in the sorted candidate list, and
