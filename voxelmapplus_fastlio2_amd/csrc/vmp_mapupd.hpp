@@ -119,17 +119,12 @@ struct BatchBufs {
   uint64_t* cand_in;   // merge candidates, see cand_key(); per session at its offset
   uint64_t* cand_out;  // sorted: session-major, then point time, then voxel
   int32_t* cand_nbr;   // per sorted candidate: 6 eligible neighbour ids at its time
-  // per point (session offset + point time): the 6 eligible neighbour ids of
-  // the merge() call at that time, + 2 (0: not looked up yet in this scan);
-  // they cannot change during the merge replay, so a call that returns to
-  // the pool reads them back instead of repeating the lookups
-  int32_t* tnbr;
   int32_t* cand_spec;  // per sorted candidate: 1 if it merges on the pre-replay state
   int32_t* cand_start; // per session: first sorted candidate
   int32_t* spl;        // positions of candidates with cand_spec = 1, ascending
   int32_t* seg_ct;     // per segment: its candidate times (up to 7, ascending)
   int32_t* seg_nct;
-  int32_t* seg_nbr;    // per segment: the six neighbour voxels (current incarnation, -1 none)
+  int2* seg_nbr;       // per segment: the six neighbour voxels, see nbr_eligible()
   int4* hlist;         // refitting voxels as (vid, start, length, session), see k_create_init
   uint32_t* seg_cls;   // per segment: how its voxel replays (replay_class)
   int32_t* seg_old;    // per segment: its voxel before this scan's creations (-1: none)
@@ -1089,10 +1084,6 @@ __global__ void __launch_bounds__(kMapThreads) k_create_init(const MapDev* maps,
       // them; k_create_evict kept its touched entries in cand_in before)
       b.cand_in[p] = ~0ull;
       b.cand_spec[p] = 0;
-      int2* tn = reinterpret_cast<int2*>(b.tnbr + size_t(p) * 6);
-      tn[0] = make_int2(0, 0);
-      tn[1] = make_int2(0, 0);
-      tn[2] = make_int2(0, 0);
       if (p < nseg) {
         const int32_t vid = b.seg_old[p];
         if (vid >= 0) {

@@ -17,7 +17,7 @@
 //                  any merge of this scan: its eligible neighbours at its
 //                  time (existence, incarnation, frozen-ness and plane-ness
 //                  do not depend on merges) and whether it would merge
-//   k_merge_replay one wave per session walks, in point order, the
+//   k_merge_replay one workgroup per session walks, in point order, the
 //                  candidates that would merge plus the calls a real merge
 //                  makes necessary: for every voxel whose closed
 //                  neighbourhood a merge changed ("tainted"), its next call
@@ -42,9 +42,8 @@ __device__ inline int32_t vid_at(const MapDev& m, int32_t vid, int tag, int t) {
 // The segment's point times ascend; the search narrows the range by sixteen
 // independent samples per step (one memory round trip each) instead of a
 // binary search's chain of dependent loads.
-__device__ inline int first_call_after(const BatchBufs& b, int q, int merge_pos, int t, int off) {
-  const int end = b.seg_end[q];
-  int lo = b.seg_start[q] + merge_pos, hi = end;  // answer in [lo, hi], hi = none
+__device__ inline int first_call_in(const BatchBufs& b, int start, int end, int t, int off) {
+  int lo = start, hi = end;  // answer in [lo, hi], hi = none
   const int tg = t + off;                          // compare global indices
   while (hi - lo > 16) {
     const int step = (hi - lo + 15) >> 4;
@@ -68,6 +67,10 @@ __device__ inline int first_call_after(const BatchBufs& b, int q, int merge_pos,
   return kNever;
 }
 
+__device__ inline int first_call_after(const BatchBufs& b, int q, int merge_pos, int t, int off) {
+  return first_call_in(b, b.seg_start[q] + merge_pos, b.seg_end[q], t, off);
+}
+
 __device__ inline int32_t lookup_vid(const MapDev& m, uint64_t key) {
   const int32_t e = hash_find_slot(m.table, m.hmask, key);
   return e < 0 ? -1 : m.table[e].vid;
@@ -81,6 +84,17 @@ __device__ inline int32_t eligible_at(const MapDev& m, int32_t cur, int tag, int
   const VoxState& ns = m.vs[nv];
   const bool frozen = !(ns.flags & kEnable) && !(ns.tag == tag && ns.freeze_t > t);
   return (frozen && (ns.flags & kPlane) && (ns.flags & kInit)) ? nv : -1;
+}
+// A face neighbour of a voxel of this scan, as k_candidates leaves it in
+// seg_nbr: (its current incarnation, -1 none; the point time from which it is
+// eligible, kNever if at no time).  Nothing here depends on merges.  A
+// neighbour that was evicted or that came back in this scan carries kNbrSlow:
+// its state at a time is read from the records.
+constexpr int32_t kNbrSlow = -2;
+__device__ inline int32_t nbr_eligible(const MapDev& m, int2 nb, int tag, int t) {
+  if (nb.x < 0) return -1;
+  if (nb.y == kNbrSlow) return eligible_at(m, nb.x, tag, t);
+  return t >= nb.y ? nb.x : -1;
 }
 __device__ inline int32_t nbr_at(const MapDev& m, uint64_t vkey, int j, int tag, int t) {
   if (!key_neighbour_ok(vkey, j)) return -1;
@@ -204,7 +218,7 @@ __global__ void k_candidates(const MapDev* maps, const SessInfo* si, BatchBufs b
     if (valid) {
       b.seg_nct[q] = 0;
       if (vid < 0)
-        for (int j = 0; j < 6; ++j) b.seg_nbr[q * 6 + j] = -1;
+        for (int j = 0; j < 6; ++j) b.seg_nbr[q * 6 + j] = make_int2(-1, kNever);
     }
     if (vid >= 0) {
       const int tag = c->tag, off = si[s].off;
@@ -224,7 +238,7 @@ __global__ void k_candidates(const MapDev* maps, const SessInfo* si, BatchBufs b
       // the six neighbours' entries, then their records, six loads at a time
       int32_t nvs[6];
       lookup_nbrs6(m, st.key, nvs);
-      int ntag[6], nfrz[6];
+      int ntag[6], nfrz[6], ncre[6], nevt[6], nprv[6];
       uint32_t nflg[6];
 #pragma unroll
       for (int j = 0; j < 6; ++j) {
@@ -232,10 +246,17 @@ __global__ void k_candidates(const MapDev* maps, const SessInfo* si, BatchBufs b
         ntag[j] = nbs.tag;
         nfrz[j] = nbs.freeze_t;
         nflg[j] = nbs.flags;
+        ncre[j] = nbs.create_t;
+        nevt[j] = nbs.evict_t;
+        nprv[j] = nbs.prev_vid;
       }
       for (int j = 0; j < 6; ++j) {
         const int32_t nv = nvs[j];
-        b.seg_nbr[q * 6 + j] = nv;
+        const bool cur = ntag[j] == tag;
+        const bool frozen_plane = !(nflg[j] & kEnable) && (nflg[j] & kPlane) && (nflg[j] & kInit);
+        int from = frozen_plane ? (cur ? max(ncre[j], nfrz[j]) : -1) : kNever;
+        if (cur && (nevt[j] != kNever || nprv[j] >= 0)) from = kNbrSlow;
+        b.seg_nbr[q * 6 + j] = make_int2(nv, from);
         if (nv < 0) continue;
         if (ntag[j] != tag || nfrz[j] < 0 || !(nflg[j] & kPlane)) continue;
         if (nfrz[j] > dirty) dirty = nfrz[j];
@@ -304,14 +325,18 @@ __global__ void k_spec_eval(const MapDev* maps, BatchBufs b) {
     // the six neighbours (cached ids of a voxel touched in this scan, else
     // looked up), their eligibility at t, then the gate, each step with the
     // six neighbours' loads together
-    int32_t nc[6], nv[6];
+    int32_t nv[6];
     if (cached) {
+      int2 nb[6];
 #pragma unroll
-      for (int j = 0; j < 6; ++j) nc[j] = b.seg_nbr[vst.seg * 6 + j];
+      for (int j = 0; j < 6; ++j) nb[j] = b.seg_nbr[vst.seg * 6 + j];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) nv[j] = nbr_eligible(m, nb[j], tag, t);
     } else {
+      int32_t nc[6];
       lookup_nbrs6(m, vst.key, nc);
+      eligible6(m, nc, tag, t, nv);
     }
-    eligible6(m, nc, tag, t, nv);
     int spec = 0;
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
@@ -389,18 +414,23 @@ __global__ void k_spl_prefetch(const MapDev* maps, const SessInfo* si, BatchBufs
     const int t = cand_t(cand_local(cur, b.cand_sshift));
     const int32_t base = cj == 6 ? cand_vid(cur) : b.cand_nbr[size_t(pos) * 6 + cj];
     int32_t X = -1;
+    bool simple = false;  // its record alone says whether it exists at t
     if (base >= 0) {
       if (j == 6) {
         X = base;
       } else {
         const VoxState& bs = m.vs[base];
-        int32_t cur_id;
-        if (bs.tag == tag && bs.seg >= 0) cur_id = b.seg_nbr[bs.seg * 6 + j];
-        else cur_id = key_neighbour_ok(bs.key, j) ? lookup_vid(m, key_neighbour(bs.key, j)) : -1;
-        X = vid_at(m, cur_id, tag, t);
+        if (bs.tag == tag && bs.seg >= 0) {
+          const int2 nb = b.seg_nbr[bs.seg * 6 + j];
+          simple = nb.y != kNbrSlow;
+          X = simple ? nb.x : vid_at(m, nb.x, tag, t);
+        } else if (key_neighbour_ok(bs.key, j)) {
+          X = vid_at(m, lookup_vid(m, key_neighbour(bs.key, j)), tag, t);
+        }
       }
     }
     int xseg = -1, tn = kNever;
+    if (simple && X >= 0 && m.vs[X].tag == tag && m.vs[X].create_t > t) X = -1;
     if (X >= 0) {
       const VoxState& xs = m.vs[X];
       if (xs.tag == tag && xs.seg >= 0 && xs.evict_t == kNever) {
@@ -414,19 +444,20 @@ __global__ void k_spl_prefetch(const MapDev* maps, const SessInfo* si, BatchBufs
   }
 }
 
-constexpr int kMrThreads = 256;  // threads of one session's merge replay
-constexpr int kWin = 36;         // window entries (36 x 7 records <= 256 threads)
-constexpr int kSPre = 2 * kWin;  // static candidates loaded per window
+constexpr int kMrWaves = 8;      // waves of one session's merge replay: acting entries evaluated per window
+constexpr int kMrThreads = 64 * kMrWaves;
+constexpr int kWin = 36;         // window entries (36 x 7 records <= 512 threads)
+constexpr int kSPre = 2 * kWin;  // static candidates and pool entries merged per window
+constexpr int kStat = 1024;      // static candidates held in LDS
 constexpr int kPoolCap = 2048;   // pending re-evaluations, kept sorted
-constexpr int kNewCap = 2048;    // keys created by one window's taint phase
-constexpr int kFxCap = 2048;     // deferred taint side effects of one window
 constexpr int kTaintPer = 49;    // up to 7 changed voxels x their closed neighbourhood
-constexpr int kFwCap = 512;      // first-writer hash: >= 2 x the kWin x 7 voxels one window writes
+constexpr int kKeysPer = 8;      // keys a tainted voxel can give: its next call and its candidates
+constexpr int kNewCap = kMrWaves * kTaintPer * kKeysPer;  // keys one window's commits can create
+constexpr int kPlS = kPlaneD + 1;  // doubles per plane record in LDS (odd: a lane per record, no bank conflicts)
 static_assert(kWin * 7 <= kMrThreads, "one thread per window record");
-static_assert(2 * kWin * 7 <= kFwCap, "first-writer hash at most half full");
 static_assert(kWin <= 64, "window bookkeeping runs in one wave");
-
-__device__ inline uint32_t fw_hash(int32_t v) { return (uint32_t(v) * 2654435761u) >> (32 - 9); }
+static_assert(kTaintPer <= 64, "an acting entry's taint phase takes a lane per item");
+static_assert(128 + kSPre <= kMrThreads && 2 * kSPre <= 3 * 64, "the window's merge");
 
 __device__ inline int rank_lt(const uint64_t* a, int n, uint64_t v) {  // elements < v
   int lo = 0, hi = n;
@@ -452,16 +483,26 @@ __device__ inline int rank_le(const uint64_t* a, int n, uint64_t v) {  // elemen
 //   fill     the next kWin keys of the static list (acting candidates) merged
 //            with the sorted pool of re-evaluations, duplicates dropped;
 //   records  each entry's voxel and six eligible neighbours (group, plane);
-//   evaluate each entry's merge() on its own copy of the current state;
-//   taint    for every acting entry, in parallel, the re-evaluations its
-//            merges make necessary (new keys and the voxels' dirty/taint
-//            marks, held back until the entry commits);
+//   gates    every entry's six gates in parallel: an entry acts if one passes;
+//   act      the first kMrWaves acting entries, a wave each: the merge() on a
+//            copy of the current state and, a lane per item, the
+//            re-evaluations its merges make necessary (new keys and the
+//            voxels' dirty/taint marks, held in registers until it commits);
 //   commit   in point order.  An entry whose records, or (if it acts) the
-//            records its taint phase read, were changed by an earlier commit
-//            of the window, or that a new key must precede, stops the commit:
-//            it and every later entry return to the pool.
+//            records its taint phase read, were changed by an earlier entry
+//            of the window, or that a new key must precede, or that acts and
+//            got no wave, stops the commit: it and every later entry return
+//            to the pool.
 // A committed entry therefore saw exactly the state the serial order gives
 // it, and its taint phase read the same records a serial one would.
+//
+// Bound by the chain of a window: a merge's re-evaluations mostly come before
+// the rest of the window, so a window commits 2 to 3 acting entries (of some
+// 20) and a scan with 30 merges takes about 15.  Hence eight barriers a
+// window, the window's merge in one wave, the statics in LDS, and the taint
+// phase's loads beside the merge's arithmetic: 11 us a window (15.5 with a
+// lane per entry for the merges, twenty barriers and a hash of first writers),
+// of which the acting waves' loads (three to five round trips) take 4.5.
 __global__ void __launch_bounds__(kMrThreads) k_merge_replay(const MapDev* maps, const SessInfo* si, int nsess,
                                                              BatchBufs b) {
   const int s = blockIdx.x;
@@ -470,505 +511,407 @@ __global__ void __launch_bounds__(kMrThreads) k_merge_replay(const MapDev* maps,
   MapCounters* c = m.ctr;
   const int tag = c->tag, off = si[s].off;
   const int spl_hi = si[s].spl_hi;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   __shared__ uint64_t pool[2][kPoolCap];
-  __shared__ uint64_t skey[kSPre];
-  __shared__ int spos[kSPre];
+  __shared__ uint64_t skey[kStat];  // statics from sbase on
+  __shared__ int spos[kStat];
   __shared__ uint64_t wkey[kWin];
   __shared__ int wpos[kWin];
   __shared__ int wspl[kWin];  // index of a static entry in spl (-1: pool entry)
-  __shared__ double pl[kWin][7][kPlaneD];
+  __shared__ double pl[kWin][7][kPlS];
   __shared__ uint64_t grp[kWin][7];
   __shared__ int32_t nbv[kWin][7];
-  __shared__ int clos[kWin][8];
-  __shared__ int nclos[kWin];
-  __shared__ int act[kWin];
-  __shared__ int32_t r2[kWin][kTaintPer];
-  __shared__ uint64_t nkey[kNewCap];
-  __shared__ int nkown[kNewCap];
-  __shared__ int32_t fx_v[kFxCap];
-  __shared__ int fx_wk[kFxCap];  // owner entry * 2 + kind (0 in-scan taint, 1 dirty flag)
-  __shared__ uint64_t gbuf[kNewCap + kWin];
-  __shared__ uint64_t sbuf[kNewCap + kWin];
-  __shared__ int sh_i[8];
-  __shared__ uint64_t mk[2 * kSPre];  // fill: statics and pool entries merged
-  __shared__ int mpos[2 * kSPre];
-  __shared__ int mspl[2 * kSPre];
-  __shared__ int mval[2 * kSPre];
-  __shared__ int mpre[2 * kSPre];
-  __shared__ int32_t rseg[kWin][7];   // record voxels: segment of this scan (-1 none), key, flags
+  __shared__ int32_t rseg[kWin][7];  // record voxels: segment of this scan (-1 none), key, flags
   __shared__ uint64_t rkey[kWin][7];
   __shared__ uint32_t rflg[kWin][7];
-  __shared__ int sh_mg;
-  __shared__ int sh_rew;  // statics of this window that are read again next window
-  __shared__ uint64_t sh_minkey[kWin];
-  __shared__ int sh_conf[kWin];
-  __shared__ int32_t fw_key[kFwCap];  // voxels written in this window -> first writing entry
-  __shared__ int32_t fw_min[kFwCap];
-  int sp = si[s].spl_lo, pb = 0, ph = 0, pn = 0;
+  __shared__ int gates[kWin];        // gates passed on the window's state (bit j)
+  __shared__ int conf[kWin];
+  __shared__ uint64_t minkey[kMrWaves];  // first new key of the waves' entries
+  __shared__ int actw[kMrWaves];     // the waves' entries (kWin: none)
+  __shared__ int clos[kMrWaves];     // their changed records (bit j)
+  __shared__ int2 wr[kMrWaves * 7];  // the voxels they change, with the entry
+  __shared__ uint64_t gbuf[kNewCap + kWin];
+  __shared__ uint64_t mk[2 * kSPre];  // fill: statics and pool entries merged
+  __shared__ int mspl[2 * kSPre];
+  __shared__ int sh_i[5];
+  int sp = si[s].spl_lo, sbase = sp, pb = 0, ph = 0, pn = 0;
   int evals = 0, merges = 0, windows = 0, requeued = 0, max_acting = 0, err = 0;
   uint64_t last = ~0ull;
+  for (int k = tid; k < min(kStat, spl_hi - sbase); k += kMrThreads) {
+    skey[k] = b.cand_in[sbase + k];
+    spos[k] = b.spl[sbase + k];
+  }
+  __syncthreads();
   while (true) {
-    // ---- fill the window: the loaded statics and pool entries merged in
+    // ---- fill the window: the next statics and pool entries merged in
     //      parallel (merge path; statics first on equal keys), duplicates and
-    //      keys beyond what is loaded dropped, the first kWin taken
+    //      keys beyond what is taken in dropped, the first kWin taken
     const int ns = min(kSPre, spl_hi - sp), np = min(kSPre, pn - ph);
-    if (tid < ns) {
-      skey[tid] = b.cand_in[sp + tid];
-      spos[tid] = b.spl[sp + tid];
+    if (sp + ns > sbase + kStat) {
+      sbase = sp;
+      for (int k = tid; k < min(kStat, spl_hi - sbase); k += kMrThreads) {
+        skey[k] = b.cand_in[sbase + k];
+        spos[k] = b.spl[sbase + k];
+      }
+      __syncthreads();
     }
-    __syncthreads();
+    const uint64_t* sseg = skey + (sp - sbase);
     const uint64_t* pseg = &pool[pb][ph];
-    uint64_t lim = ~0ull;  // keys above an unloaded static or pool entry wait
-    if (spl_hi - sp > kSPre) lim = skey[ns - 1];
-    if (pn - ph > kSPre && pseg[np - 1] < lim) lim = pseg[np - 1];
     const int M = ns + np;
     if (tid < ns) {
-      const int p = tid + rank_lt(pseg, np, skey[tid]);
-      mk[p] = skey[tid];
-      mpos[p] = spos[tid];
+      const int p = tid + rank_lt(pseg, np, sseg[tid]);
+      mk[p] = sseg[tid];
       mspl[p] = sp + tid;
     } else if (tid >= 128 && tid - 128 < np) {
       const int j = tid - 128;
-      const int p = j + rank_le(skey, ns, pseg[j]);
+      const int p = j + rank_le(sseg, ns, pseg[j]);
       mk[p] = pseg[j];
-      mpos[p] = -1;
       mspl[p] = -1;
     }
     __syncthreads();
-    // valid: not over the limit, not a duplicate of the previous key; prefix
-    // counts from wave ballots (M <= 2 * kSPre = 144 < 3 waves)
-    {
-      const int lane = tid & 63, wv = tid >> 6;
-      const bool in = tid < M;
-      const bool over = in && mk[tid] > lim;
-      const bool ok = in && !over && mk[tid] != (tid == 0 ? last : mk[tid - 1]);
-      const bool stat = in && !over && mpos[tid] >= 0;
-      const uint64_t bok = __ballot(ok), bst = __ballot(stat);
-      if (lane == 0 && wv < 3) {
-        mpre[wv] = __popcll(bok);
-        mval[wv] = __popcll(bst);
-      }
-      if (tid == 0) {
-        sh_i[0] = 0x7fffffff;  // first position over the limit
-      }
-      __syncthreads();
-      int base = 0, sbase = 0;
-      for (int q = 0; q < wv && q < 3; ++q) {
-        base += mpre[q];
-        sbase += mval[q];
-      }
-      const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-      const int pre = base + __popcll(bok & below);
-      const int spre = sbase + __popcll(bst & below);
-      if (ok && pre < kWin) {
-        wkey[pre] = mk[tid];
-        wpos[pre] = mpos[tid];
-        wspl[pre] = mspl[tid];
-      }
-      if (over && (tid == 0 || mk[tid - 1] <= lim)) atomicMin(&sh_i[0], tid);
-      // the kWin-th taken key ends the consumed range
-      if (ok && pre == kWin - 1) {
-        sh_i[3] = tid + 1;
-        sh_i[4] = spre + (stat ? 1 : 0);
-      }
-      __syncthreads();
-      if (tid == 0) {
-        const int total = mpre[0] + mpre[1] + mpre[2];
-        const int statics = mval[0] + mval[1] + mval[2];
-        int cut, used;
-        if (total >= kWin) {
-          cut = sh_i[3];
-          used = sh_i[4];
-        } else {
-          cut = sh_i[0] < M ? sh_i[0] : M;  // statics counted only below the limit
-          used = statics;
+    // valid: not over the limit, not a duplicate of the previous key; one
+    // wave, three positions a lane
+    if (wv == 0) {
+      uint64_t lim = ~0ull;  // keys above a static or pool entry left out wait
+      if (spl_hi - sp > kSPre) lim = sseg[ns - 1];
+      if (pn - ph > kSPre && pseg[np - 1] < lim) lim = pseg[np - 1];
+      int total = 0, statics = 0, cut = M, used = 0;
+      bool full = false;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const int p = 64 * q + lane;
+        const bool in = p < M;
+        const uint64_t key = in ? mk[p] : ~0ull;
+        const bool over = in && key > lim;
+        const bool ok = in && !over && key != (p == 0 ? last : mk[p - 1]);
+        const bool stat = in && !over && mspl[p] >= 0;
+        const uint64_t bok = __ballot(ok), bst = __ballot(stat), bov = __ballot(over);
+        const int pre = total + __popcll(bok & bits_below(lane));
+        if (ok && pre < kWin) {
+          wkey[pre] = key;
+          wspl[pre] = mspl[p];
+          wpos[pre] = mspl[p] >= 0 ? spos[mspl[p] - sbase] : -1;
         }
+        const uint64_t bend = __ballot(ok && pre == kWin - 1);  // the kWin-th taken key ends the range
+        if (bend) {
+          const int e = __ffsll((unsigned long long)bend) - 1;
+          full = true;
+          cut = 64 * q + e + 1;
+          used = statics + __popcll(bst & (bits_below(e) | (1ull << e)));
+        }
+        if (bov && !full && cut == M) cut = 64 * q + __ffsll((unsigned long long)bov) - 1;
+        total += __popcll(bok);
+        statics += __popcll(bst);
+      }
+      if (!full) used = statics;  // statics counted only below the limit
+      if (lane < kWin) {
+        gates[lane] = 0;
+        conf[lane] = 0;
+      }
+      if (lane < kMrWaves) minkey[lane] = ~0ull;
+      if (lane == 0) {
         sh_i[0] = total < kWin ? total : kWin;
         sh_i[1] = used;
-        sh_i[2] = ph + (cut - used);
+        sh_i[2] = cut;
+        sh_i[3] = 0;  // keys for the pool
+        sh_i[4] = 0;  // changed voxels
       }
-      __syncthreads();
     }
-    const int n = sh_i[0];
-    const int consumed = sh_i[1] + (sh_i[2] - ph);
-    const int used = sh_i[1];
+    __syncthreads();
+    const int n = sh_i[0], used = sh_i[1], cut = sh_i[2];
     sp += used;
-    ph = sh_i[2];
+    ph += cut - used;
     if (n == 0) {
-      if (consumed == 0) break;  // nothing left
-      continue;                  // only duplicates of the last key were loaded
+      if (cut == 0) break;  // nothing left
+      __syncthreads();      // (sh_i is read before the next fill writes it)
+      continue;             // only duplicates of the last key were taken in
     }
     ++windows;
     // ---- records: thread w*7+j, j = 6 is the voxel itself
+    const int rw = tid / 7, rj = tid - 7 * rw;
+    int32_t rv = -1;
+    double rp[kPlaneD];
     if (tid < n * 7) {
-      const int w = tid / 7, j = tid % 7;
-      const uint64_t cur = wkey[w];
+      const uint64_t cur = wkey[rw];
       const int t = cand_t(cur);
       const int32_t V = cand_vid(cur);
-      int32_t nv;
-      if (j == 6) {
-        nv = V;
-      } else if (wpos[w] >= 0) {
-        nv = b.cand_nbr[size_t(wpos[w]) * 6 + j];
-      } else {  // a re-evaluation: the ids from its first evaluation in this scan, if any
-        int32_t* slot = b.tnbr + (size_t(off) + size_t(t)) * 6 + j;
-        const int32_t cached = *slot;
-        if (cached != 0) {
-          nv = cached - 2;
+      if (rj == 6) {
+        rv = V;
+      } else if (wpos[rw] >= 0) {
+        rv = b.cand_nbr[size_t(wpos[rw]) * 6 + rj];
+      } else {  // a re-evaluation
+        const VoxState& vst = m.vs[V];
+        rv = (vst.tag == tag && vst.seg >= 0) ? nbr_eligible(m, b.seg_nbr[vst.seg * 6 + rj], tag, t)
+                                              : nbr_at(m, vst.key, rj, tag, t);
+      }
+      nbv[rw][rj] = rv;
+      if (rv >= 0) {
+        const VoxState& ns_ = m.vs[rv];
+        for (int k = 0; k < kPlaneD; ++k) rp[k] = m.plane[size_t(rv) * kPlaneD + k];
+        grp[rw][rj] = ns_.group_id;
+        rseg[rw][rj] = (ns_.tag == tag && ns_.seg >= 0) ? ns_.seg : -1;
+        rkey[rw][rj] = ns_.key;
+        rflg[rw][rj] = ns_.flags;
+        for (int k = 0; k < kPlaneD; ++k) pl[rw][rj][k] = rp[k];
+      }
+    }
+    __syncthreads();
+    // ---- gates on the window's state (an entry no neighbour passes changes
+    //      nothing)
+    if (rv >= 0 && rj < 6 && grp[rw][rj] != grp[rw][6]) {
+      double pv[6];
+      for (int k = 0; k < 6; ++k) pv[k] = pl[rw][6][k];
+      if (merge_gate(pv, rp, m.merge_a, m.merge_d)) atomicOr(&gates[rw], 1 << rj);
+    }
+    __syncthreads();
+    uint64_t am = __ballot(lane < n && gates[min(lane, kWin - 1)] != 0);  // the acting entries
+    max_acting = max(max_acting, __popcll(am));
+    int w = kWin, nlim = n;  // this wave's entry; the first acting one without a wave
+    {
+      uint64_t r = am;
+      for (int a = 0; a < kMrWaves && r; ++a) {
+        const int e = __ffsll((unsigned long long)r) - 1;
+        if (a == wv) w = e;
+        r &= r - 1;
+      }
+      if (r) nlim = __ffsll((unsigned long long)r) - 1;
+    }
+    w = __builtin_amdgcn_readfirstlane(w);
+    int32_t X = -1;  // this lane's taint item: a voxel of a record's closed neighbourhood
+    bool need = false;
+    int nl = 0, xseg = -1;
+    uint64_t loc[kKeysPer];
+    int cl = 0;
+    if (w < kWin) {
+      const int t = cand_t(wkey[w]);
+      // ---- taint item r: voxel j (6: itself) next to record cj.  What does
+      //      not depend on the merge is loaded before it; nothing here is
+      //      written before the commit.
+      const int cj = lane / 7, j = lane - 7 * cj;
+      const bool item = lane < kTaintPer && nbv[w][min(cj, 6)] >= 0;
+      int pre_tn = kNever;
+      const bool pre = wspl[w] >= 0 && wspl[w] < b.pre_cap;  // a static entry's come precomputed
+      bool simple = false;
+      if (item) {
+        if (pre) {
+          const int at = wspl[w] * kPreItems + lane;
+          X = b.pre_x[at];
+          xseg = b.pre_seg[at];
+          pre_tn = b.pre_tn[at];
+        } else if (j == 6) {
+          X = nbv[w][cj];
         } else {
-          const VoxState& vst = m.vs[V];
-          nv = (vst.tag == tag && vst.seg >= 0) ? eligible_at(m, b.seg_nbr[vst.seg * 6 + j], tag, t)
-                                                : nbr_at(m, vst.key, j, tag, t);
-          *slot = nv + 2;
-        }
-      }
-      nbv[w][j] = nv;
-      if (nv >= 0) {
-        const VoxState& ns_ = m.vs[nv];
-        grp[w][j] = ns_.group_id;
-        rseg[w][j] = (ns_.tag == tag && ns_.seg >= 0) ? ns_.seg : -1;
-        rkey[w][j] = ns_.key;
-        rflg[w][j] = ns_.flags;
-        for (int k = 0; k < kPlaneD; ++k) pl[w][j][k] = m.plane[size_t(nv) * kPlaneD + k];
-      }
-    }
-    __syncthreads();
-    // ---- merge(): each entry's six neighbours in order against its own
-    //      plane, one thread per entry with its seven records in registers
-    //      (an entry no neighbour passes changes nothing)
-    if (tid < n) {
-      const int w = tid;
-      double pv[kPlaneD], pn[6][kPlaneD];
-#pragma unroll
-      for (int k = 0; k < kPlaneD; ++k) pv[k] = pl[w][6][k];
-#pragma unroll
-      for (int j = 0; j < 6; ++j)
-#pragma unroll
-        for (int k = 0; k < kPlaneD; ++k) pn[j][k] = pl[w][j][k];
-      const uint64_t g6 = grp[w][6];
-      int nc = 0;
-#pragma unroll
-      for (int j = 0; j < 6; ++j) {
-        if (nbv[w][j] < 0 || grp[w][j] == g6) continue;
-        if (!merge_gate(pv, pn[j], m.merge_a, m.merge_d)) continue;
-        merge_fuse(pv, pn[j]);
-#pragma unroll
-        for (int k = 0; k < kPlaneD; ++k) pl[w][j][k] = pn[j][k];
-        grp[w][j] = g6;
-        clos[w][nc++] = j;
-      }
-      if (nc > 0) {
-#pragma unroll
-        for (int k = 0; k < kPlaneD; ++k) pl[w][6][k] = pv[k];
-        clos[w][nc++] = 6;
-      }
-      nclos[w] = nc;
-    }
-    __syncthreads();
-    if (tid < 64) {  // acting entries in order (n <= kWin < 64: one wave)
-      const bool a = tid < n && nclos[tid] > 0;
-      const uint64_t bm = __ballot(a);
-      const uint64_t below = tid == 0 ? 0ull : (~0ull >> (64 - tid));
-      if (a) act[__popcll(bm & below)] = tid;
-      if (tid == 0) {
-        sh_i[3] = __popcll(bm);
-        sh_i[4] = 0;  // new keys
-        sh_i[5] = 0;  // side effects
-      }
-    }
-    __syncthreads();
-    const int na = sh_i[3];
-    max_acting = max(max_acting, na);
-    // ---- conflicts through the records: the first writer of every voxel the
-    //      acting entries change, then for each entry whether one of its
-    //      seven records has an earlier writer.  The commit stops at the
-    //      first such entry at the latest, so only the acting entries before
-    //      it run the taint phase.
-    for (int i = tid; i < kFwCap; i += kMrThreads) {
-      fw_key[i] = -1;
-      fw_min[i] = kWin;
-    }
-    if (tid < kWin) {
-      sh_minkey[tid] = ~0ull;
-      sh_conf[tid] = 0;
-    }
-    __syncthreads();
-    // na * 8 can exceed the block (kWin * 8 > kMrThreads): strided
-    for (int q = tid; q < na * 8; q += kMrThreads) {
-      const int a = q >> 3, ci = q & 7;
-      const int k = act[a];
-      if (ci < nclos[k]) {
-        const int32_t X = nbv[k][clos[k][ci]];
-        uint32_t h = fw_hash(X);
-        while (true) {  // at most half full: the probe ends
-          const int32_t old = atomicCAS(&fw_key[h], -1, X);
-          if (old == -1 || old == X) {
-            atomicMin(&fw_min[h], k);
-            break;
-          }
-          h = (h + 1) & (kFwCap - 1);
-        }
-      }
-    }
-    __syncthreads();
-    for (int q = tid; q < n * 7; q += kMrThreads) {
-      const int w = q / 7;
-      const int32_t v = nbv[w][q % 7];
-      if (v < 0) continue;
-      uint32_t h = fw_hash(v);
-      while (true) {
-        const int32_t kk = fw_key[h];
-        if (kk == -1) break;
-        if (kk == v) {
-          if (fw_min[h] < w) sh_conf[w] = 1;
-          break;
-        }
-        h = (h + 1) & (kFwCap - 1);
-      }
-    }
-    __syncthreads();
-    if (tid < 64) {  // acting entries before the first record conflict (act ascends)
-      const uint64_t cm = __ballot(tid < n && sh_conf[tid]);
-      const int pre = cm ? __ffsll((unsigned long long)cm) - 1 : n;
-      const uint64_t am = __ballot(tid < na && act[tid] < pre);
-      if (tid == 0) sh_i[6] = __popcll(am);
-    }
-    __syncthreads();
-    const int nat = sh_i[6];
-    // ---- taint phase of those acting entries: for each changed voxel and
-    //      each voxel of its closed neighbourhood X: X re-evaluates its next
-    //      call and its later candidates if X changed itself, or if X (a plane
-    //      not in the group) passes the gates against a new record.  A voxel
-    //      of the scan records its dirty/taint times, one outside is marked
-    //      dirty.
-    for (int T = tid; T < nat * kTaintPer; T += kMrThreads) {
-      const int a = T / kTaintPer, r = T % kTaintPer, ci = r / 7, j = r % 7;
-      const int w = act[a];
-      const int nc0 = nclos[w];
-      int32_t X = -1;
-      if (ci < nc0) {
-        const int t = cand_t(wkey[w]);
-        const int cj = clos[w][ci];
-        const int32_t base_v = nbv[w][cj];
-        // a static entry's X, its segment and next call come precomputed
-        const int pre = (wspl[w] >= 0 && wspl[w] < b.pre_cap) ? wspl[w] * kPreItems + cj * 7 + j : -1;
-        int pre_seg = -1, pre_tn = kNever;
-        X = base_v;
-        if (pre >= 0) {
-          X = b.pre_x[pre];
-          pre_seg = b.pre_seg[pre];
-          pre_tn = b.pre_tn[pre];
-        } else if (j < 6) {
           const int bseg = rseg[w][cj];
-          const uint64_t bkey = rkey[w][cj];
-          int32_t cur_id;
-          if (bseg >= 0) cur_id = b.seg_nbr[bseg * 6 + j];
-          else cur_id = key_neighbour_ok(bkey, j) ? lookup_vid(m, key_neighbour(bkey, j)) : -1;
-          X = vid_at(m, cur_id, tag, t);
-        }
-        bool need = false;
-        if (X >= 0) {
-          // what depends only on X (and, for a static entry, on its
-          // precomputed segment) is loaded in one round; nothing here is
-          // written before the commit
-          const VoxState* xv = m.vs + X;
-          const uint32_t xflags = xv->flags;
-          const uint64_t xkey = xv->key, xgrp = xv->group_id;
-          const int32_t xtag = xv->tag, xsg = xv->seg, xev = xv->evict_t, xmp = xv->merge_pos;
-          double px[kPlaneD];
-          for (int k = 0; k < kPlaneD; ++k) px[k] = m.plane[size_t(X) * kPlaneD + k];
-          int32_t nct = 0, ct[7];
-          if (pre_seg >= 0) {
-            nct = b.seg_nct[pre_seg];
-            for (int k = 0; k < 7; ++k) ct[k] = b.seg_ct[pre_seg * 7 + k];
-          }
-          for (int k = 0; k < nc0; ++k) need |= (nbv[w][clos[w][k]] == X);
-          if (!need && (xflags & kPlane) && (xflags & kInit)) {
-            int64_t ax, ay, az;
-            unpack_key(xkey, ax, ay, az);
-            for (int k = 0; k < nc0; ++k) {
-              const int cc = clos[w][k];
-              int64_t bx, by, bz;
-              unpack_key(rkey[w][cc], bx, by, bz);
-              const int64_t dist = (ax > bx ? ax - bx : bx - ax) + (ay > by ? ay - by : by - ay) +
-                                   (az > bz ? az - bz : bz - az);
-              if (dist == 1 && grp[w][cc] != xgrp && merge_gate(px, pl[w][cc], m.merge_a, m.merge_d)) need = true;
-            }
-          }
-          if (need) {
-            int xseg = pre_seg, tn = pre_tn;
-            if (pre < 0) {
-              xseg = (xtag == tag && xsg >= 0 && xev == kNever) ? xsg : -1;
-              tn = (xseg >= 0 && xmp != kNever) ? first_call_after(b, xsg, xmp, t, off) : kNever;
-              if (xseg >= 0) {
-                nct = b.seg_nct[xseg];
-                for (int k = 0; k < nct; ++k) ct[k] = b.seg_ct[xseg * 7 + k];
-              }
-            }
-            if (xseg >= 0) {
-              uint64_t loc[8];
-              int nl = 0;
-              if (tn != kNever) loc[nl++] = cand_key(0, tn, X);
-              for (int k = 0; k < nct; ++k) {
-                const int tc = ct[k];
-                if (tc > t) loc[nl++] = cand_key(0, tc, X);
-              }
-              if (nl > 0) {
-                const int at = atomicAdd(&sh_i[4], nl);
-                for (int k = 0; k < nl; ++k)
-                  if (at + k < kNewCap) {
-                    nkey[at + k] = loc[k];
-                    nkown[at + k] = w;
-                  }
-              }
-              const int f = atomicAdd(&sh_i[5], 1);
-              if (f < kFxCap) {
-                fx_v[f] = X;
-                fx_wk[f] = w * 2;
-              }
-            } else if (xflags & kAlive) {
-              const int f = atomicAdd(&sh_i[5], 1);
-              if (f < kFxCap) {
-                fx_v[f] = X;
-                fx_wk[f] = w * 2 + 1;
-              }
-            }
+          if (bseg >= 0) {
+            const int2 nb = b.seg_nbr[bseg * 6 + j];
+            simple = nb.y != kNbrSlow;
+            X = simple ? nb.x : vid_at(m, nb.x, tag, t);
+          } else if (key_neighbour_ok(rkey[w][cj], j)) {
+            X = vid_at(m, lookup_vid(m, key_neighbour(rkey[w][cj], j)), tag, t);
           }
         }
       }
-      r2[w][r] = X;
-    }
-    __syncthreads();
-    const int nnew = sh_i[4], nfx = sh_i[5];
-    if (nnew > kNewCap || nfx > kFxCap) {
-      err |= 16;
-      break;
-    }
-    // ---- commit in point order, all at once: the first entry that read a
-    //      voxel an earlier acting entry of the window writes (its seven
-    //      records, found above, and if it acts the records of its taint
-    //      phase), or that an earlier entry's new key must precede, stops the
-    //      commit.  The entries before it commit together: their write sets
-    //      are disjoint (an entry that writes a voxel also read it).
-    for (int q = tid; q < nnew; q += kMrThreads)
-      atomicMin(reinterpret_cast<unsigned long long*>(&sh_minkey[nkown[q]]), (unsigned long long)nkey[q]);
-    for (int q = tid; q < nat * kTaintPer; q += kMrThreads) {  // the taint reads
-      const int w = act[q / kTaintPer];
-      const int32_t v = r2[w][q % kTaintPer];
-      if (v < 0) continue;
-      uint32_t h = fw_hash(v);
-      while (true) {
-        const int32_t kk = fw_key[h];
-        if (kk == -1) break;
-        if (kk == v) {
-          if (fw_min[h] < w) sh_conf[w] = 1;
-          break;
+      uint32_t xflags = 0;
+      uint64_t xkey = 0, xgrp = 0;
+      int xmp = kNever;
+      double px[kPlaneD];
+      int nct = 0, ct[7], xs0 = 0, xs1 = 0;
+      if (X >= 0) {
+        const VoxState* xv = m.vs + X;
+        const int xtag = xv->tag, xsg = xv->seg, xev = xv->evict_t, xct = xv->create_t;
+        xflags = xv->flags;
+        xkey = xv->key;
+        xgrp = xv->group_id;
+        xmp = xv->merge_pos;
+        for (int k = 0; k < kPlaneD; ++k) px[k] = m.plane[size_t(X) * kPlaneD + k];
+        if (!pre) {
+          xseg = (xtag == tag && xsg >= 0 && xev == kNever) ? xsg : -1;
+          if (simple && xtag == tag && xct > t) X = -1;  // created later in the scan
         }
-        h = (h + 1) & (kFwCap - 1);
+        if (xseg >= 0) {
+          nct = b.seg_nct[xseg];
+          for (int k = 0; k < 7; ++k) ct[k] = b.seg_ct[xseg * 7 + k];
+          xs0 = b.seg_start[xseg];
+          xs1 = b.seg_end[xseg];
+        }
       }
+      // ---- merge(): the six neighbours in order against the entry's own
+      //      plane (the gates after a merge on the fused plane)
+      double pv[kPlaneD];
+      for (int k = 0; k < kPlaneD; ++k) pv[k] = pl[w][6][k];
+      const uint64_t g6 = grp[w][6];
+      const int cand = lane < 6 && nbv[w][min(lane, 5)] >= 0 && grp[w][min(lane, 5)] != g6;
+      uint64_t pass = uint64_t(uint32_t(gates[w]));
+      while (pass) {
+        const int jj = __ffsll((unsigned long long)pass) - 1;
+        double pn[kPlaneD];
+        for (int k = 0; k < kPlaneD; ++k) pn[k] = pl[w][jj][k];
+        merge_fuse(pv, pn);
+        wave_lds_sync();
+        if (lane == 0)
+          for (int k = 0; k < kPlaneD; ++k) pl[w][jj][k] = pn[k];
+        wave_lds_sync();
+        cl |= 1 << jj;
+        bool ok = cand && lane > jj;
+        if (ok) {
+          double pq[6];
+          for (int k = 0; k < 6; ++k) pq[k] = pl[w][lane][k];
+          ok = merge_gate(pv, pq, m.merge_a, m.merge_d);
+        }
+        pass = __ballot(ok);
+      }
+      cl |= 1 << 6;
+      wave_lds_sync();
+      if (lane == 0)
+        for (int k = 0; k < kPlaneD; ++k) pl[w][6][k] = pv[k];
+      wave_lds_sync();
+      // ---- for each changed voxel and each voxel X of its closed
+      //      neighbourhood: X re-evaluates its next call and its later
+      //      candidates if X changed itself, or if X (a plane not in the
+      //      group) passes the gates against a new record.  A voxel of the
+      //      scan records its dirty/taint times, one outside is marked dirty.
+      if (!(item && ((cl >> cj) & 1))) X = -1;
+      if (X >= 0) {
+        int64_t ax, ay, az;
+        unpack_key(xkey, ax, ay, az);
+        for (int cc = 0; cc < 7; ++cc) {
+          if (!((cl >> cc) & 1)) continue;
+          if (nbv[w][cc] == X) need = true;
+          if (need || !(xflags & kPlane) || !(xflags & kInit) || xgrp == g6) continue;
+          int64_t bx, by, bz;
+          unpack_key(rkey[w][cc], bx, by, bz);
+          const int64_t dist = (ax > bx ? ax - bx : bx - ax) + (ay > by ? ay - by : by - ay) +
+                               (az > bz ? az - bz : bz - az);
+          if (dist != 1) continue;
+          double pc[6];
+          for (int k = 0; k < 6; ++k) pc[k] = pl[w][cc][k];
+          if (merge_gate(px, pc, m.merge_a, m.merge_d)) need = true;
+        }
+        need = need && (xseg >= 0 || (xflags & kAlive));
+        if (need && xseg >= 0) {
+          const int tn = pre ? pre_tn : (xmp != kNever ? first_call_in(b, xs0 + xmp, xs1, t, off) : kNever);
+          uint64_t first = ~0ull;
+#pragma unroll
+          for (int k = 0; k < kKeysPer; ++k) {
+            const int tc = k == 0 ? tn : ct[k > 0 ? k - 1 : 0];
+            const bool use = k == 0 ? tn != kNever : (k <= nct && tc > t);
+            loc[k] = use ? cand_key(0, tc, X) : ~0ull;
+            nl += use ? 1 : 0;
+            if (loc[k] < first) first = loc[k];
+          }
+          if (nl > 0) atomicMin(reinterpret_cast<unsigned long long*>(&minkey[wv]), (unsigned long long)first);
+        }
+      }
+    }
+    if (lane == 0) {
+      actw[wv] = w;
+      clos[wv] = cl;
+    }
+    if (w < kWin) {
+      int at = lane == 0 ? atomicAdd(&sh_i[4], __popc(unsigned(cl))) : 0;
+      at = __builtin_amdgcn_readfirstlane(at);
+      if (lane < 7 && ((cl >> lane) & 1)) wr[at + __popc(unsigned(cl) & ((1u << lane) - 1u))] = make_int2(nbv[w][lane], w);
     }
     __syncthreads();
-    if (tid < 64) {  // one wave (n <= kWin < 64): exclusive prefix minimum of the new keys
-      uint64_t pm = tid < n ? sh_minkey[tid] : ~0ull;
-      for (int o = 1; o < 64; o <<= 1) {
-        const uint64_t u = __shfl_up(pm, o, 64);
-        if (tid >= o && u < pm) pm = u;
+    // ---- conflicts: an entry whose records, or whose taint items, an earlier
+    //      entry of the window changes
+    {
+      const int me = rv >= 0 ? rw : -1, mx = X >= 0 ? w : -1, nw = sh_i[4];
+      bool hit_r = false, hit_x = false;
+#pragma unroll 8
+      for (int q = 0; q < nw; ++q) {
+        const int2 u = wr[q];
+        hit_r |= (u.x == rv) & (u.y < me);
+        hit_x |= (u.x == X) & (u.y < mx);
       }
-      uint64_t before = __shfl_up(pm, 1, 64);
-      if (tid == 0) before = ~0ull;
-      const bool stop_here = tid < n && (sh_conf[tid] || before <= wkey[tid]);
-      const uint64_t bm = __ballot(stop_here);
-      const int stop = bm ? __ffsll((unsigned long long)bm) - 1 : n;
-      int mg = (tid < stop && nclos[tid] > 0) ? nclos[tid] - 1 : 0;
-      for (int o = 32; o > 0; o >>= 1) mg += __shfl_xor(mg, o, 64);
-      if (tid == 0) {
-        sh_i[7] = stop;
-        sh_mg = mg;
-        // the statics from the stop on are read again from the static list
-        // (with their precomputed taint data) rather than sent to the pool;
-        // consumed statics ascend, so they are those with key >= the stop key
-        sh_rew = stop < n ? used - rank_lt(skey, used, wkey[stop]) : 0;
-      }
+      if (hit_r) conf[me] = 1;
+      if (hit_x) conf[w] = 1;
     }
     __syncthreads();
-    const int w = sh_i[7];
-    sp -= sh_rew;
-    merges += sh_mg;
-    evals += w;
-    for (int q = tid; q < w * 8; q += kMrThreads) {
-      const int e = q >> 3, ci = q & 7;
-      if (ci >= nclos[e]) continue;
-      const int j = clos[e][ci];
-      const int32_t X = nbv[e][j];
-      for (int k = 0; k < kPlaneD; ++k) m.plane[size_t(X) * kPlaneD + k] = pl[e][j][k];
-      m.vs[X].group_id = grp[e][j];
-      // an atomic bit set: another entry of this commit may set kDirty on X
-      atomicOr(&m.vs[X].flags, kMerged);
-      // the observe record from the LDS copies (merges never change the
-      // plane bit, which is all the observe pass reads of the flags)
-      int64_t kx, ky, kz;
-      unpack_key(rkey[e][j], kx, ky, kz);
-      VoxHot h;
-      h.mx = float(pl[e][j][0] - double(kx) * m.vs64);
-      h.my = float(pl[e][j][1] - double(ky) * m.vs64);
-      h.mz = float(pl[e][j][2] - double(kz) * m.vs64);
-      h.flags = rflg[e][j] | kMerged;
-      h.nx = float(pl[e][j][3]);
-      h.ny = float(pl[e][j][4]);
-      h.nz = float(pl[e][j][5]);
-      h.pad = 0.f;
-      m.hot[X] = h;
+    // ---- commit in point order, all at once: the first entry in conflict, or
+    //      that an earlier entry's new key must precede, stops it.  The
+    //      entries before it commit together: their write sets are disjoint
+    //      (an entry that writes a voxel also read it).  Every wave finds the
+    //      stop for itself.
+    int stop;
+    {
+      const int l = min(lane, kWin - 1);
+      const uint64_t key = wkey[l];
+      bool late = conf[l] != 0;
+#pragma unroll
+      for (int a = 0; a < kMrWaves; ++a) late |= (actw[a] < l) & (minkey[a] <= key);
+      const uint64_t bm = __ballot(lane < n && late);
+      stop = bm ? __ffsll((unsigned long long)bm) - 1 : n;
+      stop = min(stop, nlim);
+      // the statics from the stop on are read again from the static list
+      // (with their precomputed taint data) rather than sent to the pool;
+      // consumed statics ascend, so they are the last ones
+      sp -= __popcll(__ballot(lane >= stop && lane < n && wspl[l] >= 0));
     }
-    for (int f = tid; f < nfx; f += kMrThreads) {
-      const int e = fx_wk[f] >> 1;
-      if (e >= w) continue;
-      VoxState& xs = m.vs[fx_v[f]];
-      if (fx_wk[f] & 1) {
-        atomicOr(&xs.flags, kDirty);
-      } else {
-        const int t = cand_t(wkey[e]);
-        atomicMax(&xs.dirty_t, t);
-        atomicMin(&xs.taint_t, t);
+    evals += stop;
+    requeued += n - stop;
+#pragma unroll
+    for (int a = 0; a < kMrWaves; ++a) merges += actw[a] < stop ? __popc(unsigned(clos[a])) - 1 : 0;
+    if (w < stop) {
+      if (lane < 7 && ((cl >> lane) & 1)) {  // a lane per changed record
+        const int32_t Y = nbv[w][lane];
+        double q[kPlaneD];
+        for (int k = 0; k < kPlaneD; ++k) q[k] = pl[w][lane][k];
+        for (int k = 0; k < kPlaneD; ++k) m.plane[size_t(Y) * kPlaneD + k] = q[k];
+        m.vs[Y].group_id = grp[w][6];
+        // an atomic bit set: another entry of this commit may set kDirty on Y
+        atomicOr(&m.vs[Y].flags, kMerged);
+        // the observe record from the LDS copies (merges never change the
+        // plane bit, which is all the observe pass reads of the flags)
+        int64_t kx, ky, kz;
+        unpack_key(rkey[w][lane], kx, ky, kz);
+        write_hot_pl(m, Y, rflg[w][lane] | kMerged, q, kx, ky, kz);
+      }
+      if (need) {
+        VoxState& xs = m.vs[X];
+        if (xseg >= 0) {
+          const int t = cand_t(wkey[w]);
+          atomicMax(&xs.dirty_t, t);
+          atomicMin(&xs.taint_t, t);
+        } else {
+          atomicOr(&xs.flags, kDirty);
+        }
+      }
+      if (nl > 0) {
+        int at = atomicAdd(&sh_i[3], nl);
+#pragma unroll
+        for (int k = 0; k < kKeysPer; ++k)
+          if (loc[k] != ~0ull) gbuf[at++] = loc[k];
       }
     }
-    requeued += n - w;
     // ---- pool := pool[ph, pn) merged with the committed entries' new keys and
-    //      the entries sent back (duplicates are dropped at the next fill)
-    if (tid == 0) sh_i[6] = 0;
+    //      the pool entries sent back (duplicates are dropped at the next fill)
+    if (tid >= stop && tid < n && wspl[tid] < 0) gbuf[atomicAdd(&sh_i[3], 1)] = wkey[tid];
+    // duplicates of a key sent back must not be dropped against it: the last
+    // processed key is the last committed one
+    if (stop > 0) last = wkey[stop - 1];
     __syncthreads();
-    for (int k = tid; k < nnew + n; k += kMrThreads) {
-      uint64_t v;
-      bool keep;
-      if (k < nnew) {
-        v = nkey[k];
-        keep = nkown[k] < w;
-      } else {
-        v = wkey[k - nnew];
-        keep = k - nnew >= w && wspl[k - nnew] < 0;  // a static sent back is read again
-      }
-      if (keep) gbuf[atomicAdd(&sh_i[6], 1)] = v;
-    }
-    __syncthreads();
-    const int g = sh_i[6], rest = pn - ph;
+    const int g = sh_i[3], rest = pn - ph;
     if (g + rest > kPoolCap) {
       err |= 16;
       break;
     }
-    for (int k = tid; k < g; k += kMrThreads) {  // rank sort (ties by index)
-      const uint64_t v = gbuf[k];
-      int rk = 0;
-      for (int q = 0; q < g; ++q) rk += (gbuf[q] < v) || (gbuf[q] == v && q < k);
-      sbuf[rk] = v;
-    }
-    __syncthreads();
     const uint64_t* prest = &pool[pb][ph];
     uint64_t* dst = pool[1 - pb];
-    for (int k = tid; k < g; k += kMrThreads) dst[k + rank_lt(prest, rest, sbuf[k])] = sbuf[k];
-    for (int k = tid; k < rest; k += kMrThreads) dst[k + rank_le(sbuf, g, prest[k])] = prest[k];
-    // duplicates of a key sent back must not be dropped against it: the last
-    // processed key is the last committed one
-    if (w > 0) last = wkey[w - 1];
+    for (int k = tid; k < g; k += kMrThreads) {  // ties by index
+      const uint64_t v = gbuf[k];
+      int rk = rank_lt(prest, rest, v);
+#pragma unroll 4
+      for (int q = 0; q < g; ++q) rk += (gbuf[q] < v) || (gbuf[q] == v && q < k);
+      dst[rk] = v;
+    }
+    for (int k = tid; k < rest; k += kMrThreads) {
+      const uint64_t v = prest[k];
+      int rk = k;
+#pragma unroll 4
+      for (int q = 0; q < g; ++q) rk += gbuf[q] <= v;
+      dst[rk] = v;
+    }
     pb = 1 - pb;
     ph = 0;
     pn = g + rest;
