@@ -27,7 +27,6 @@
 // entries of the per-tile first-session table: every tile of the largest
 // input the library's compaction takes, and one past the last
 constexpr int kSfirstEntries = vmp::kPrimMaxItems / vmp::kPrimTile + 2;
-static_assert(vmp::kCsThreads == vmp::kPrimThreads, "the candidate starts run as the tail of a compaction tile");
 
 using namespace vmp;
 
@@ -620,9 +619,7 @@ static bool ws_layout(vmp_ctx* c, BatchWs& w, size_t n, int ns, size_t pre_cap, 
   ok = ok && dev(&b.seg_start, n) && dev(&b.seg_end, n) && dev(&b.seg_sess, n) && dev(&b.seg_vid, n) &&
        dev(&b.seg_entry, n);
   ok = ok && dev(&b.cre_t, n) && dev(&b.cre_seg, n) && dev(&b.co, n) && dev(&b.ev_vid, n);
-  ok = ok && dev(&b.cand_in, n) && dev(&b.cand_out, n) && dev(&b.cand_nbr, n * 6) &&
-       dev(&b.cand_spec, n) &&
-       dev(&b.cand_start, size_t(ns)) && dev(&b.spl, n);
+  ok = ok && dev(&b.cand_in, n) && dev(&b.cand_out, n) && dev(&b.cand_nbr, n * 6) && dev(&b.spl, n);
   ok = ok && dev(&b.seg_ct, n * 7) && dev(&b.seg_nct, n) && dev(&b.seg_nbr, n * 6);
   ok = ok && dev(&b.seg_cls, n) && dev(&b.seg_old, n);
   ok = ok && dev(&b.lv, n * 2) && dev(&b.lv2, n * 2) && dev(&b.lv_cnt, (n * 2 >> 6) + size_t(ns) + 2);
@@ -669,11 +666,10 @@ static bool ws_layout(vmp_ctx* c, BatchWs& w, size_t n, int ns, size_t pre_cap, 
   ok = ok && host(&w.h_out, sizeof(BatchOut) * S) && host(&w.h_motion, sizeof(MotionRec) * S) &&
        host(&w.h_vg, sizeof(VgJob) * S) && host(&w.h_vgst, sizeof(int32_t) * kVgStat * S);
   if (!ok) return false;
-  size_t t[3] = {0, 0, 0};
+  size_t t[2] = {0, 0};
   rocprim::radix_sort_pairs(nullptr, t[0], b.skey_in, b.skey_out, b.sval_in, b.sval_out, n, 0, 64, c->stream);
-  rocprim::radix_sort_keys(nullptr, t[1], b.cand_in, b.cand_out, n, 0, 64, c->stream);
-  rocprim::select(nullptr, t[2], rocprim::counting_iterator<int32_t>(0), b.flags, b.sel, b.cnt, n, c->stream);
-  w.temp_bytes = *std::max_element(t, t + 3) + 256;
+  rocprim::select(nullptr, t[1], rocprim::counting_iterator<int32_t>(0), b.flags, b.sel, b.cnt, n, c->stream);
+  w.temp_bytes = *std::max_element(t, t + 2) + 256;
   uint8_t* temp = nullptr;
   if (!dev(&temp, w.temp_bytes)) return false;
   w.temp = temp;
@@ -1823,28 +1819,10 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
         }
         if (!(mode & kStepBuild)) {
           timed_launch(c, kTkCandidates, [&] { hipLaunchKernelGGL(k_candidates, dim3(gn), dim3(T), 0, st, M, S, b); });
-          // the call at point time t is made by the voxel that received point
-          // t, so each candidate sits at its session offset plus t: the
-          // non-empty slots in order are the list sorted on (session, time)
-          if (prim) {
-            select_stable(st, ntot, PredCand{b.cand_in}, OutCand{b.cand_in, b.cand_out}, b.prim, b.cnt + 7,
-                          TailCandStarts{M, n, b});
-          } else {
-            size_t tb = w.temp_bytes;
-            if (rocprim::radix_sort_keys(w.temp, tb, b.cand_in, b.cand_out, size_t(ntot), 25, b.cand_sshift + sbits,
-                                         st) != hipSuccess)
-              return VMP_EDEVICE;
-            hipLaunchKernelGGL(k_cand_starts, dim3(1), dim3(kCsThreads), 0, st, M, n, b);
-          }
-          timed_launch(c, kTkSpecEval, [&] { hipLaunchKernelGGL(k_spec_eval, dim3(gn), dim3(T), 0, st, M, b); });
-          if (prim) {
-            select_stable(st, ntot, PredFlag{b.cand_spec}, OutSpl{b.spl, b.cand_in, b.cand_out, b.cand_sshift},
-                          b.prim, b.cnt + 4, TailSplRanges{M, S, n, b});
-          } else {
-            if (!select_flags(b.cand_spec, b.spl, b.cnt + 4)) return VMP_EDEVICE;
-            hipLaunchKernelGGL(k_spl_ranges, dim3(grid_for(n, 64)), dim3(64), 0, st, M, S, n, b);
-            hipLaunchKernelGGL(k_spl_keys, dim3(gn), dim3(T), 0, st, b);
-          }
+          timed_launch(c, kTkSpecEval, [&] {
+            hipLaunchKernelGGL(k_spec_eval, dim3(std::max(1, prim_tiles(ntot))), dim3(kPrimThreads), 0, st, M, S, b,
+                               prim_ws(b.prim));
+          });
           hipLaunchKernelGGL(k_spl_prefetch, dim3(std::min(gn * kPreItems, 4096)), dim3(T), 0, st, M, S, b);
           timed_launch(c, kTkMergeReplay,
                        [&] { hipLaunchKernelGGL(k_merge_replay, dim3(n), dim3(kMrThreads), 0, st, M, S, n, b); });

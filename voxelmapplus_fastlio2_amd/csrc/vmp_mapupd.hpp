@@ -87,7 +87,7 @@ struct SessInfo {
   int32_t is_build;
   int32_t seg_lo, seg_hi;  // its segments in the batch segment list
   int32_t cre_lo, cre_hi;  // its creation events in the batch creation list
-  int32_t spl_lo, spl_hi;  // its acting merge candidates in the compacted list
+  int32_t spl_lo, spl_hi;  // its acting merge candidates in spl
   int32_t ftop0, bump0;    // free-list top and bump pointer before its fast creations
 };
 
@@ -116,12 +116,10 @@ struct BatchBufs {
                        // (vid, segment, point time, evicted incarnation or -1);
                        // the r-th takes group id group_counter - ncre + r
   int32_t* ev_vid;     // evicted voxels in order, per session at its offset
-  uint64_t* cand_in;   // merge candidates, see cand_key(); per session at its offset
-  uint64_t* cand_out;  // sorted: session-major, then point time, then voxel
-  int32_t* cand_nbr;   // per sorted candidate: 6 eligible neighbour ids at its time
-  int32_t* cand_spec;  // per sorted candidate: 1 if it merges on the pre-replay state
-  int32_t* cand_start; // per session: first sorted candidate
-  int32_t* spl;        // positions of candidates with cand_spec = 1, ascending
+  uint64_t* cand_in;   // merge candidates, see cand_key(), at session offset + point time (~0 none)
+  uint64_t* cand_out;  // keys of the acting ones, in order
+  int32_t* cand_nbr;   // per candidate record: 6 eligible neighbour ids at its time
+  int32_t* spl;        // records (cand_nbr) of the candidates that act on the pre-replay state, in order
   int32_t* seg_ct;     // per segment: its candidate times (up to 7, ascending)
   int32_t* seg_nct;
   int2* seg_nbr;       // per segment: the six neighbour voxels, see nbr_eligible()
@@ -1081,9 +1079,8 @@ __global__ void __launch_bounds__(kMapThreads) k_create_init(const MapDev* maps,
         }
       }
       // the merge stage's per-point slots start empty (k_candidates fills
-      // them; k_create_evict kept its touched entries in cand_in before)
+      // them; k_create_evict kept its touched entries there before)
       b.cand_in[p] = ~0ull;
-      b.cand_spec[p] = 0;
       if (p < nseg) {
         const int32_t vid = b.seg_old[p];
         if (vid >= 0) {
@@ -1969,48 +1966,6 @@ __global__ void k_lru_append(OutLru out, BatchBufs b) {
   const int nsel = b.cnt[2];
   VMP_GRID_LOOP(r, nsel) out(r, b.sel[r], b.flags[b.sel[r]]);
 }
-
-// start of each session's candidates in the sorted candidate list, and
-// their total (cnt[3])
-// (one workgroup: every session's count is loaded at once, then an
-// exclusive scan in LDS, kCsThreads sessions per round)
-constexpr int kCsThreads = 256;
-__device__ inline void cand_starts_block(const MapDev* maps, int nsess, const BatchBufs& b) {
-  __shared__ int sc[kCsThreads];
-  __shared__ int carry;
-  const int tid = threadIdx.x;
-  if (tid == 0) carry = 0;
-  for (int s0 = 0; s0 < nsess; s0 += kCsThreads) {
-    const int s = s0 + tid;
-    const int v = s < nsess ? maps[s].ctr->ncand : 0;
-    sc[tid] = v;
-    __syncthreads();
-    for (int o = 1; o < kCsThreads; o <<= 1) {  // inclusive Hillis-Steele scan
-      const int u = tid >= o ? sc[tid - o] : 0;
-      __syncthreads();
-      sc[tid] += u;
-      __syncthreads();
-    }
-    if (s < nsess) b.cand_start[s] = carry + sc[tid] - v;
-    __syncthreads();
-    if (tid == kCsThreads - 1) carry += sc[tid];
-    __syncthreads();
-  }
-  if (tid == 0) b.cnt[3] = carry;
-}
-__global__ void __launch_bounds__(kCsThreads) k_cand_starts(const MapDev* maps, int nsess, BatchBufs b) {
-  cand_starts_block(maps, nsess, b);
-}
-// the same as the tail of the candidate compaction (a block of kCsThreads)
-struct TailCandStarts {
-  const MapDev* maps;
-  int nsess;
-  BatchBufs b;
-  static constexpr bool kActive = true;
-  __device__ void at_tile(int, int, int, const int32_t (&)[kPrimIpt]) const {}
-  __device__ void operator()(int) const { cand_starts_block(maps, nsess, b); }
-};
-
 
 // ---------------------------------------------------- housekeeping -----
 // Hash rebuild of the listed sessions (grid row y: session l.s[y] of the
