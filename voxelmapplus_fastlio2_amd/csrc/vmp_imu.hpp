@@ -6,11 +6,11 @@
 //
 //   k_imu_init      one thread per session: means of the cached samples,
 //                   gravity alignment, bg, P
-//   k_imu_predict   one 64-lane workgroup per session: the package's IMU
-//                   pairs in order (per-step increments across lanes, the
-//                   state chain on one lane, P = F P F^T + G Q G^T over the
-//                   structurally non-zero products across lanes); the IMU
-//                   pose table and its running minimum of offsets
+//   k_imu_predict   one workgroup per session: the package's IMU pairs in
+//                   order (per-step increments across lanes, the state chain,
+//                   P = F P F^T + G Q G^T over the structurally non-zero
+//                   products, a column of P per lane); the IMU pose table and
+//                   its running minimum of offsets
 //   k_undistort     one lane per point: the pose interval it falls in (a
 //                   binary search over the running minimum, which is the
 //                   interval the reference's backward walk reaches it in),
@@ -180,45 +180,48 @@ __global__ void k_imu_init(ImuDev* imu, FilterDev* f, const double* t, const dou
 }
 
 // IMU propagation of one package (IESKF::predict per IMU pair, ieskf.cpp:
-// 83-111, from lio_builder.cpp:80-119): one four-wave workgroup per session,
-// the pairs in chunks of up to 64 steps, each chunk in four phases (A-C on
-// the first wave's lanes, D on all four waves).
-//   A  lanes: each step's input (mid-point acc and gyro, dt), its rotation
-//      increment exp((gyro - bg) dt) and -Jr dt (IMU data and the biases,
-//      which do not change while a package is propagated)
+// 83-111, from lio_builder.cpp:80-119): one workgroup per session, the pairs
+// in chunks of up to 64 steps, each chunk in four phases
+//   A  lanes of the first wave: each step's input (mid-point acc and gyro,
+//      dt), its rotation increment exp((gyro - bg) dt) and -Jr dt (IMU data
+//      and the biases, which do not change while a package is propagated)
 //   B  the first wave: the state chain in order (velocity, position,
-//      rotation; the rotation's entries cross lanes by shuffles), keeping the
-//      rotation before each step and the state after it
-//   C  lanes: each step's blocks that depend on the rotation before it,
-//      (-rot hat(acc - ba)) dt and (-rot) dt, and the IMU pose table entry
-//      at the step's tail
-//   D  all waves, step after step: P = F P F^T + G Q G^T.  F is the identity
-//      except in rows 0-5, 12-14 and 21-22, so F P is formed for those rows
-//      only (its other rows are rows of P) and (F P) F^T for those columns
-//      only (its other columns are columns of F P).  Every sum runs over the
-//      structurally non-zero terms in ascending index order, the order of
-//      the dense product's sums; G Q G^T adds to the diagonal blocks 3-5,
-//      12-14, 15-17 and 18-20.
+//      rotation), in registers, the same in every lane, keeping the rotation
+//      before each step and the state after it
+//   C  its lanes: each step's blocks that depend on the rotation before it,
+//      (-rot hat(acc - ba)) dt and (-rot) dt; the third wave, at the end:
+//      the IMU pose table entry at the step's tail
+//   D  the second wave, step after step: P = F P F^T + G Q G^T.  F is the
+//      identity except in rows 0-5, 12-14 and 21-22, so only those rows (then
+//      columns) change; G Q G^T adds to the diagonal blocks 3-5, 12-14, 15-17
+//      and 18-20.
 // exp(-w) is exp(w)^T bit for bit (the quaternion form only flips signs),
 // so F's rotation block is the transpose of the step's increment.
 constexpr int kPredChunk = 64;
-constexpr int kFpRows = 11;  // rows of F that differ from the identity's
-__device__ inline int fp_slot(int r) { return r < 6 ? r : (r >= 12 && r < 15) ? r - 6 : r >= 21 ? r - 12 : -1; }
-__device__ inline int fp_row(int slot) { return slot < 6 ? slot : slot < 9 ? slot + 6 : slot + 12; }
-// G's row groups: rows 3-5 (ng), 12-14 (na), 15-17 (nbg), 18-20 (nba)
-__device__ inline int g_group(int r) {
-  return (r >= 3 && r < 6) ? 0 : (r >= 12 && r < 15) ? 1 : (r >= 15 && r < 18) ? 2 : (r >= 18 && r < 21) ? 3 : -1;
-}
+constexpr int kPredThreads = 192;  // three waves
+constexpr int kPredBlk = 4;        // steps between two barriers of phases B-D
+constexpr int kFpRows = 11;  // rows of F that differ from the identity's: 0-5, 12-14, 21-22
 
+// one step: F's blocks (in this order from the front), then G Q G^T's and the
+// inputs
+struct PredF {
+  double dt;
+  double E[9];   // exp((gyro - bg) dt), row-major
+  double J[9];   // -Jr((gyro - bg) dt) dt (F and G)
+  double A[9];   // (-rot hat(acc - ba)) dt
+  double Rd[9];  // (-rot) dt (F and G)
+  double md[6];  // Mx dt
+};
+struct PredStep {
+  PredF f;
+  double GJ[9], GR[9];  // the blocks of G Q G^T at 3-5 and 12-14
+  double d2, d3;        // its diagonal at 15-17 and 18-20
+  double tt;
+  double ab[3], gyro[3];  // acc - ba, gyro
+};
 struct PredShared {
-  double P[529];            // row-major
-  double FP[kFpRows * 23];  // rows fp_row(0..10) of F P
-  double E[kPredChunk][9];  // per step of the chunk: exp((gyro - bg) dt), row-major
-  double J[kPredChunk][9];  // -Jr((gyro - bg) dt) dt (F and G)
-  double A[kPredChunk][9];  // (-rot hat(acc - ba)) dt
-  double Rd[kPredChunk][9]; // (-rot) dt (F and G)
-  double acc[kPredChunk][3], gyro[kPredChunk][3];
-  double dt[kPredChunk], tt[kPredChunk];
+  PredStep s[kPredChunk];
+  double T[23][25];             // F P crossing the lanes (odd rows: no bank conflicts)
   double R[kPredChunk + 1][9];  // rotation before each step, and after the last
   double vel[kPredChunk + 1][3], pos[kPredChunk + 1][3];  // after step j at j + 1
   double Mx[6], NM[4], q[4];
@@ -226,197 +229,82 @@ struct PredShared {
   vmp_state sx;
 };
 
-// phase D for step j of the chunk, P in place, on the block's four waves.
-// F P: lane c of every wave holds column c of P (the entries its rows need)
-// and forms column c of some of the 11 non-identity rows of F P: wave 0 rows
-// 0-2, wave 1 rows 3-5, wave 2 rows 12-13, wave 3 rows 14, 21 and 22.
-// (F P) F^T + G Q G^T: lane r of every wave reads row r of F P (a row of P
-// for an identity row of F) into registers; after a barrier each wave
-// rewrites its columns of row r of P (wave 0 columns 0-2, wave 1 columns 3-5,
-// wave 2 columns 12-13, wave 3 columns 14, 21, 22), wave 0 also the identity
-// columns of a non-identity row (from F P) and the diagonal of G Q G^T's
-// identity blocks.  Every entry is the same expression, summed in the same
-// order, whichever wave forms it.
-constexpr int kPredThreads = 256;
-__device__ inline void predict_cov_step(PredShared& S, int j, int w, int l) {
-  double* P = S.P;
-  const double dt = S.dt[j];
-  const double* E = S.E[j];
-  const double* Jd = S.J[j];
-  const double* Ad = S.A[j];
-  const double* Rd = S.Rd[j];
-  double* fp = S.FP;
-  if (l < 23) {  // F P
-    const int c = l;
-    if (w == 0) {  // rows 0-2
+// F u for the rows of F that differ from the identity's, sums over the
+// structurally non-zero terms in ascending order
+__device__ inline void predict_rows(const PredF& f, const double NM[4], const double u[23], double v[kFpRows]) {
 #pragma unroll
-      for (int r = 0; r < 3; ++r) {
-        double s = P[r * 23 + c];
-        s += dt * P[(12 + r) * 23 + c];
-        fp[r * 23 + c] = s;
-      }
-    } else if (w == 1) {  // rows 3-5: exp(-w) row i = exp(w) column i
-      double p[6];
+  for (int r = 0; r < 3; ++r) v[r] = fma(f.dt, u[12 + r], u[r]);
 #pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        p[t] = P[(3 + t) * 23 + c];
-        p[3 + t] = P[(15 + t) * 23 + c];
-      }
+  for (int i = 0; i < 3; ++i) {  // exp(-w) row i = exp(w) column i
+    double s = f.E[i] * u[3];
+    s = fma(f.E[3 + i], u[4], s);
+    s = fma(f.E[6 + i], u[5], s);
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        double s = E[i] * p[0];
-        s += E[3 + i] * p[1];
-        s += E[6 + i] * p[2];
-        s += Jd[i * 3] * p[3];
-        s += Jd[i * 3 + 1] * p[4];
-        s += Jd[i * 3 + 2] * p[5];
-        fp[(3 + i) * 23 + c] = s;
-      }
-    } else {  // rows 12-14 (waves 2, 3) and 21-22 (wave 3)
-      const double md[6] = {S.Mx[0] * dt, S.Mx[1] * dt, S.Mx[2] * dt, S.Mx[3] * dt, S.Mx[4] * dt, S.Mx[5] * dt};
-      double p[3], q[3], u[5];
-#pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        p[t] = P[(3 + t) * 23 + c];
-        q[t] = P[(12 + t) * 23 + c];
-      }
-#pragma unroll
-      for (int t = 0; t < 5; ++t) u[t] = P[(18 + t) * 23 + c];
-      const int i0 = w == 2 ? 0 : 2, i1 = w == 2 ? 2 : 3;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {  // rows 12-14
-        if (i < i0 || i >= i1) continue;
-        double s = Ad[i * 3] * p[0];
-        s += Ad[i * 3 + 1] * p[1];
-        s += Ad[i * 3 + 2] * p[2];
-        s += q[i];
-        s += Rd[i * 3] * u[0];
-        s += Rd[i * 3 + 1] * u[1];
-        s += Rd[i * 3 + 2] * u[2];
-        s += md[i * 2] * u[3];
-        s += md[i * 2 + 1] * u[4];
-        fp[(6 + i) * 23 + c] = s;
-      }
-      if (w == 3) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {  // rows 21-22
-          double s = S.NM[i * 2] * u[3];
-          s += S.NM[i * 2 + 1] * u[4];
-          fp[(9 + i) * 23 + c] = s;
-        }
-      }
-    }
+    for (int t = 0; t < 3; ++t) s = fma(f.J[i * 3 + t], u[15 + t], s);
+    v[3 + i] = s;
   }
-  __syncthreads();
-  // (F P) F^T + G Q G^T: every wave first reads the entries of row r it needs
-  const int r = l;
-  const int rs = r < 23 ? fp_slot(r) : -1;
-  const double* fr = rs >= 0 ? &S.FP[rs * 23] : &P[(r < 23 ? r : 0) * 23];
-  double f[11];
-  if (r < 23) {
-    if (w == 0) {
 #pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        f[t] = fr[t];
-        f[3 + t] = fr[12 + t];
-      }
-    } else if (w == 1) {
+  for (int i = 0; i < 3; ++i) {
+    double s = f.A[i * 3] * u[3];
+    s = fma(f.A[i * 3 + 1], u[4], s);
+    s = fma(f.A[i * 3 + 2], u[5], s);
+    s += u[12 + i];
 #pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        f[t] = fr[3 + t];
-        f[3 + t] = fr[15 + t];
-      }
-    } else {
-#pragma unroll
-      for (int t = 0; t < 3; ++t) {
-        f[t] = fr[3 + t];
-        f[3 + t] = fr[12 + t];
-      }
-#pragma unroll
-      for (int t = 0; t < 5; ++t) f[6 + t] = fr[18 + t];
-    }
+    for (int t = 0; t < 3; ++t) s = fma(f.Rd[i * 3 + t], u[18 + t], s);
+    s = fma(f.md[i * 2], u[21], s);
+    v[6 + i] = fma(f.md[i * 2 + 1], u[22], s);
   }
-  __syncthreads();  // every read of P's row r comes before the writes below
-  if (r < 23) {
-    double* pr = &P[r * 23];
-    const int gr = g_group(r);
-    if (w == 0) {  // columns 0-2
 #pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        double s = f[c];
-        s += f[3 + c] * dt;
-        pr[c] = s;
-      }
-      if (rs >= 0) {  // identity columns of a non-identity row: F P's entries
+  for (int i = 0; i < 2; ++i) v[9 + i] = fma(NM[i * 2 + 1], u[22], NM[i * 2] * u[21]);
+}
+__device__ inline void put_rows(double u[23], const double v[kFpRows]) {
 #pragma unroll
-        for (int c = 6; c < 12; ++c) pr[c] = fr[c];
+  for (int r = 0; r < 6; ++r) u[r] = v[r];
 #pragma unroll
-        for (int c = 15; c < 21; ++c) pr[c] = fr[c];
-      } else if (gr >= 2) {  // identity row and column: only G Q G^T's diagonal
-        pr[r] = pr[r] + (dt * S.q[gr]) * dt;
-      }
-    } else if (w == 1) {  // columns 3-5 (+ G Q G^T's block 3-5)
-      double o[3];
+  for (int r = 0; r < 3; ++r) u[12 + r] = v[6 + r];
+  u[21] = v[9];
+  u[22] = v[10];
+}
+
+// Phase D, one step on one wave: lane c (< 23) holds column c of P in u and
+// leaves with row c of the step's P.  F P needs a lane's own column only; it
+// is transposed through LDS, and F applied to row c of F P is row c of
+// F P F^T.  The next step takes the rows as columns (it forms the transpose).
+__device__ inline void predict_cov_step(PredShared& S, const PredStep& g, const PredF& f, const double NM[4],
+                                        double u[23], int c) {
+  double v[kFpRows];
+  predict_rows(f, NM, u, v);
+  put_rows(u, v);
+  if (c < 23) {
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        double s = f[0] * E[i];
-        s += f[1] * E[3 + i];
-        s += f[2] * E[6 + i];
-        s += f[3] * Jd[i * 3];
-        s += f[4] * Jd[i * 3 + 1];
-        s += f[5] * Jd[i * 3 + 2];
-        o[i] = s;
-      }
-      if (gr == 0) {
-        const double q = S.q[0];
-        const double* Gr = &Jd[(r - 3) * 3];
+    for (int r = 0; r < 23; ++r) S.T[r][c] = u[r];
+  }
+  const bool b0 = c >= 3 && c < 6, b1 = c >= 12 && c < 15;
+  const double* gb = b0 ? g.GJ + (c - 3) : g.GR + (b1 ? c - 12 : 0);
+  const double g0 = gb[0], g1 = gb[3], g2 = gb[6];
+  const double d2 = g.d2, d3 = g.d3;
+  wave_lds_sync();
+  const int row = min(c, 22);
 #pragma unroll
-        for (int i = 0; i < 3; ++i) {
-          double g = (Gr[0] * q) * Jd[i * 3];
-          g += (Gr[1] * q) * Jd[i * 3 + 1];
-          g += (Gr[2] * q) * Jd[i * 3 + 2];
-          o[i] = o[i] + g;
-        }
-      }
+  for (int k = 0; k < 23; ++k) u[k] = S.T[row][k];
+  wave_lds_sync();
+  predict_rows(f, NM, u, v);
+  put_rows(u, v);
+  const double gv[3] = {g0, g1, g2};
 #pragma unroll
-      for (int i = 0; i < 3; ++i) pr[3 + i] = o[i];
-    } else {  // columns 12-13 (wave 2), 14, 21, 22 (wave 3) (+ G Q G^T's block 12-14)
-      const double md[6] = {S.Mx[0] * dt, S.Mx[1] * dt, S.Mx[2] * dt, S.Mx[3] * dt, S.Mx[4] * dt, S.Mx[5] * dt};
-      const int i0 = w == 2 ? 0 : 2, i1 = w == 2 ? 2 : 3;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        if (i < i0 || i >= i1) continue;
-        double s = f[0] * Ad[i * 3];
-        s += f[1] * Ad[i * 3 + 1];
-        s += f[2] * Ad[i * 3 + 2];
-        s += f[3 + i];
-        s += f[6] * Rd[i * 3];
-        s += f[7] * Rd[i * 3 + 1];
-        s += f[8] * Rd[i * 3 + 2];
-        s += f[9] * md[i * 2];
-        s += f[10] * md[i * 2 + 1];
-        if (gr == 1) {
-          const double q = S.q[1];
-          const double* Gr = &Rd[(r - 12) * 3];
-          double g = (Gr[0] * q) * Rd[i * 3];
-          g += (Gr[1] * q) * Rd[i * 3 + 1];
-          g += (Gr[2] * q) * Rd[i * 3 + 2];
-          s = s + g;
-        }
-        pr[12 + i] = s;
-      }
-      if (w == 3) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          double s = f[9] * S.NM[i * 2];
-          s += f[10] * S.NM[i * 2 + 1];
-          pr[21 + i] = s;
-        }
-      }
-    }
+  for (int i = 0; i < 3; ++i) {
+    u[3 + i] += b0 ? gv[i] : 0.0;
+    u[12 + i] += b1 ? gv[i] : 0.0;
+    u[15 + i] += c == 15 + i ? d2 : 0.0;
+    u[18 + i] += c == 18 + i ? d3 : 0.0;
   }
 }
 
+// Bound by the chain of its steps on one compute unit (21 for a 10 Hz sweep
+// with 200 Hz IMU).  With P in registers a step of phase D takes one exchange
+// through LDS and no barrier, with the state chain in every lane's registers
+// a step of phase B takes no shuffle, and phase D follows phases B and C on
+// another wave, kPredBlk steps behind: 44 us -> 26.
 __global__ void __launch_bounds__(kPredThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 k_imu_predict(const PreJob* jobs, int nsess) {
   if (int(blockIdx.x) >= nsess) return;
@@ -424,21 +312,32 @@ k_imu_predict(const PreJob* jobs, int nsess) {
   ImuDev* im = Jb.imu;
   const ImuPkg* pkg = Jb.pkg;
   FilterDev* f = Jb.f;
-  const int lane = threadIdx.x;  // phases A-C and the set-up run on the first wave's lanes
+  const int lane = threadIdx.x & 63;
+  const int wv = threadIdx.x >> 6;  // the first wave carries the state, the second P, the third the pose table
   __shared__ PredShared S;
-  for (int i = lane; i < 529; i += kPredThreads) S.P[(i % 23) * 23 + i / 23] = f->P[i];  // column-major -> rows
-  load_state(f->x, S.sx, lane);
-  if (lane < 4) S.q[lane] = im->q[lane];
-  __syncthreads();
+  double u[23];
+#pragma unroll
+  for (int k = 0; k < 23; ++k) u[k] = wv == 1 && lane < 23 ? f->P[lane * 23 + k] : 0.0;
+  load_state(f->x, S.sx, threadIdx.x);
+  if (threadIdx.x < 4) S.q[threadIdx.x] = im->q[threadIdx.x];
   const int m = pkg->m;
   const double lce = im->last_cloud_end;
   const double cstart = pkg->cloud_start;
   // active IMU pairs (head k-1 or last_imu, tail k) are those whose tail is
   // not before the last scan end: a prefix of the ascending samples is skipped
   int k0 = 0;
-  while (k0 < m && pkg->s[k0][0] < lce) ++k0;
+  while (k0 < m) {
+    const bool stop = k0 + lane < m && !(pkg->s[k0 + lane][0] < lce);
+    const uint64_t bal = __ballot(stop);
+    if (bal) {
+      k0 += __ffsll((unsigned long long)bal) - 1;
+      break;
+    }
+    k0 = min(m, k0 + 64);
+  }
   const int nsteps = (m - k0) + 1;  // the pairs, then the step to the sweep's end
-  if (lane == 0) {
+  __syncthreads();
+  if (threadIdx.x == 128) {
     double Bx[6];
     getBx_d(S.sx.g, Bx);
     const D33 hg = hat_d(S.sx.g);
@@ -496,122 +395,170 @@ k_imu_predict(const PreJob* jobs, int nsess) {
       dt = pkg->cloud_end - imu_end;
     }
   };
+  auto gq = [](const double* G, double q, double* out) {  // G q G^T of a 3x3 block
+    for (int r = 0; r < 3; ++r)
+      for (int i = 0; i < 3; ++i) {
+        double g = (G[r * 3] * q) * G[i * 3];
+        g += (G[r * 3 + 1] * q) * G[i * 3 + 1];
+        g += (G[r * 3 + 2] * q) * G[i * 3 + 2];
+        out[r * 3 + i] = g;
+      }
+  };
+  D33 R = d33_from_cm(S.sx.rot);
+  double vel[3], pos[3], g[3];
+  for (int c = 0; c < 3; ++c) {
+    g[c] = S.sx.g[c];
+    vel[c] = S.sx.vel[c];
+    pos[c] = S.sx.pos[c];
+  }
   int np = 1;  // pose table entries
   for (int c0 = 0; c0 < nsteps; c0 += kPredChunk) {
     const int cn = min(kPredChunk, nsteps - c0);
-    if (lane < cn) {  // A
-      double a[3], g[3], dt, tt;
-      step_input(c0 + lane, a, g, dt, tt);
+    if (wv == 0 && lane < cn) {  // A
+      PredStep& s = S.s[lane];
+      double a[3], w[3], dt, tt;
+      step_input(c0 + lane, a, w, dt, tt);
       double wdt[3];
-      for (int c = 0; c < 3; ++c) wdt[c] = dt * (g[c] - S.sx.bg[c]);
+      for (int c = 0; c < 3; ++c) wdt[c] = dt * (w[c] - S.sx.bg[c]);
       const D33 E = so3_exp_d(wdt);
       const D33 Jr = d33_t(left_jac_d(wdt));
+      double J[9];
       for (int i = 0; i < 9; ++i) {
-        S.E[lane][i] = E.m[i];
-        S.J[lane][i] = ((-1.0) * Jr.m[i]) * dt;
+        s.f.E[i] = E.m[i];
+        s.f.J[i] = J[i] = ((-1.0) * Jr.m[i]) * dt;
       }
+      gq(J, S.q[0], s.GJ);
       for (int c = 0; c < 3; ++c) {
-        S.acc[lane][c] = a[c];
-        S.gyro[lane][c] = g[c];
+        s.ab[c] = a[c] - S.sx.ba[c];
+        s.gyro[c] = w[c];
       }
-      S.dt[lane] = dt;
-      S.tt[lane] = tt;
+      s.f.dt = dt;
+      s.tt = tt;
+      s.d2 = (dt * S.q[2]) * dt;
+      s.d3 = (dt * S.q[3]) * dt;
     }
     __syncthreads();
-    {  // B: x += delta step after step, the rotation in lanes 0-8 (entry
-       // lane), velocity and position in lanes 0-2; the blocks of a step come
-       // from the state before it
-      vmp_state& x = S.sx;
-      double rv = 0.0, vel = 0.0, pos = 0.0;
-      if (lane < 9) rv = x.rot[(lane % 3) * 3 + lane / 3];  // column-major storage
-      if (lane < 3) {
-        vel = x.vel[lane];
-        pos = x.pos[lane];
-      }
-      if (lane < 64) {  // the first wave alone: the rotation's entries cross lanes by shuffles
-        const int r = lane < 9 ? lane / 3 : 0, c = lane % 3, vr = lane < 3 ? lane : 0;
-        for (int j = 0; j < cn; ++j) {
-          if (lane < 9) S.R[j][lane] = rv;  // the rotation before step j (lane k: entry k, row-major)
-          const double Rv0 = __shfl(rv, vr * 3, 64), Rv1 = __shfl(rv, vr * 3 + 1, 64), Rv2 = __shfl(rv, vr * 3 + 2, 64);
-          const double Rr0 = __shfl(rv, r * 3, 64), Rr1 = __shfl(rv, r * 3 + 1, 64), Rr2 = __shfl(rv, r * 3 + 2, 64);
-          const double* E = S.E[j];
-          if (lane < 3) {
-            const double dt = S.dt[j];
-            const double ab0 = S.acc[j][0] - x.ba[0], ab1 = S.acc[j][1] - x.ba[1], ab2 = S.acc[j][2] - x.ba[2];
-            double ra = Rv0 * ab0;
-            ra += Rv1 * ab1;
-            ra += Rv2 * ab2;
-            const double dvel = dt * (ra + x.g[lane]);
-            const double dpos = dt * vel;
-            pos = pos + dpos;
-            vel = vel + dvel;
-            S.vel[j + 1][lane] = vel;
-            S.pos[j + 1][lane] = pos;
+    const double NM[4] = {S.NM[0], S.NM[1], S.NM[2], S.NM[3]};
+    for (int j0 = 0; j0 < cn + kPredBlk; j0 += kPredBlk) {
+      if (wv == 0 && j0 < cn) {
+        const int j1 = min(j0 + kPredBlk, cn);
+        for (int j = j0; j < j1; ++j) {  // B: x += delta step after step
+          const PredStep& s = S.s[j];
+          const double dt = s.f.dt, ab0 = s.ab[0], ab1 = s.ab[1], ab2 = s.ab[2];
+          double E[9];
+#pragma unroll
+          for (int i = 0; i < 9; ++i) E[i] = s.f.E[i];
+          if (lane == 0)
+            for (int i = 0; i < 9; ++i) S.R[j][i] = R.m[i];  // the rotation before step j
+#pragma unroll
+          for (int r = 0; r < 3; ++r) {
+            double ra = R.m[r * 3] * ab0;
+            ra += R.m[r * 3 + 1] * ab1;
+            ra += R.m[r * 3 + 2] * ab2;
+            const double dvel = dt * (ra + g[r]);
+            pos[r] = pos[r] + dt * vel[r];
+            vel[r] = vel[r] + dvel;
           }
-          if (lane < 9) {
-            double v = Rr0 * E[c];
-            v += Rr1 * E[3 + c];
-            v += Rr2 * E[6 + c];
-            rv = v;
-          }
+          if (lane == 0)
+            for (int r = 0; r < 3; ++r) {
+              S.vel[j + 1][r] = vel[r];
+              S.pos[j + 1][r] = pos[r];
+            }
+          D33 n;
+#pragma unroll
+          for (int r = 0; r < 3; ++r)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              double v = R.m[r * 3] * E[c];
+              v += R.m[r * 3 + 1] * E[3 + c];
+              v += R.m[r * 3 + 2] * E[6 + c];
+              n.m[r * 3 + c] = v;
+            }
+          R = n;
         }
-        if (lane < 9) S.R[cn][lane] = rv;
+        if (lane == 0)
+          for (int i = 0; i < 9; ++i) S.R[j1][i] = R.m[i];
+        wave_lds_sync();
+        if (lane < j1 - j0) {  // C: the step's blocks
+          const int j = j0 + lane;
+          PredStep& s = S.s[j];
+          const double dt = s.f.dt, ab[3] = {s.ab[0], s.ab[1], s.ab[2]};
+          D33 nrot;
+          for (int i = 0; i < 9; ++i) nrot.m[i] = (-1.0) * S.R[j][i];
+          const D33 Ah = d33_mul(nrot, hat_d(ab));
+          double Rd[9];
+          for (int i = 0; i < 9; ++i) {
+            s.f.A[i] = Ah.m[i] * dt;
+            s.f.Rd[i] = Rd[i] = nrot.m[i] * dt;
+          }
+          for (int i = 0; i < 6; ++i) s.f.md[i] = S.Mx[i] * dt;
+          gq(Rd, S.q[1], s.GR);
+        }
+      } else if (wv == 1 && j0 > 0) {  // D, the steps before
+        const int j1 = min(j0, cn);
+        for (int j = j0 - kPredBlk; j < j1; ++j) {
+          const PredF f = S.s[j].f;
+          predict_cov_step(S, S.s[j], f, NM, u, lane);
+        }
       }
       __syncthreads();
-      if (lane < 9) x.rot[(lane % 3) * 3 + lane / 3] = rv;
-      if (lane < 3) {
-        x.vel[lane] = vel;
-        x.pos[lane] = pos;
-      }
     }
-    __syncthreads();
-    if (lane < cn) {  // C
+    if (wv == 2 && lane < cn && c0 + lane != nsteps - 1) {  // the IMU pose at the pair's tail
       const int j = lane;
-      const double dt = S.dt[j];
-      const double ab[3] = {S.acc[j][0] - S.sx.ba[0], S.acc[j][1] - S.sx.ba[1], S.acc[j][2] - S.sx.ba[2]};
-      D33 nrot, rot;
-      for (int i = 0; i < 9; ++i) {
-        rot.m[i] = S.R[j][i];
-        nrot.m[i] = (-1.0) * rot.m[i];
+      const PredStep& s = S.s[j];
+      D33 rn;
+      for (int i = 0; i < 9; ++i) rn.m[i] = S.R[j + 1][i];
+      const D3 rb = d33_mulv(rn, D3{{s.ab[0], s.ab[1], s.ab[2]}});
+      double* p = im->pose[np + j];
+      p[0] = s.tt - cstart;
+      S.off[np + j] = p[0];
+      double la[3], lg[3];
+      for (int c = 0; c < 3; ++c) {
+        lg[c] = s.gyro[c] - S.sx.bg[c];
+        la[c] = rb.v[c] + S.sx.g[c];
+        p[1 + c] = la[c];
+        p[4 + c] = lg[c];
+        p[7 + c] = S.vel[j + 1][c];
+        p[10 + c] = S.pos[j + 1][c];
       }
-      const D33 Ah = d33_mul(nrot, hat_d(ab));
-      for (int i = 0; i < 9; ++i) {
-        S.A[j][i] = Ah.m[i] * dt;
-        S.Rd[j][i] = nrot.m[i] * dt;
-      }
-      if (c0 + j != nsteps - 1) {  // the IMU pose at the pair's tail
-        D33 rn;
-        for (int i = 0; i < 9; ++i) rn.m[i] = S.R[j + 1][i];
-        const D3 rb = d33_mulv(rn, D3{{ab[0], ab[1], ab[2]}});
-        double* p = im->pose[np + j];
-        p[0] = S.tt[j] - cstart;
-        S.off[np + j] = p[0];
-        double la[3], lg[3];
+      for (int c = 0; c < 9; ++c) p[13 + c] = rn.m[c];
+      if (c0 + j == nsteps - 2)  // the last pair: LIODataGroup's last acc / gyro
         for (int c = 0; c < 3; ++c) {
-          lg[c] = S.gyro[j][c] - S.sx.bg[c];
-          la[c] = rb.v[c] + S.sx.g[c];
-          p[1 + c] = la[c];
-          p[4 + c] = lg[c];
-          p[7 + c] = S.vel[j + 1][c];
-          p[10 + c] = S.pos[j + 1][c];
+          im->last_acc[c] = la[c];
+          im->last_gyro[c] = lg[c];
         }
-        for (int c = 0; c < 9; ++c) p[13 + c] = rn.m[c];
-        if (c0 + j == nsteps - 2)  // the last pair: LIODataGroup's last acc / gyro
-          for (int c = 0; c < 3; ++c) {
-            im->last_acc[c] = la[c];
-            im->last_gyro[c] = lg[c];
-          }
-      }
-    }
-    for (int j = 0; j < cn; ++j) {  // D
-      __syncthreads();
-      predict_cov_step(S, j, lane >> 6, lane & 63);
     }
     np += (c0 + cn == nsteps) ? cn - 1 : cn;
-    __syncthreads();
+    if (c0 + cn < nsteps) __syncthreads();
   }
-  for (int i = lane; i < 529; i += kPredThreads) f->P[i] = S.P[(i % 23) * 23 + i / 23];
-  if (lane == 0) {
+  if (wv == 2) {
+    wave_lds_sync();
+    if (lane == 0) im->npose = np;
+    // running minimum of the offsets of the interval heads (entries 0..np-2)
+    double mn = 1e300;
+    for (int i0 = (np - 2) & ~63; i0 >= 0; i0 -= 64) {
+      const int i = i0 + lane;
+      double v = i <= np - 2 ? S.off[i] : 1e300;
+      for (int o = 1; o < 64; o <<= 1) {
+        const double w = __shfl_down(v, o, 64);
+        if (lane + o < 64) v = fmin(v, w);
+      }
+      v = fmin(mn, v);
+      if (i <= np - 2) im->pose_min[i] = v;
+      mn = __shfl(v, 0, 64);
+    }
+    return;
+  }
+  if (wv == 1 && lane < 23) {
+#pragma unroll
+    for (int k = 0; k < 23; ++k) f->P[nsteps & 1 ? k * 23 + lane : lane * 23 + k] = u[k];
+  }
+  if (threadIdx.x == 0) {
+    d33_to_cm(R, S.sx.rot);
+    for (int c = 0; c < 3; ++c) {
+      S.sx.vel[c] = vel[c];
+      S.sx.pos[c] = pos[c];
+    }
     f->x = S.sx;
     if (m > 0) {
       im->last_imu_t = pkg->s[m - 1][0];
@@ -621,13 +568,6 @@ k_imu_predict(const PreJob* jobs, int nsess) {
       }
     }
     im->last_cloud_end = pkg->cloud_end;
-    im->npose = np;
-    // running minimum of the offsets of the interval heads (entries 0..np-2)
-    double mn = 1e300;
-    for (int i = np - 2; i >= 0; --i) {
-      mn = fmin(mn, S.off[i]);
-      im->pose_min[i] = mn;
-    }
   }
 }
 
