@@ -235,7 +235,18 @@ __device__ inline int32_t hash_find_or_insert(HashEntry* table, uint32_t mask, u
                                               int* inserted = nullptr) {
   const HashSeq seq = hash_seq(key);
   uint32_t h = hash_home(seq, mask);
-  for (uint32_t probe = 0; probe <= mask;) {
+  // The probes up to the first empty slot on loads that the caches may serve:
+  // no kernel that inserts removes or replaces a key, so only a slot seen
+  // empty can hold something else by now, and is looked at again below.
+  uint32_t probe = 0;
+  while (probe <= mask) {
+    const unsigned long long k = __hip_atomic_load(reinterpret_cast<unsigned long long*>(&table[h].key),
+                                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (k == key) return int32_t(h);
+    if (k == kKeyEmpty) break;
+    h = hash_probe(seq, ++probe, mask);
+  }
+  while (probe <= mask) {
     unsigned long long* kp = reinterpret_cast<unsigned long long*>(&table[h].key);
     unsigned long long k = __hip_atomic_load(kp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (k == key) return int32_t(h);
@@ -493,6 +504,11 @@ __global__ void k_ins_keys(const MapDev* maps, const SessInfo* si, int nsess, Ba
     b.cnt[6] = 0;
   }
   VMP_GRID_LOOP(s, nsess) begin_scan(maps[s].ctr);
+  // claimed slots: one atomic per block for a session alone (one per wave of a
+  // 120,000-point scan queued up behind each other), else per wave and session
+  __shared__ int claimed;
+  if (threadIdx.x == 0) claimed = 0;
+  __syncthreads();
   VMP_UNIFORM_LOOP(g, valid, b.ntot) {
     int ins = 0;
     const int s = valid ? sess_of(si, nsess, g) : 0;
@@ -516,8 +532,15 @@ __global__ void k_ins_keys(const MapDev* maps, const SessInfo* si, int nsess, Ba
     b.sval_in[g] = g;
     b.flags[g] = 0;
     }
-    wave_fetch_add(&maps[s].ctr->used_entries, ins);
+    if (nsess > 1) {
+      wave_fetch_add(&maps[s].ctr->used_entries, ins);
+    } else {
+      const uint64_t bal = __ballot(ins);
+      if ((threadIdx.x & 63) == 0 && bal) atomicAdd(&claimed, __popcll(bal));
+    }
   }
+  __syncthreads();
+  if (threadIdx.x == 0 && claimed) atomicAdd(&maps[0].ctr->used_entries, claimed);
 }
 
 // ------------------------------------------------------------------ K3 ----
