@@ -206,6 +206,9 @@ __device__ inline void merge_fuse(double* pv, double* pn) {
 __global__ void k_candidates(const MapDev* maps, const SessInfo* si, BatchBufs b) {
   const int nseg = b.cnt[0];
   const MapDev m0 = maps[0];  // a one-session step reads its map's record once
+  __shared__ int cands;       // and adds its candidates once per block
+  if (threadIdx.x == 0) cands = 0;
+  __syncthreads();
   VMP_UNIFORM_LOOP(q, valid, nseg) {
     const int32_t vid = valid ? b.seg_vid[q] : -1;
     const int s = b.nsess == 1 || !valid ? 0 : b.seg_sess[q];
@@ -270,10 +273,11 @@ __global__ void k_candidates(const MapDev* maps, const SessInfo* si, BatchBufs b
         for (int j = 0; j < 6; ++j)
           if (nvs[j] >= 0 && ntag[j] != tag && (nflg[j] & kAlive)) atomicOr(&m.vs[nvs[j]].flags, kDirty);
     }
-    // the session's candidate count, one atomic per wave and session; each
-    // candidate goes to its session's offset plus its point time (a call
-    // time belongs to one voxel), so the filled slots are in sorted order
-    wave_fetch_add(&c->ncand, ne);
+    // the session's candidate count; each candidate goes to its session's
+    // offset plus its point time (a call time belongs to one voxel), so the
+    // filled slots are in sorted order
+    if (b.nsess > 1) wave_fetch_add(&c->ncand, ne);
+    else if (ne) atomicAdd(&cands, ne);
     if (ne > 0) {
       const int off = si[s].off, ns_pts = si[s].n;
       for (int k = 0; k < ne; ++k) {
@@ -294,6 +298,8 @@ __global__ void k_candidates(const MapDev* maps, const SessInfo* si, BatchBufs b
       b.seg_nct[q] = ne;
     }
   }
+  __syncthreads();
+  if (threadIdx.x == 0 && cands) atomicAdd(&m0.ctr->ncand, cands);
 }
 
 // ------------------------------------------------------------------ K8 ----
