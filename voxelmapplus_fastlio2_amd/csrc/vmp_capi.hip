@@ -1818,7 +1818,7 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
           replay_lanes();
         }
         if (!(mode & kStepBuild)) {
-          timed_launch(c, kTkCandidates, [&] { hipLaunchKernelGGL(k_candidates, dim3(gn), dim3(T), 0, st, M, S, b); });
+          timed_launch(c, kTkCandidates, [&] { hipLaunchKernelGGL(k_candidates, dim3(2 * gn), dim3(T), 0, st, M, S, b); });
           timed_launch(c, kTkSpecEval, [&] {
             hipLaunchKernelGGL(k_spec_eval, dim3(std::max(1, prim_tiles(ntot))), dim3(kPrimThreads), 0, st, M, S, b,
                                prim_ws(b.prim));

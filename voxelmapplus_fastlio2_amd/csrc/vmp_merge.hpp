@@ -203,99 +203,91 @@ __device__ inline void merge_fuse(double* pv, double* pn) {
 }
 
 // ------------------------------------------------------------------ K7 ----
-__global__ void k_candidates(const MapDev* maps, const SessInfo* si, BatchBufs b) {
+// Eight lanes per touched voxel: lane j < 6 its face neighbour j (id, record,
+// and the first call after the neighbour's freezing), lane 6 its own freezing
+// and carried dirty mark; the distinct call times are then sorted within the
+// eight lanes.  Bound by the chain of round trips of one lane; with a lane per
+// voxel the searches of up to seven call times ran one after the other
+// (22 us at 120,000 points, 13 now).
+constexpr int kCandLanes = 8;
+__global__ void __launch_bounds__(kMapThreads) k_candidates(const MapDev* maps, const SessInfo* si, BatchBufs b) {
   const int nseg = b.cnt[0];
   const MapDev m0 = maps[0];  // a one-session step reads its map's record once
   __shared__ int cands;       // and adds its candidates once per block
   if (threadIdx.x == 0) cands = 0;
   __syncthreads();
-  VMP_UNIFORM_LOOP(q, valid, nseg) {
+  constexpr int kPer = kMapThreads / kCandLanes;
+  const int j = threadIdx.x % kCandLanes, lane = threadIdx.x & 63, g0 = lane & ~(kCandLanes - 1);
+  for (int q0 = blockIdx.x * kPer; q0 < nseg; q0 += gridDim.x * kPer) {
+    const int q = q0 + int(threadIdx.x) / kCandLanes;
+    const bool valid = q < nseg;
     const int32_t vid = valid ? b.seg_vid[q] : -1;
     const int s = b.nsess == 1 || !valid ? 0 : b.seg_sess[q];
     MapDev m;
     if (b.nsess == 1) m = m0;
     else m = maps[s];
     MapCounters* c = m.ctr;
-    int emitted[7];
-    int ne = 0;
-    if (valid) {
-      b.seg_nct[q] = 0;
-      if (vid < 0)
-        for (int j = 0; j < 6; ++j) b.seg_nbr[q * 6 + j] = make_int2(-1, kNever);
-    }
+    constexpr int kNone = -2;
+    int after = kNone;  // a candidate is the first call after this time
+    int dirty = -2, call = kNever;
+    int2 nb = make_int2(-1, kNever);
     if (vid >= 0) {
       const int tag = c->tag, off = si[s].off;
       VoxState& st = m.vs[vid];
-      int dirty = (st.flags & kDirty) ? -1 : -2;
-      const bool own_freeze = st.freeze_t >= 0 && (st.flags & kPlane);
-      if (own_freeze && st.freeze_t > dirty) dirty = st.freeze_t;
-      const bool has_calls = st.merge_pos != kNever;
-      auto emit = [&](int after) {
-        const int t = first_call_after(b, q, st.merge_pos, after, off);
-        if (t == kNever) return;
-        for (int k = 0; k < ne; ++k)
-          if (emitted[k] == t) return;  // one candidate per distinct call
-        emitted[ne++] = t;
-      };
-      if (has_calls && ((st.flags & kDirty) || own_freeze)) emit(-1);
-      // the six neighbours' entries, then their records, six loads at a time
-      int32_t nvs[6];
-      lookup_nbrs6(m, st.key, nvs);
-      int ntag[6], nfrz[6], ncre[6], nevt[6], nprv[6];
-      uint32_t nflg[6];
-#pragma unroll
-      for (int j = 0; j < 6; ++j) {
-        const VoxState& nbs = m.vs[nvs[j] < 0 ? 0 : nvs[j]];
-        ntag[j] = nbs.tag;
-        nfrz[j] = nbs.freeze_t;
-        nflg[j] = nbs.flags;
-        ncre[j] = nbs.create_t;
-        nevt[j] = nbs.evict_t;
-        nprv[j] = nbs.prev_vid;
+      const int start = b.seg_start[q], end = b.seg_end[q];
+      const uint32_t flags = st.flags;
+      const int freeze_t = st.freeze_t, merge_pos = st.merge_pos;
+      const bool own_freeze = freeze_t >= 0 && (flags & kPlane);
+      if (j == 6) {
+        dirty = (flags & kDirty) ? -1 : -2;
+        if (own_freeze) dirty = freeze_t;
+        if ((flags & kDirty) || own_freeze) after = -1;
+      } else if (j < 6 && key_neighbour_ok(st.key, j)) {
+        const int32_t nv = lookup_vid(m, key_neighbour(st.key, j));
+        if (nv >= 0) {
+          const VoxState& ns = m.vs[nv];
+          const int ntag = ns.tag, nfrz = ns.freeze_t, ncre = ns.create_t, nevt = ns.evict_t, nprv = ns.prev_vid;
+          const uint32_t nflg = ns.flags;
+          const bool cur = ntag == tag;
+          const bool frozen_plane = !(nflg & kEnable) && (nflg & kPlane) && (nflg & kInit);
+          nb = make_int2(nv, frozen_plane ? (cur ? max(ncre, nfrz) : -1) : kNever);
+          if (cur && (nevt != kNever || nprv >= 0)) nb.y = kNbrSlow;
+          if (cur && nfrz >= 0 && (nflg & kPlane)) dirty = after = nfrz;
+          // a frozen plane marks its untouched live neighbours dirty for later
+          // scans (only their kDirty bit changes: this kernel reads kPlane and
+          // kAlive of neighbours, and the own flags of touched voxels only)
+          if (own_freeze && !cur && (nflg & kAlive)) atomicOr(&m.vs[nv].flags, kDirty);
+        }
       }
-      for (int j = 0; j < 6; ++j) {
-        const int32_t nv = nvs[j];
-        const bool cur = ntag[j] == tag;
-        const bool frozen_plane = !(nflg[j] & kEnable) && (nflg[j] & kPlane) && (nflg[j] & kInit);
-        int from = frozen_plane ? (cur ? max(ncre[j], nfrz[j]) : -1) : kNever;
-        if (cur && (nevt[j] != kNever || nprv[j] >= 0)) from = kNbrSlow;
-        b.seg_nbr[q * 6 + j] = make_int2(nv, from);
-        if (nv < 0) continue;
-        if (ntag[j] != tag || nfrz[j] < 0 || !(nflg[j] & kPlane)) continue;
-        if (nfrz[j] > dirty) dirty = nfrz[j];
-        if (has_calls) emit(nfrz[j]);
-      }
-      st.dirty_t = dirty;
-      // a frozen plane marks its untouched live neighbours dirty for later
-      // scans (only their kDirty bit changes: this kernel reads kPlane and
-      // kAlive of neighbours, and the own flags of touched voxels only)
-      if (st.freeze_t >= 0 && (st.flags & kPlane))
-        for (int j = 0; j < 6; ++j)
-          if (nvs[j] >= 0 && ntag[j] != tag && (nflg[j] & kAlive)) atomicOr(&m.vs[nvs[j]].flags, kDirty);
+      if (after != kNone && merge_pos != kNever) call = first_call_in(b, start + merge_pos, end, after, off);
     }
+    if (valid && j < 6) b.seg_nbr[q * 6 + j] = nb;
+    // one candidate per distinct call, ascending
+    int tv[kCandLanes];
+#pragma unroll
+    for (int o = 0; o < kCandLanes; ++o) tv[o] = __shfl(call, g0 + o, 64);
+    bool emits = call != kNever;
+#pragma unroll
+    for (int o = 0; o < kCandLanes; ++o) emits &= !(o < j && tv[o] == call);
+    const uint64_t all = __ballot(emits);
+    const uint32_t em = uint32_t(all >> g0) & ((1u << kCandLanes) - 1u);
+    int pos = 0;
+#pragma unroll
+    for (int o = 0; o < kCandLanes; ++o) pos += ((em >> o) & 1u) && tv[o] < call ? 1 : 0;
+#pragma unroll
+    for (int o = 1; o < kCandLanes; o <<= 1) dirty = max(dirty, __shfl_xor(dirty, o, 64));
+    if (valid && j == 0) b.seg_nct[q] = __popc(em);
+    if (vid >= 0 && j == 6) m.vs[vid].dirty_t = dirty;
     // the session's candidate count; each candidate goes to its session's
     // offset plus its point time (a call time belongs to one voxel), so the
     // filled slots are in sorted order
-    if (b.nsess > 1) wave_fetch_add(&c->ncand, ne);
-    else if (ne) atomicAdd(&cands, ne);
-    if (ne > 0) {
-      const int off = si[s].off, ns_pts = si[s].n;
-      for (int k = 0; k < ne; ++k) {
-        if (emitted[k] < ns_pts) b.cand_in[off + emitted[k]] = cand_key_batch(s, emitted[k], vid, b.cand_sshift);
-        else atomicOr(&c->error, 16);
-      }
-      // candidate times, ascending (insertion sort of <= 7)
-      for (int i = 1; i < ne; ++i) {
-        const int v = emitted[i];
-        int k = i - 1;
-        while (k >= 0 && emitted[k] > v) {
-          emitted[k + 1] = emitted[k];
-          --k;
-        }
-        emitted[k + 1] = v;
-      }
-      for (int k = 0; k < ne; ++k) b.seg_ct[q * 7 + k] = emitted[k];
-      b.seg_nct[q] = ne;
+    if (b.nsess > 1) wave_fetch_add(&c->ncand, emits ? 1 : 0);
+    else if (lane == 0 && all) atomicAdd(&cands, __popcll(all));
+    if (emits) {
+      const int off = si[s].off;
+      if (call < si[s].n) b.cand_in[off + call] = cand_key_batch(s, call, vid, b.cand_sshift);
+      else atomicOr(&c->error, 16);
+      b.seg_ct[q * 7 + pos] = call;
     }
   }
   __syncthreads();
