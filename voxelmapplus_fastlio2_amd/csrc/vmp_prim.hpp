@@ -178,14 +178,16 @@ struct NoTail {
 };
 
 // ---- stable compaction: for the k-th i < n (ascending) whose pred(i) = v is
-// non-zero, out(k, i, v).  pred is called once per item and may clear what it
-// read.  tail(count), if active, runs in every thread of the last tile to
+// non-zero, out(k, i, v), a tile's selected items a thread each (packed in
+// LDS: a thread's own items one after the other made a chain of their loads).
+// pred is called once per item and may clear what it read.  tail(count), if active, runs in every thread of the last tile to
 // finish, after the outputs of all tiles are visible.
 template <class Pred, class Out, class Tail>
 __global__ void __launch_bounds__(kPrimThreads) k_select1(int n, Pred pred, Out out, Tail tail, int32_t* count,
                                                           PrimWs ws) {
   using Scan = rocprim::block_scan<int32_t, kPrimThreads>;
   __shared__ typename Scan::storage_type st;
+  __shared__ int32_t s_idx[kPrimTile], s_val[kPrimTile];
   __shared__ int s_tile, s_last;
   __shared__ uint32_t s_prefix;
   const int nt = gridDim.x;
@@ -202,6 +204,13 @@ __global__ void __launch_bounds__(kPrimThreads) k_select1(int n, Pred pred, Out 
   }
   int32_t pos = 0, agg = 0;
   Scan().exclusive_scan(c, pos, 0, agg, st);
+  int at = pos;
+#pragma unroll
+  for (int k = 0; k < kPrimIpt; ++k)
+    if (v[k] != 0) {
+      s_idx[at] = base + k;
+      s_val[at++] = v[k];
+    }
   if (threadIdx.x < 64) {
     const bool l0 = threadIdx.x == 0;
     uint32_t prefix = 0;
@@ -215,11 +224,8 @@ __global__ void __launch_bounds__(kPrimThreads) k_select1(int n, Pred pred, Out 
     if (l0) s_prefix = prefix;
   }
   __syncthreads();
-  pos += int32_t(s_prefix);
-  tail.at_tile(tile, base, pos, v);
-#pragma unroll
-  for (int k = 0; k < kPrimIpt; ++k)
-    if (v[k] != 0) out(pos++, base + k, v[k]);
+  tail.at_tile(tile, base, pos + int32_t(s_prefix), v);
+  for (int i = threadIdx.x; i < agg; i += kPrimThreads) out(int32_t(s_prefix) + i, s_idx[i], s_val[i]);
   if (threadIdx.x == 0 && tile == nt - 1) *count = int32_t(s_prefix) + agg;
   if (finish_tile(ws.ctl, nt, ws.status, nt, nullptr, 0, &s_last, Tail::kActive) && Tail::kActive) tail(*count);
 }
