@@ -83,10 +83,33 @@ __global__ void k_check_points(PtsRefs inl, const PtsRef* refs, int nref, int32_
                                int32_t* sig, int32_t want) {
   for (int r = blockIdx.y; r < nref; r += gridDim.y) {
     const PtsRef R = nref <= kCheckInline ? inl.r[r] : refs[r];
+    // four points a thread, every load of them in flight together (past the
+    // end the last point again; tests that skip a load made a chain of up to
+    // sixteen round trips: 9 us at 20,000 points, 12 at 120,000)
     int b = 0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < R.n; i += gridDim.x * blockDim.x) {
-      b |= !(isfinite(R.x[i]) && isfinite(R.y[i]) && isfinite(R.z[i]));
-      if (R.t) b |= !isfinite(R.t[i]) || (i > 0 && !(R.t[i] >= R.t[i - 1]));
+    const int last = R.n - 1;
+    for (int i0 = blockIdx.x * 4 * blockDim.x + threadIdx.x; i0 <= last; i0 += gridDim.x * 4 * blockDim.x) {
+      float x[4], y[4], z[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int i = min(i0 + k * int(blockDim.x), last);
+        x[k] = R.x[i];
+        y[k] = R.y[i];
+        z[k] = R.z[i];
+      }
+      if (R.t) {
+        float t[4], u[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int i = min(i0 + k * int(blockDim.x), last);
+          t[k] = R.t[i];
+          u[k] = R.t[max(i - 1, 0)];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) b |= int(!isfinite(t[k])) | int(!(t[k] >= u[k]));
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) b |= int(!isfinite(x[k])) | int(!isfinite(y[k])) | int(!isfinite(z[k]));
     }
     if (__ballot(b) != 0ull && (threadIdx.x & 63) == 0) {
       __hip_atomic_store(bad + r, gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);

@@ -1,7 +1,8 @@
 // Map update: VoxelMap::update / build (voxel_map.cpp:200-256) with
 // VoxelGrid::pushPoint / updatePlane / merge (voxel_map.cpp:42-186), executed
 // for a batch of independent sessions as a pipeline of data-parallel stages
-// plus two short ordered replays (one wave per session).
+// plus, for the scans that need them, the evictions' decisions and the merge
+// replay (one workgroup per session each).
 //
 // Points of all sessions in a batch share one global index space, session
 // after session (g = off[s] + i); times inside a session are its point
@@ -13,13 +14,13 @@
 //                    points become a contiguous segment in point order
 //   K3/K4 segments   segment heads, the existing voxel of each segment, new
 //                    keys flagged at their first point
-//   K5 create        creation events in point order: parallel when the LRU
-//                    cannot overflow, else one wave per session replays
-//                    creations and evictions against the LRU queue
-//   K6 replay        one lane per voxel walks its points through the pushPoint
-//                    state machine; the voxels whose walk reaches a refit
-//                    (known from counts) take the FP64 moment path, the others
-//                    a light one that queues their points (no point pool)
+//   K5 create        creation events in point order; where the LRU can
+//                    overflow, one workgroup per session decides all creations
+//                    and evictions against the LRU queue at once
+//   K6 replay        each voxel's points through the pushPoint state machine;
+//                    the voxels whose walk reaches a refit (known from counts)
+//                    take the FP64 moment path (a wave or a lane each), the
+//                    others a light one that queues their points
 //   K7/K8 merge      see vmp_merge.hpp
 //   K9 finalize      dirty bits, LRU queue append, hash tombstones, free list
 // Every ordering decision (LRU order, victims, group ids, merge order) is
