@@ -834,8 +834,8 @@ def main():
         "stage_ms_per_scan": {
             "filter_stage_graph": float(np.mean(stage_graph["filter"])),
             "map_stage_graph": float(np.mean(stage_graph["map"])),
-            "graph_measured_over": f"{RG} scans after the timed region, hipGraph replays between the library's "
-            "HIP events (filter: IESKF begin, iterations and end; map: the whole map update)",
+            "graph_measured_over": f"{RG} scans after the timed region, hipGraph replays, by the device clock "
+            "(filter: IESKF begin, iterations and end; map: the whole map update)",
             "observe_kernels": tt["obs_ms"] / max(RF, 1),
             "map_update_eager": tt["map_ms"] / max(tt["map_calls"], 1),
             "measured_over": f"{RF} scans after those, launched kernel by kernel with per-launch HIP events",
