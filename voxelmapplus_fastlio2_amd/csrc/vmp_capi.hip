@@ -453,10 +453,18 @@ struct vmp_session {
   ImuPkg* stage = nullptr;  // the pending package's IMU samples (host memory)
   float *own_fx = nullptr, *own_fy = nullptr, *own_fz = nullptr;  // VoxelGrid output (scan_resolution > 0)
   // x and P as the last step left them (k_finish), while nothing has been
-  // launched since that changes them
+  // launched since that changes them.  Every call that changes them counts
+  // itself in state_gen, a step when it is launched; step_finish hands out the
+  // step's copy only if nothing came behind the step (a motion prior may be
+  // enqueued while a submitted batch runs).
   bool state_known = false;
+  uint64_t state_gen = 0, step_gen = 0;
   vmp_state known_x{};
   double known_P[529]{};
+  void state_changes() {
+    state_known = false;
+    ++state_gen;
+  }
 };
 
 static uint32_t next_pow2(uint64_t v) {
@@ -985,7 +993,7 @@ extern "C" int vmp_state_set(vmp_session* s, const vmp_state* x, const double* P
   std::lock_guard<std::mutex> lk(s->ctx->mu);
   VMP_HIP(hipSetDevice(s->ctx->device));
   hipStream_t st = s->ctx->stream;
-  s->state_known = false;
+  s->state_changes();
   if (x) VMP_HIP(hipMemcpyAsync(&s->f->x, x, sizeof(vmp_state), hipMemcpyHostToDevice, st));
   if (P) VMP_HIP(hipMemcpyAsync(s->f->P, P, sizeof(double) * 529, hipMemcpyHostToDevice, st));
   VMP_HIP(hipStreamSynchronize(st));
@@ -1017,7 +1025,7 @@ extern "C" int vmp_state_apply_motion(vmp_session* s, const double* dR, const do
   Diag23 d;
   for (int i = 0; i < 23; ++i) d.q[i] = qdiag[i];
   // ordered before the next call on this context's stream
-  s->state_known = false;
+  s->state_changes();
   hipLaunchKernelGGL(k_apply_motion, dim3(1), dim3(64), 0, s->ctx->stream, s->f, R, p, d);
   VMP_HIP(hipGetLastError());
   return VMP_OK;
@@ -1034,7 +1042,7 @@ static int enqueue_motion(vmp_ctx* c, vmp_session** ss, int n, const double* dR,
   VMP_HIP(upload_wait(c, w.motion_after));  // the pinned table is reused
   for (int i = 0; i < n; ++i) {
     MotionRec& r = w.h_motion[i];
-    ss[i]->state_known = false;
+    ss[i]->state_changes();
     r.f = ss[i]->f;
     std::memcpy(r.dR, dR + 9 * size_t(i), sizeof(r.dR));
     std::memcpy(r.dp, dp + 3 * size_t(i), sizeof(r.dp));
@@ -1150,7 +1158,7 @@ extern "C" int vmp_imu_init(vmp_session* s, const vmp_imu_cfg* cfg, const double
   std::lock_guard<std::mutex> lk(c->mu);
   VMP_HIP(hipSetDevice(c->device));
   settle(c);
-  s->state_known = false;
+  s->state_changes();
   double* buf = nullptr;
   VMP_HIP(hipMalloc(&buf, sizeof(double) * 7 * size_t(total)));
   hipStream_t st = c->stream;
@@ -2225,7 +2233,10 @@ static int step_begin(vmp_ctx* c, vmp_session** ss, int n, int mode) {
         return VMP_ESTATE;
       }
   }
-  for (int i = 0; i < n; ++i) ss[i]->state_known = false;
+  for (int i = 0; i < n; ++i) {
+    ss[i]->state_changes();
+    ss[i]->step_gen = ss[i]->state_gen;
+  }
   rc = prepare_scans(c, ss, n, (mode & kStepBuild) != 0);
   if (rc != VMP_OK) {
     s->err = "undistortion / scan filter failed";
@@ -2300,9 +2311,11 @@ static int step_finish(vmp_ctx* c, vmp_obs_stats* ost, vmp_map_stats* mst) {
     vmp_session* si = ss[i];
     const BatchOut& o = c->ws.h_out[i];
     si->h_ctr = o.ctr;
-    si->known_x = o.x;
-    std::memcpy(si->known_P, o.P, sizeof(o.P));
-    si->state_known = true;
+    if (si->state_gen == si->step_gen) {
+      si->known_x = o.x;
+      std::memcpy(si->known_P, o.P, sizeof(o.P));
+      si->state_known = true;
+    }
     ok[i] = 0;
     if ((mode & kStepIeskf) && o.obs[7]) {
       si->err = "hash probe overflow";
@@ -2400,7 +2413,7 @@ extern "C" int vmp_observe(vmp_session* s, const vmp_state* x, double* H, double
   const int crc = check_bound_points(c, one, 1);
   if (crc != VMP_OK) return crc;
   if (ws_reserve(c, std::max(s->n, 1), 1) != VMP_OK) return VMP_ENOMEM;
-  s->state_known = false;
+  s->state_changes();
   if (s->raw_pending) {
     // undistortion propagates the state the session holds: the call's x first
     VMP_HIP(hipMemcpyAsync(&s->f->x, x, sizeof(vmp_state), hipMemcpyHostToDevice, c->stream));
