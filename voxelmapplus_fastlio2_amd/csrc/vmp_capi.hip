@@ -179,6 +179,7 @@ __global__ void __launch_bounds__(kFinishThreads) k_finish(const MapDev* maps, c
   for (int i = tid; i < 529; i += kFinishThreads) o.P[i] = f->P[i];
   if (tid < 8) o.obs[tid] = obs_stat[s][tid];
   if (tid == 8) o.iters = f->iters;
+  wait_stores();
   __syncthreads();
   if (tid != 0) return;
   if (*prim_err) o.ctr.error |= 64;  // a bounded wait of the compaction / sort ran out

@@ -483,11 +483,9 @@ __global__ void __launch_bounds__(kObsThreads) k_obs_reduce(const ObsJob* __rest
   if (!out) return;
   if (tid < 4) out->ctr[tid] = int32_t(red[0][NACC + tid]);
   else if (tid < 8) out->ctr[tid] = J.counters[tid];
+  wait_stores();
   __syncthreads();
-  if (tid == 0) {
-    __threadfence_system();
-    if (sig) __hip_atomic_store(sig, want, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+  if (tid == 0 && sig) __hip_atomic_store(sig, want, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 }  // namespace vmp
