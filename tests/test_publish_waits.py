@@ -114,3 +114,13 @@ def test_results_for_the_host_are_stored_before_the_signal(code_object, name):
         publish, bad = barriers_with_stores_in_flight(ins)
         assert publish, symbol
         assert not bad, (symbol, [hex(ins[i][0]) for i in bad])
+
+
+@pytest.mark.parametrize("name", ["k_select1", "k_rs_pass", "k_spec_eval"])
+def test_a_tile_is_stored_before_it_counts_itself_done(code_object, name):
+    found = kernels(code_object, name)
+    assert found
+    for symbol, ins in found.items():
+        publish, bad = barriers_with_stores_in_flight(ins)
+        assert publish, symbol
+        assert not bad, (symbol, [hex(ins[i][0]) for i in bad])

@@ -15,6 +15,8 @@
 #include <rocprim/block/block_reduce.hpp>
 #include <rocprim/block/block_scan.hpp>
 
+#include "vmp_common.hpp"
+
 namespace vmp {
 
 constexpr int kPrimThreads = 256;
@@ -145,13 +147,14 @@ __device__ inline uint32_t look_back_wave(const uint32_t* status, int tile, Prim
 }
 // end of a tile: the last to finish clears `nclear` status words (and the
 // extra words, if any) and the done counter; returns true in that tile
-// (every thread of it).  With `publish`, the tile's stores are released
-// device-wide before it counts itself done (the workgroup barrier orders
-// every thread's stores before thread 0's agent-scope release fence, which
-// the memory model makes cumulative), and the last tile acquires them, so it
-// may read what every tile wrote.
+// (every thread of it).  Every wave waits for its stores before the tile
+// counts itself done: the words that the last tile clears must not arrive
+// behind it.  With `publish` thread 0 then releases them device-wide (its
+// fence writes back the L2 that all waves of the tile store through) and the
+// last tile acquires them, so it may read what every tile wrote.
 __device__ inline bool finish_tile(PrimCtl* ctl, int nt, uint32_t* status, int nclear, int32_t* extra, int nextra,
                                    int* s_last, bool publish = false) {
+  wait_stores();
   __syncthreads();
   if (threadIdx.x == 0) {
     if (publish) __threadfence();
