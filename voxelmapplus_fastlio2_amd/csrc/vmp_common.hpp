@@ -245,8 +245,8 @@ __host__ __device__ inline void split_f32(double v, float& hi, float& lo) {
   lo = float(v - double(hi));
 }
 
-// 1 / sqrt(x) and 1 / x for normal x > 0: the hardware's estimate (about 23
-// bits) and one third-order step
+// 1 / sqrt(x) and 1 / x for normal x > 0 (not for zero or infinity): the
+// hardware's estimate (about 23 bits) and one third-order step
 __device__ inline double rsqrt_pos(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-x * y, y, 1.0);

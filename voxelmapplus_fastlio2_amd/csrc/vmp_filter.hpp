@@ -94,11 +94,22 @@ __global__ void __launch_bounds__(kBeginEndThreads) k_ieskf_begin(FilterDev** fs
   double a[23];  // row `lane` of P (column-major in memory), factored in lanes
 #pragma unroll
   for (int c = 0; c < 23; ++c) a[c] = lane < 23 ? f->P[c * 23 + lane] : 0.0;
+  // An entry with an infinite variance, of which nothing is known: its row
+  // and column of P^-1 are zero.  The factorisation's reciprocal square root
+  // takes finite pivots, so a row of the identity stands in for it there.
+  const int l = lane & 63;
+  const uint64_t unknown = __ballot(l < 23 && f->P[l < 23 ? l * 24 : 0] == __builtin_inf());
+  if (unknown) {
+#pragma unroll
+    for (int c = 0; c < 23; ++c)
+      if (((unknown >> c) | (unknown >> l)) & 1) a[c] = c == lane ? 1.0 : 0.0;
+  }
   double dinv;
   __shared__ double S[23 * 24], Pi[529];
   chol_rows(a, dinv, lane);
   chol_inverse_rows(a, dinv, Pi, lane, S);  // P^-1
-  for (int i = lane; i < 529; i += kBeginEndThreads) as_global(f->Pinv)[i] = Pi[i];
+  for (int i = lane; i < 529; i += kBeginEndThreads)
+    as_global(f->Pinv)[i] = i % 24 == 0 && (unknown >> (i / 24) & 1) ? 0.0 : Pi[i];
   __syncthreads();
   load_state(sx, f->xp, lane);
   if (lane == 0) {
