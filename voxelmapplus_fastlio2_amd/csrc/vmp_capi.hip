@@ -257,7 +257,7 @@ struct BatchWs {
   int32_t* h_vgst = nullptr;
   ObsJob job{};             // the first observe job as last uploaded
   bool job_known = false;
-  int32_t motion_after = -1;  // signals launched before the last motion table upload (-1: none)
+  bool motion_pending = false;  // the motion table's last upload may still be reading h_motion
   std::vector<void*> host_allocs;
 
   void release() {
@@ -303,11 +303,12 @@ struct vmp_ctx {
   // observe launches back to back between one event pair (the kernel is
   // idempotent: the repetitions rewrite the same slots and partial rows)
   int obs_time_reps = 1;
-  // Pinned coherent word that kernels set to their generation once the
-  // stream's earlier work is complete; sig_gen: the last generation
-  // launched, sig_seen: the latest one known complete.
+  // Pinned coherent words that kernels set to their generation once the
+  // stream's earlier work is complete: the steps' and checks' (sig_gen: the
+  // last one launched) and, a line on, the motion priors'.  Only compared for
+  // equality, so they may wrap.
   int32_t* h_sig = nullptr;
-  int32_t sig_gen = 0, sig_seen = 0;
+  uint32_t sig_gen = 0, motion_gen = 0;
   int32_t* d_done = nullptr;  // finished-block counters: [0] k_check_points, [1] k_finish
   ObsOut* h_obs = nullptr;      // results of vmp_observe, written by k_obs_reduce
   double clk_khz = 1e5;       // rate of the device clock
@@ -486,27 +487,16 @@ extern "C" const char* vmp_version(void) { return "voxelmapplus_fastlio2_amd 0.2
 // completed (a fault stops the stream before it), so a seen signal ends the
 // wait; otherwise, after 2 ms, hipStreamSynchronize waits for the rest and
 // reports any fault.
-static hipError_t wait_signal(vmp_ctx* c, int32_t want) {
-  if (c->h_sig) {
+static hipError_t wait_word(vmp_ctx* c, const int32_t* word, int32_t want) {
+  if (word) {
     const auto t0 = std::chrono::steady_clock::now();
     while (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(2))
-      if (__atomic_load_n(c->h_sig, __ATOMIC_ACQUIRE) == want) {
-        c->sig_seen = want;
-        return hipSuccess;
-      }
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) == want) return hipSuccess;
   }
-  const hipError_t e = hipStreamSynchronize(c->stream);
-  if (e == hipSuccess) c->sig_seen = c->sig_gen;
-  return e;
+  return hipStreamSynchronize(c->stream);
 }
-// Whether an upload enqueued when `after` generations had been launched may
-// still be reading its pinned source: not once a later signal has been seen.
-static hipError_t upload_wait(vmp_ctx* c, int32_t& after) {
-  if (after < 0) return hipSuccess;
-  const bool done = c->sig_seen > after;
-  after = -1;
-  return done ? hipSuccess : hipStreamSynchronize(c->stream);
-}
+static hipError_t wait_signal(vmp_ctx* c, int32_t want) { return wait_word(c, c->h_sig, want); }
+constexpr int kSigMotion = 32;  // of h_sig: the motion priors' word
 
 static void noalloc_setup(vmp_ctx* c);
 
@@ -526,7 +516,7 @@ extern "C" int vmp_ctx_create(int device, vmp_ctx** out) {
   void* hs = nullptr;
   if (hipHostMalloc(&hs, 256, hipHostMallocCoherent) == hipSuccess) {
     c->h_sig = static_cast<int32_t*>(hs);
-    *c->h_sig = 0;
+    c->h_sig[0] = c->h_sig[kSigMotion] = 0;
   }
   const int32_t zero[64] = {};
   if (hipMalloc(&c->d_done, sizeof(zero)) != hipSuccess ||
@@ -621,7 +611,7 @@ static int check_device_points(vmp_ctx* c, const PtsRef* refs, int nref) {
   // four points per thread, at most 64 blocks per set (every block counts
   // itself done on one counter)
   const int gx = int(std::max<int64_t>(1, std::min<int64_t>((most + 1023) / 1024, nref > 1 ? 64 : 256)));
-  const int32_t want = ++c->sig_gen;
+  const int32_t want = int32_t(++c->sig_gen);
   hipLaunchKernelGGL(k_check_points, dim3(gx, std::min(nref, 65535)), dim3(256), 0, st, inl, c->d_refs, nref,
                      c->h_bad, gen, c->d_done, c->h_sig, want);
   if (hipGetLastError() != hipSuccess || wait_signal(c, want) != hipSuccess) return -2;
@@ -731,7 +721,7 @@ static int ws_reserve(vmp_ctx* c, int64_t points, int nsess, bool exact = false)
     *p = static_cast<std::remove_reference_t<decltype(**p)>*>(q);
     return true;
   };
-  w.motion_after = -1;
+  w.motion_pending = false;
   if (!ws_layout(c, w, size_t(np), ns, size_t(1) << 18, dev, host) ||
       hipMemsetAsync(w.b.prim, 0, prim_ws_entries(np) * sizeof(int32_t), c->stream) != hipSuccess) {
     w.release();
@@ -1040,7 +1030,12 @@ static int enqueue_motion(vmp_ctx* c, vmp_session** ss, int n, const double* dR,
   VMP_HIP(hipSetDevice(c->device));
   if (ws_reserve(c, 1, n) != VMP_OK) return VMP_ENOMEM;
   BatchWs& w = c->ws;
-  VMP_HIP(upload_wait(c, w.motion_after));  // the pinned table is reused
+  // the pinned table is reused: until the last prior's kernel has started, its
+  // upload may be reading it (a batch submitted behind that prior is not
+  // waited for)
+  int32_t* word = c->h_sig ? c->h_sig + kSigMotion : nullptr;
+  if (w.motion_pending) VMP_HIP(wait_word(c, word, int32_t(c->motion_gen)));
+  w.motion_pending = false;
   for (int i = 0; i < n; ++i) {
     MotionRec& r = w.h_motion[i];
     ss[i]->state_changes();
@@ -1050,8 +1045,9 @@ static int enqueue_motion(vmp_ctx* c, vmp_session** ss, int n, const double* dR,
     std::memcpy(r.q, qdiag + size_t(qstride) * size_t(i), sizeof(r.q));
   }
   VMP_HIP(hipMemcpyAsync(w.d_motion, w.h_motion, sizeof(MotionRec) * n, hipMemcpyHostToDevice, c->stream));
-  w.motion_after = c->sig_gen;
-  hipLaunchKernelGGL(k_apply_motion_batch, dim3((n + 63) / 64), dim3(64), 0, c->stream, w.d_motion, n);
+  w.motion_pending = true;
+  hipLaunchKernelGGL(k_apply_motion_batch, dim3((n + 63) / 64), dim3(64), 0, c->stream, w.d_motion, n, word,
+                     int32_t(++c->motion_gen));
   VMP_HIP(hipGetLastError());
   return VMP_OK;
 }
@@ -1685,7 +1681,7 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
   };
   if (mode & kStepObserveOnce) {
     if (obs_x) {
-      c->fl_want = ++c->sig_gen;
+      c->fl_want = int32_t(++c->sig_gen);
       hipLaunchKernelGGL(k_obs_prep_at, dim3(1), dim3(64), 0, st, ss[0]->f, *obs_x, ss[0]->obs_ctr);
     } else {
       hipLaunchKernelGGL(k_obs_prep, dim3(n), dim3(64), 0, st, w.d_flist, w.d_obsctr);
@@ -1887,7 +1883,7 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
     }
   }
   stage_event(3);
-  c->fl_want = ++c->sig_gen;
+  c->fl_want = int32_t(++c->sig_gen);
   hipLaunchKernelGGL(k_finish, dim3(n), dim3(kFinishThreads), 0, st, w.d_maps, w.d_si, w.d_flist, w.d_obsstat, w.h_out,
                      (mode & kStepMap) ? 1 : 0, &prim_ws(w.b.prim).ctl->err, w.d_clk, c->d_done + 1, c->h_sig,
                      c->fl_want);

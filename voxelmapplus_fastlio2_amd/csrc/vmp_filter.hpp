@@ -53,15 +53,18 @@ __global__ void k_apply_motion(FilterDev* f, D33 dR, D3 dp, Diag23 q) {
   for (int i = 0; i < 23; ++i) f->P[i * 23 + i] += q.q[i];
 }
 
-// the same for many sessions: one thread per session
+// the same for many sessions: one thread per session.  Once it runs, the copy
+// of recs before it in the stream is complete: the word tells the host, which
+// may then fill the copy's source again.
 struct MotionRec {
   FilterDev* f;
   double dR[9];  // column-major
   double dp[3];
   double q[23];
 };
-__global__ void k_apply_motion_batch(const MotionRec* recs, int n) {
+__global__ void k_apply_motion_batch(const MotionRec* recs, int n, int32_t* word, int32_t gen) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0 && word) __hip_atomic_store(word, gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   if (i >= n) return;
   const MotionRec& r = recs[i];
   FilterDev* f = r.f;
