@@ -47,3 +47,57 @@ def test_sessions_without_candidates_between_those_with(count, large):
         g.close()
     a.close()
     b.close()
+
+
+def test_states_of_a_large_batch():
+    """The covariances of a batch of more than 64 sessions are fetched when one
+    is asked for: every state bitwise as from batches of at most 64, before and
+    after a change, another step, a larger workspace and a step without them."""
+    n, count = 300, 70
+    a, b = Context(0), Context(0)
+    seq = [Sequence(ROOM, SEED0 + 700 + i % 5, n) for i in range(count)]
+    small, large = [start(a, q, n) for q in seq], [start(b, q, n) for q in seq]
+    qdiag = np.full(23, 1e-5)
+
+    def check(which):
+        for i in which:
+            for u, v in zip(small[i].get_state(), large[i].get_state()):
+                assert np.array_equal(u, v), i
+
+    def scans(k, which):
+        for i in which:
+            for g in (small[i], large[i]):
+                g.apply_motion(*seq[i].motion(k), qdiag)
+                g.set_points(*(v[:n].copy() for v in seq[i].scan(k)))
+
+    def step(k, which):
+        scans(k, which)
+        register_batch([large[i] for i in which])
+        for lo in range(0, len(which), 64):
+            register_batch([small[i] for i in which[lo : lo + 64]])
+
+    everyone = list(range(count))
+    check(everyone)
+    step(1, everyone)
+    check([69, 0, 33])
+    check(everyone)
+    for g in (small[5], large[5]):  # a change of one session
+        g.apply_motion(*seq[5].motion(2), qdiag)
+    for g in (small[6], large[6]):
+        g.set_state(state_vector(*seq[6].pose(2)))
+    check(everyone)
+    step(3, everyone[:66])  # large again, without some
+    check(everyone)
+    step(4, everyone)
+    step(5, everyone[10:20])  # a small one behind it
+    check(everyone)
+    step(6, everyone)
+    b.reserve(n * 100, 100)
+    check(everyone)
+    step(7, everyone)
+    scans(8, everyone)  # priors of all behind the step
+    check(everyone)
+    for g in small + large:
+        g.close()
+    a.close()
+    b.close()

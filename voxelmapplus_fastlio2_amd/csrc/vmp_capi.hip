@@ -129,17 +129,24 @@ __global__ void k_check_points(PtsRefs inl, const PtsRef* refs, int nref, int32_
 }
 
 // A step's results of one session, written by k_finish into pinned host
-// memory: the counters, the posterior state and covariance, the statistics.
+// memory: the counters, the posterior state, the statistics.
 struct BatchOut {
   MapCounters ctr;
   vmp_state x;
-  double P[529];
   uint64_t clk[3];  // entry 0: start of the filter stage, of the map stage, end (device clock)
   int32_t obs[8];
   int32_t iters;
   int32_t pad[3];
 };
 constexpr int kFinishThreads = 256;
+// Up to this many sessions k_finish also writes the posterior covariances to
+// the host, 529 doubles a session; in larger batches they go to a device array
+// that vmp_state_get fetches whole once it is asked for one.  The writes and
+// the host's copy into each session, 0.25 us a session, are lost where nobody
+// reads them: a step of 2,048 sessions of 100 points 1,745 us with them, 1,238
+// without, of 512 608 and 513.  The first read then takes longer by a copy,
+// 27 us of 128 sessions and 170 of 2,048; at 64 the two sides are equal.
+constexpr int kDirectP = 64;
 // End of a step, a block per session: the map update's counters advance (the
 // LRU appends, the points, and the evicted voxels that k_finalize
 // pushed above the free-list top; nevict stays 0 in a scan without points),
@@ -148,9 +155,10 @@ constexpr int kFinishThreads = 256;
 // three (counters, gather, signal) and a copy, about 14 us less on a step of
 // one session, and the state is read by the host without another copy.
 __global__ void __launch_bounds__(kFinishThreads) k_finish(const MapDev* maps, const SessInfo* si, FilterDev** fs,
-                                                           int32_t** obs_stat, BatchOut* out, int map_step,
-                                                           const int32_t* prim_err, const uint64_t* clk,
-                                                           int32_t* done, int32_t* sig, int32_t want) {
+                                                           int32_t** obs_stat, BatchOut* out, double* P,
+                                                           int map_step, const int32_t* prim_err,
+                                                           const uint64_t* clk, int32_t* done, int32_t* sig,
+                                                           int32_t want) {
   const int s = blockIdx.x, tid = threadIdx.x;
   MapCounters* c = maps[s].ctr;
   BatchOut& o = out[s];
@@ -176,7 +184,7 @@ __global__ void __launch_bounds__(kFinishThreads) k_finish(const MapDev* maps, c
   double* xd = reinterpret_cast<double*>(&o.x);
   for (int i = tid; i < kC; i += kFinishThreads) cd[i] = cs[i];
   for (int i = tid; i < kX; i += kFinishThreads) xd[i] = xs[i];
-  for (int i = tid; i < 529; i += kFinishThreads) o.P[i] = f->P[i];
+  for (int i = tid; i < 529; i += kFinishThreads) P[size_t(s) * 529 + i] = f->P[i];
   if (tid < 8) o.obs[tid] = obs_stat[s][tid];
   if (tid == 8) o.iters = f->iters;
   wait_stores();
@@ -249,6 +257,8 @@ struct BatchWs {
   int32_t** h_obsctr = nullptr;
   int32_t** h_obsstat = nullptr;
   BatchOut* h_out = nullptr;  // written by k_finish
+  double* h_P = nullptr;      // the covariances, written by k_finish or copied from d_P (see kDirectP)
+  double* d_P = nullptr;
   MotionRec* d_motion = nullptr;
   MotionRec* h_motion = nullptr;
   VgJob* d_vg = nullptr;    // sessions of a step whose scan is filtered
@@ -366,6 +376,11 @@ struct vmp_ctx {
   bool fl = false;
   int fl_mode = 0;
   int32_t fl_want = 0;  // its k_finish's generation
+  // the last step of more than kDirectP sessions, while its results are the
+  // workspace's (0: none), and whether its covariances have been fetched
+  uint64_t bulk_step = 0, bulk_steps = 0;
+  int32_t bulk_n = 0;
+  bool bulk_fetched = false;
   std::vector<vmp_session*> fl_ss;
   std::vector<int32_t> fl_n;
   std::vector<vmp_obs_stats> res_ost;  // results of the last submitted batch, once finished
@@ -463,8 +478,13 @@ struct vmp_session {
   uint64_t state_gen = 0, step_gen = 0;
   vmp_state known_x{};
   double known_P[529]{};
+  // After a step of more than kDirectP sessions they stay in the context's
+  // workspace instead (entry `slot`), while bulk_step is the context's.
+  uint64_t bulk_step = 0;
+  int32_t slot = 0;
   void state_changes() {
     state_known = false;
+    bulk_step = 0;
     ++state_gen;
   }
 };
@@ -684,6 +704,7 @@ static bool ws_layout(vmp_ctx* c, BatchWs& w, size_t n, int ns, size_t pre_cap, 
     w.h_obsctr = reinterpret_cast<int32_t**>(w.h_tab + o_oc);
     w.h_obsstat = reinterpret_cast<int32_t**>(w.h_tab + o_os);
   }
+  ok = ok && (ns <= kDirectP || dev(&w.d_P, S * 529)) && host(&w.h_P, sizeof(double) * 529 * S);
   ok = ok && dev(&w.d_clk, size_t(2)) && dev(&w.d_motion, S) && dev(&w.d_vg, S) && dev(&w.d_vgst, S * kVgStat);
   ok = ok && host(&w.h_out, sizeof(BatchOut) * S) && host(&w.h_motion, sizeof(MotionRec) * S) &&
        host(&w.h_vg, sizeof(VgJob) * S) && host(&w.h_vgst, sizeof(int32_t) * kVgStat * S);
@@ -704,6 +725,7 @@ static int ws_reserve(vmp_ctx* c, int64_t points, int nsess, bool exact = false)
   if (points <= w.cap_points && nsess <= w.cap_sess) return VMP_OK;
   if (w.fixed) return VMP_ENOMEM;  // the no-allocation workspace never grows
   settle(c);  // a batch in flight still reads the old workspace
+  c->bulk_step = 0;
   hipStreamSynchronize(c->stream);
   c->ws_gen++;  // captured filter graphs hold the old workspace pointers
   // growth keeps a quarter of headroom, so scans that vary in size do not
@@ -1001,6 +1023,18 @@ extern "C" int vmp_state_get(vmp_session* s, vmp_state* x, double* P) {
   }
   VMP_HIP(hipSetDevice(s->ctx->device));
   hipStream_t st = s->ctx->stream;
+  vmp_ctx* c = s->ctx;
+  if (s->bulk_step != 0 && s->bulk_step == c->bulk_step) {
+    if (P && !c->bulk_fetched) {
+      const size_t bytes = sizeof(double) * 529 * size_t(c->bulk_n);
+      VMP_HIP(hipMemcpyAsync(c->ws.h_P, c->ws.d_P, bytes, hipMemcpyDeviceToHost, st));
+      VMP_HIP(hipStreamSynchronize(st));
+      c->bulk_fetched = true;
+    }
+    if (x) *x = c->ws.h_out[s->slot].x;
+    if (P) std::memcpy(P, c->ws.h_P + size_t(s->slot) * 529, sizeof(double) * 529);
+    return VMP_OK;
+  }
   if (x) VMP_HIP(hipMemcpyAsync(x, &s->f->x, sizeof(vmp_state), hipMemcpyDeviceToHost, st));
   if (P) VMP_HIP(hipMemcpyAsync(P, s->f->P, sizeof(double) * 529, hipMemcpyDeviceToHost, st));
   VMP_HIP(hipStreamSynchronize(st));
@@ -1885,8 +1919,8 @@ static int enqueue_step(vmp_ctx* c, vmp_session** ss, int n, int mode, const vmp
   stage_event(3);
   c->fl_want = int32_t(++c->sig_gen);
   hipLaunchKernelGGL(k_finish, dim3(n), dim3(kFinishThreads), 0, st, w.d_maps, w.d_si, w.d_flist, w.d_obsstat, w.h_out,
-                     (mode & kStepMap) ? 1 : 0, &prim_ws(w.b.prim).ctl->err, w.d_clk, c->d_done + 1, c->h_sig,
-                     c->fl_want);
+                     n <= kDirectP ? w.h_P : w.d_P, (mode & kStepMap) ? 1 : 0, &prim_ws(w.b.prim).ctl->err, w.d_clk,
+                     c->d_done + 1, c->h_sig, c->fl_want);
   return hipGetLastError() == hipSuccess ? VMP_OK : VMP_EDEVICE;
 }
 
@@ -2230,6 +2264,7 @@ static int step_begin(vmp_ctx* c, vmp_session** ss, int n, int mode) {
         return VMP_ESTATE;
       }
   }
+  c->bulk_step = 0;  // the results of this step replace the last one's
   for (int i = 0; i < n; ++i) {
     ss[i]->state_changes();
     ss[i]->step_gen = ss[i]->state_gen;
@@ -2291,6 +2326,11 @@ static int step_finish(vmp_ctx* c, vmp_obs_stats* ost, vmp_map_stats* mst) {
       }
     }
   }
+  if (n > kDirectP) {
+    c->bulk_step = ++c->bulk_steps;
+    c->bulk_n = n;
+    c->bulk_fetched = false;
+  }
   int first_err = VMP_OK;
   uint8_t ok_small[16];
   int32_t did_small[16];
@@ -2309,9 +2349,14 @@ static int step_finish(vmp_ctx* c, vmp_obs_stats* ost, vmp_map_stats* mst) {
     const BatchOut& o = c->ws.h_out[i];
     si->h_ctr = o.ctr;
     if (si->state_gen == si->step_gen) {
-      si->known_x = o.x;
-      std::memcpy(si->known_P, o.P, sizeof(o.P));
-      si->state_known = true;
+      if (n <= kDirectP) {
+        si->known_x = o.x;
+        std::memcpy(si->known_P, c->ws.h_P + size_t(i) * 529, sizeof(si->known_P));
+        si->state_known = true;
+      } else if (si->ctx == c) {
+        si->bulk_step = c->bulk_step;
+        si->slot = i;
+      }
     }
     ok[i] = 0;
     if ((mode & kStepIeskf) && o.obs[7]) {
