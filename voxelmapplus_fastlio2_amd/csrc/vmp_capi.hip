@@ -473,7 +473,11 @@ struct vmp_session {
   // launched since that changes them.  Every call that changes them counts
   // itself in state_gen, a step when it is launched; step_finish hands out the
   // step's copy only if nothing came behind the step (a motion prior may be
-  // enqueued while a submitted batch runs).
+  // enqueued while a submitted batch runs).  A step writes them under the
+  // mutex of the context that runs it, vmp_state_get reads them under the
+  // session's own: a server's sessions, which its executors' contexts run, are
+  // read by the server while no batch holds them (ServSess::busy) and by a
+  // caller between two runs only (vmp_server_session).
   bool state_known = false;
   uint64_t state_gen = 0, step_gen = 0;
   vmp_state known_x{};
@@ -628,8 +632,8 @@ static int check_device_points(vmp_ctx* c, const PtsRef* refs, int nref) {
       hipMemcpyAsync(c->d_refs, c->h_refs, sizeof(PtsRef) * nref, hipMemcpyHostToDevice, st) != hipSuccess)
     return -2;
   const int32_t gen = ++c->check_gen;
-  // four points per thread, at most 64 blocks per set (every block counts
-  // itself done on one counter)
+  // four points per thread; every block counts itself done on one counter, so
+  // at most 256 blocks for one set, 64 a set for several
   const int gx = int(std::max<int64_t>(1, std::min<int64_t>((most + 1023) / 1024, nref > 1 ? 64 : 256)));
   const int32_t want = int32_t(++c->sig_gen);
   hipLaunchKernelGGL(k_check_points, dim3(gx, std::min(nref, 65535)), dim3(256), 0, st, inl, c->d_refs, nref,

@@ -124,7 +124,7 @@ struct __align__(16) VoxState {
   int32_t prev_vid;   // incarnation of the same key evicted in this scan
   int32_t first_t;    // first point of this scan that touched it
   int32_t seg;        // its segment in this scan's key-sorted points
-  int32_t taint_t;    // first point time a merge changed its neighbourhood
+  int32_t pad1;
 };
 static_assert(sizeof(VoxState) == 80, "VoxState is 80 bytes");
 static_assert(offsetof(VoxState, merge_pos) == 40 && offsetof(VoxState, tag) == 48 &&

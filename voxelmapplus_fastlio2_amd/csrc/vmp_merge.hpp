@@ -523,7 +523,7 @@ __device__ inline int rank_le(const uint64_t* a, int n, uint64_t v) {  // elemen
 //   act      the first kMrWaves acting entries, a wave each: the merge() on a
 //            copy of the current state and, a lane per item, the
 //            re-evaluations its merges make necessary (new keys and the
-//            voxels' dirty/taint marks, held in registers until it commits);
+//            voxels' dirty marks, held in registers until it commits);
 //   commit   in point order.  An entry whose records, or (if it acts) the
 //            records its taint phase read, were changed by an earlier entry
 //            of the window, or that a new key must precede, or that acts and
@@ -805,7 +805,7 @@ __global__ void __launch_bounds__(kMrThreads) k_merge_replay(const MapDev* maps,
       //      neighbourhood: X re-evaluates its next call and its later
       //      candidates if X changed itself, or if X (a plane not in the
       //      group) passes the gates against a new record.  A voxel of the
-      //      scan records its dirty/taint times, one outside is marked dirty.
+      //      scan records its dirty time, one outside is marked dirty.
       if (!(item && ((cl >> cj) & 1))) X = -1;
       if (X >= 0) {
         int64_t ax, ay, az;
@@ -905,13 +905,8 @@ __global__ void __launch_bounds__(kMrThreads) k_merge_replay(const MapDev* maps,
       }
       if (need) {
         VoxState& xs = m.vs[X];
-        if (xseg >= 0) {
-          const int t = cand_t(wkey[w]);
-          atomicMax(&xs.dirty_t, t);
-          atomicMin(&xs.taint_t, t);
-        } else {
-          atomicOr(&xs.flags, kDirty);
-        }
+        if (xseg >= 0) atomicMax(&xs.dirty_t, cand_t(wkey[w]));
+        else atomicOr(&xs.flags, kDirty);
       }
       if (nl > 0) {
         int at = atomicAdd(&sh_i[3], nl);

@@ -69,11 +69,6 @@ __device__ inline double wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
-__device__ inline int wave_sum_i(int v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
 
 // DPP lane moves within 16-lane rows (no LDS traffic): quad_perm [1,0,3,2]
 // (0xB1), quad_perm [2,3,0,1] (0x4E), row_half_mirror (0x141), row_mirror

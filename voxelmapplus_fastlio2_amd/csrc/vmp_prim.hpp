@@ -183,8 +183,9 @@ struct NoTail {
 // ---- stable compaction: for the k-th i < n (ascending) whose pred(i) = v is
 // non-zero, out(k, i, v), a tile's selected items a thread each (packed in
 // LDS: a thread's own items one after the other made a chain of their loads).
-// pred is called once per item and may clear what it read.  tail(count), if active, runs in every thread of the last tile to
-// finish, after the outputs of all tiles are visible.
+// pred is called once per item and may clear what it read.  tail(count), if
+// active, runs in every thread of the last tile to finish, after the outputs
+// of all tiles are visible.
 template <class Pred, class Out, class Tail>
 __global__ void __launch_bounds__(kPrimThreads) k_select1(int n, Pred pred, Out out, Tail tail, int32_t* count,
                                                           PrimWs ws) {
@@ -361,8 +362,8 @@ __global__ void __launch_bounds__(kPrimThreads) k_rs_pass(const K* kin, const in
 }
 
 // The whole sort of one tile in one launch: the passes' keys stay in LDS, in
-// the same order.  18 key bits of 2,003 points in 9.7 us; the histogram and three
-// pass launches took 25.
+// the same order.  18 key bits of 2,003 points in 9.7 us; the histogram and
+// three pass launches took 25.
 template <class K>
 __global__ void __launch_bounds__(kPrimThreads) k_rs_tile(const K* kin, const int32_t* vin, K* kout, int32_t* vout,
                                                          int n, int passes, int width) {
@@ -415,7 +416,8 @@ inline int rs_passes(int bits) {
 }
 // Sorts (kin, vin) into (kout, vout) by the low `bits` bits of the keys,
 // stably; kin / vin are overwritten (ping-pong buffers).  One launch for a
-// single tile, else one histogram launch, then one launch per pass.  work: prim_ws_entries(n) int32 entries.
+// single tile, else one histogram launch, then one launch per pass.  work:
+// prim_ws_entries(n) int32 entries.
 template <class K>
 inline void radix_sort_stable(hipStream_t st, K* kin, int32_t* vin, K* kout, int32_t* vout, int n, int bits,
                               int32_t* work) {
