@@ -126,7 +126,9 @@ int vmp_session_destroy(vmp_session* s);
 int64_t vmp_session_bytes(const vmp_map_cfg* cfg);
 const char* vmp_last_error(const vmp_session* s);
 
-/* Filter state resident on the device (x and P, P column-major 23x23). */
+/* Filter state resident on the device (x and P, P column-major 23x23).
+ * vmp_state_get gives the state behind every call made so far, a motion prior
+ * enqueued behind a submitted batch included. */
 int vmp_state_set(vmp_session* s, const vmp_state* x, const double* P);
 int vmp_state_get(vmp_session* s, vmp_state* x, double* P);
 /* Motion prior between scans (stand-in for IMU propagation, which is outside
